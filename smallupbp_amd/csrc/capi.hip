@@ -187,7 +187,7 @@ Workspace context_workspace(Ctx& ctx, const upbp_query_batch* q) {
     const int64_t Q = q->count;
     if (q->order == UPBP_ORDER_SORTED && Q > 64) {
         for (DevBuf* b : {&ctx.qkeys, &ctx.qkeys2, &ctx.qperm, &ctx.qperm2}) b->ensure((size_t)Q * 4);
-        ctx.sort_tmp.ensure(sort_pairs_u32_temp_bytes(Q, 30));
+        ctx.sort_tmp.ensure(sort_pairs_u32_temp_bytes(Q, kQueryKeyBits));
         w.keys = ctx.qkeys.as<uint32_t>();
         w.keys2 = ctx.qkeys2.as<uint32_t>();
         w.perm = ctx.qperm.as<uint32_t>();
@@ -200,7 +200,9 @@ Workspace context_workspace(Ctx& ctx, const upbp_query_batch* q) {
 }
 
 // Device view of a batch (copies host batches), with the sorted permutation when requested.
-QueryView make_view(Ctx& ctx, const upbp_query_batch* q, const float* lo, const float* hi, const Workspace& ws) {
+// by_direction: see launch_query_keys (evaluations without beams).
+QueryView make_view(Ctx& ctx, const upbp_query_batch* q, const float* lo, const float* hi, bool by_direction,
+                    const Workspace& ws) {
     QueryView v;
     v.count = q->count;
     v.beam_type = q->beam_type;
@@ -219,8 +221,9 @@ QueryView make_view(Ctx& ctx, const upbp_query_batch* q, const float* lo, const 
     if (q->order == UPBP_ORDER_SORTED && q->count > 64) {
         UPBP_REQUIRE(q->count <= ws.max_sorted && ws.keys && ws.keys2 && ws.perm && ws.perm2, UPBP_EINVAL,
                      "more queries to sort than the workspace holds");
-        launch_query_keys(ctx, v, lo, hi, ws.keys, ws.perm);
-        sort_pairs_u32_in(ctx, ws.sort_tmp, ws.sort_tmp_bytes, ws.keys, ws.keys2, ws.perm, ws.perm2, q->count, 30);
+        launch_query_keys(ctx, v, lo, hi, by_direction, ws.keys, ws.perm);
+        sort_pairs_u32_in(ctx, ws.sort_tmp, ws.sort_tmp_bytes, ws.keys, ws.keys2, ws.perm, ws.perm2, q->count,
+                          kQueryKeyBits);
         v.perm = ws.perm2;
     }
     return v;
@@ -322,7 +325,7 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
         own = context_workspace(ctx, q);
         ws = &own;
     }
-    QueryView v = make_view(ctx, q, lo, hi, *ws);
+    QueryView v = make_view(ctx, q, lo, hi, !want_bm, *ws);
     launch_clear_u64(ctx, (uint64_t*)ws->stats, kStatSlots);
     // the UPBP light walks read per-vertex tails, built once here for both estimators
     MisDev mis_t;
@@ -708,7 +711,7 @@ upbp_status upbp_beams_grid_stats(upbp_ctx* ctx, const upbp_beams* beams, const 
         upbp_query_batch qb = *queries;
         qb.order = UPBP_ORDER_AS_GIVEN;
         const float none[3] = {0.f, 0.f, 0.f};
-        const QueryView v = make_view(*ctx, &qb, none, none, Workspace{});
+        const QueryView v = make_view(*ctx, &qb, none, none, false, Workspace{});
         DevBuf tmp;
         uint32_t* dout = out_stats;
         if (out_memory == UPBP_MEM_HOST) {
@@ -1314,9 +1317,9 @@ upbp_status upbp_batch_plan_create(upbp_ctx* ctx, const upbp_instance* instances
                 ctx->qkeys.ensure(v.count * 4);
                 ctx->qkeys2.ensure(v.count * 4);
                 ctx->qperm.ensure(v.count * 4);
-                launch_query_keys(*ctx, v, lo, hi, ctx->qkeys.as<uint32_t>(), ctx->qperm.as<uint32_t>());
+                launch_query_keys(*ctx, v, lo, hi, !d.has_beams, ctx->qkeys.as<uint32_t>(), ctx->qperm.as<uint32_t>());
                 sort_pairs_u32(*ctx, ctx->qkeys.as<uint32_t>(), ctx->qkeys2.as<uint32_t>(), ctx->qperm.as<uint32_t>(),
-                               perm->as<uint32_t>(), v.count, 30);
+                               perm->as<uint32_t>(), v.count, kQueryKeyBits);
                 d.perm = perm->as<uint32_t>();
             }
             tiles += (in.queries.count + 63) / 64;

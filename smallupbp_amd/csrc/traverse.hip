@@ -1393,13 +1393,70 @@ __global__ void k_combine_media(const float* gm, const float* sign, int n, float
     if (ga) ga[i] += sign[6 * m + c] * dt;
 }
 
-// Morton key of the first segment's entry point, for coherent query bundles.
+// Distance along the 15-bit Hilbert curve of the cell (x, y), in 30 bits.
+__device__ __forceinline__ uint32_t hilbert2(uint32_t x, uint32_t y) {
+    uint32_t d = 0;
+    for (int b = 14; b >= 0; --b) {
+        const uint32_t rx = (x >> b) & 1u, ry = (y >> b) & 1u;
+        d = (d << 2) | ((3u * rx) ^ ry);
+        const uint32_t low = (1u << b) - 1u;
+        x &= low;
+        y &= low;
+        if (!ry) {
+            const uint32_t f = rx ? low : 0u;  // reflected, then transposed
+            const uint32_t t = x ^ f;
+            x = y ^ f;
+            y = t;
+        }
+    }
+    return d;
+}
+
+constexpr uint32_t kOtherOrigin = 1u << (kQueryKeyBits - 1);  // key bit of the queries that do not start at query 0's origin
+
+// Sort key of a query, so that consecutive lanes hold coherent queries: the Morton code of its
+// first segment's entry point, or with by_direction
+//  - for a query from query 0's origin (the camera rays of a frame) its direction alone: the place
+//    on the octahedral map, turned so that query 0's main axis is the map's centre (the map's seam
+//    then lies opposite), along a Hilbert curve. 64 consecutive cells of that curve are one connected
+//    patch, so a wave's frustum is small wherever its run of 64 starts, while a run of the Morton
+//    order jumps: on 1920x1080 rays the frusta span 0.0055 x 0.0081 of the z = 0 plane on average
+//    in Morton order, 0.0045 x 0.0045 here (8 x 8 tiles: 0.0036 x 0.0036). The segments are not read.
+//  - for the others, after those, the Morton code.
+// Only evaluations without beams go by direction (256x256 rays x 100k photons: 402 -> 295 us). A beam's
+// end ties (test_beam_beam) are found where the wave's other rays visit the leaf, so which of them are
+// found depends on the rays that share a wave: beams keep the one order, and with it the same hits.
 __global__ void k_query_keys(int64_t n, const float* __restrict__ origin, const float* __restrict__ direction,
                              const int64_t* __restrict__ offsets, const upbp_volume_segment* __restrict__ seg,
-                             float lx, float ly, float lz, float sx, float sy, float sz, uint32_t* keys,
-                             uint32_t* idx) {
+                             float lx, float ly, float lz, float sx, float sy, float sz,
+                             bool by_direction, uint32_t* keys, uint32_t* idx) {
     int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (q >= n) return;
+    idx[q] = (uint32_t)q;
+    const float ox = origin[3 * q], oy = origin[3 * q + 1], oz = origin[3 * q + 2];
+    const float dx = direction[3 * q], dy = direction[3 * q + 1], dz = direction[3 * q + 2];
+    if (by_direction && ox == origin[0] && oy == origin[1] && oz == origin[2]) {
+        const float ax = __builtin_fabsf(direction[0]), ay = __builtin_fabsf(direction[1]),
+                    az = __builtin_fabsf(direction[2]);
+        float u = dx, v = dy, w = dz, s = direction[2];  // w: along query 0's main axis
+        if (ax >= ay && ax >= az)
+            u = dy, v = dz, w = dx, s = direction[0];
+        else if (ay >= az)
+            u = dz, v = dx, w = dy, s = direction[1];
+        w = s < 0.f ? -w : w;
+        const float l1 = (__builtin_fabsf(u) + __builtin_fabsf(v)) + __builtin_fabsf(w);
+        u /= l1, v /= l1;
+        if (w < 0.f) {
+            const float fu = 1.f - __builtin_fabsf(v), fv = 1.f - __builtin_fabsf(u);
+            u = u < 0.f ? -fu : fu;
+            v = v < 0.f ? -fv : fv;
+        }
+        // a zero or non-finite direction maps to cell 0: the evaluation reports it
+        const float cu = fminf(fmaxf((u + 1.f) * 16384.f, 0.f), 32767.f),
+                    cv = fminf(fmaxf((v + 1.f) * 16384.f, 0.f), 32767.f);
+        keys[q] = hilbert2((uint32_t)cu, (uint32_t)cv);
+        return;
+    }
     const int64_t s0 = offsets[q], s1 = offsets[q + 1], sn = offsets[n];
     float t = 0.f;
     // first segment in a scattering-capable position: use its start
@@ -1409,8 +1466,7 @@ __global__ void k_query_keys(int64_t n, const float* __restrict__ origin, const 
         // skip a leading clear segment (camera outside the media) when there is a next one
         if (s0 < last) t = seg[s0 + 1].dist_min;
     }
-    float p[3] = {origin[3 * q] + direction[3 * q] * t, origin[3 * q + 1] + direction[3 * q + 1] * t,
-                  origin[3 * q + 2] + direction[3 * q + 2] * t};
+    float p[3] = {ox + dx * t, oy + dy * t, oz + dz * t};
     const float l[3] = {lx, ly, lz}, s[3] = {sx, sy, sz};
     uint32_t key = 0;
     uint32_t c[3];
@@ -1421,8 +1477,7 @@ __global__ void k_query_keys(int64_t n, const float* __restrict__ origin, const 
     }
     for (int b = 9; b >= 0; --b)
         key = (key << 3) | (((c[0] >> b) & 1u) << 2) | (((c[1] >> b) & 1u) << 1) | ((c[2] >> b) & 1u);
-    keys[q] = key;
-    idx[q] = (uint32_t)q;
+    keys[q] = by_direction ? kOtherOrigin | key : key;
 }
 
 inline unsigned grid_for(int64_t n, int block = 256) {
@@ -1753,15 +1808,16 @@ void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total
     UPBP_HIP(hipGetLastError());
 }
 
-void launch_query_keys(Ctx& ctx, const QueryView& q, const float* lo, const float* hi, uint32_t* keys,
-                       uint32_t* idx) {
+void launch_query_keys(Ctx& ctx, const QueryView& q, const float* lo, const float* hi, bool by_direction,
+                       uint32_t* keys, uint32_t* idx) {
     float sc[3];
     for (int a = 0; a < 3; ++a) {
         const float e = hi[a] - lo[a];
         sc[a] = e > 0.f ? 1024.f / e : 0.f;
     }
     hipLaunchKernelGGL(k_query_keys, dim3(grid_for(q.count)), dim3(256), 0, ctx.stream, q.count, q.origin,
-                       q.direction, q.offsets, q.segments, lo[0], lo[1], lo[2], sc[0], sc[1], sc[2], keys, idx);
+                       q.direction, q.offsets, q.segments, lo[0], lo[1], lo[2], sc[0], sc[1], sc[2],
+                       by_direction, keys, idx);
     UPBP_HIP(hipGetLastError());
 }
 

@@ -332,8 +332,9 @@ void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& 
 void launch_beams(Ctx& ctx, Mode mode, const BeamArgs& bm, const QueryView& q, float* out,
                   uint32_t* sig, const AdjointOut* adj, const MisDev* mis = nullptr,
                   unsigned long long* stats = nullptr);
-void launch_query_keys(Ctx& ctx, const QueryView& q, const float* lo, const float* hi, uint32_t* keys,
-                       uint32_t* idx);
+constexpr int kQueryKeyBits = 31;  // sort keys of launch_query_keys
+void launch_query_keys(Ctx& ctx, const QueryView& q, const float* lo, const float* hi, bool by_direction,
+                       uint32_t* keys, uint32_t* idx);
 // Folds each light vertex's light walk below it into a float4 (the O(1) light walk of the
 // UPBP weights) into ctx.light_tails and points mis.tails at it; nothing for no vertices.
 void launch_light_tails(Ctx& ctx, MisDev& mis);
