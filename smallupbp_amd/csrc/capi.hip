@@ -54,9 +54,9 @@ struct upbp_batch_plan {
 // ends. In host code `scratch` names a host-side stand-in: only the address that
 // hipGetSymbolAddress returns for the current device (kept per device below) is ever used.
 constexpr size_t kScratchBytes = (size_t)UPBP_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kScratchStatsBytes = 256;
+constexpr size_t kScratchStatsBytes = 4096;
 constexpr int64_t kScratchMaxSorted = UPBP_NOALLOC_MAX_SORTED_QUERIES;
-static_assert(kStatSlots * 8 <= kScratchStatsBytes, "counters fit the scratch header");
+static_assert(kStatWords * 8 <= kScratchStatsBytes, "counters fit the scratch header");
 static_assert(kScratchStatsBytes + 4 * (size_t)kScratchMaxSorted * 4 < kScratchBytes, "scratch keeps room for the sort");
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -86,21 +86,28 @@ void* scratch_address(int device, std::string& why) {
     return g_scratch_ptr[device];
 }
 
-// The workspace carved out of a device's scratch region: counters first, then the four
-// [kScratchMaxSorted] key / permutation arrays, then the sort storage in what remains.
-Workspace scratch_workspace(void* base) {
+// The workspace carved out of a device's scratch region for a batch of `count` queries whose tiles
+// are split over `blocks` blocks per estimator: counters first, then the four key / permutation arrays, then the
+// sort storage in what remains below the blocks' sums at the end (none with one block).
+Workspace scratch_workspace(void* base, int64_t count, const uint32_t blocks[2]) {
     Workspace w;
     char* p = static_cast<char*>(base);
     w.stats = reinterpret_cast<unsigned long long*>(p);
     p += kScratchStatsBytes;
     uint32_t** arrays[4] = {&w.keys, &w.keys2, &w.perm, &w.perm2};
+    w.max_sorted = std::min(count, kScratchMaxSorted);
     for (uint32_t** a : arrays) {
         *a = reinterpret_cast<uint32_t*>(p);
-        p += (size_t)kScratchMaxSorted * 4;
+        p += ((size_t)w.max_sorted * 4 + 255) / 256 * 256;
     }
-    w.max_sorted = kScratchMaxSorted;
     w.sort_tmp = p;
-    w.sort_tmp_bytes = kScratchBytes - (size_t)(p - static_cast<char*>(base));
+    char* end = static_cast<char*>(base) + kScratchBytes;
+    for (int e = 0; e < 2; ++e)
+        if (blocks[e] > 1) {
+            end -= ((size_t)blocks[e] * count * 12 + 255) / 256 * 256;
+            w.partial[e] = reinterpret_cast<float*>(end);
+        }
+    w.sort_tmp_bytes = (size_t)(end - p);
     return w;
 }
 
@@ -179,12 +186,17 @@ void check_batch(const Ctx& ctx, const upbp_query_batch* q) {
     UPBP_REQUIRE(ctx.n_media > 0, UPBP_EINVAL, "upbp_set_media must be called before evaluation");
 }
 
-// The context's own workspace: its counters, and for a sorted batch of Q queries its key and
-// permutation buffers and sort storage, grown to fit.
-Workspace context_workspace(Ctx& ctx, const upbp_query_batch* q) {
+// The context's own workspace: its counters, for a sorted batch of Q queries its key and
+// permutation buffers and sort storage, and the sums of a split evaluation's parts, grown to fit.
+Workspace context_workspace(Ctx& ctx, const upbp_query_batch* q, const uint32_t blocks[2]) {
     Workspace w;
     w.stats = ctx.stats.as<unsigned long long>();
     const int64_t Q = q->count;
+    for (int e = 0; e < 2; ++e)
+        if (blocks[e] > 1) {
+            ctx.partial[e].ensure((size_t)blocks[e] * Q * 12);
+            w.partial[e] = ctx.partial[e].as<float>();
+        }
     if (q->order == UPBP_ORDER_SORTED && Q > 64) {
         for (DevBuf* b : {&ctx.qkeys, &ctx.qkeys2, &ctx.qperm, &ctx.qperm2}) b->ensure((size_t)Q * 4);
         ctx.sort_tmp.ensure(sort_pairs_u32_temp_bytes(Q, kQueryKeyBits));
@@ -306,10 +318,10 @@ struct RunOut {
     uint32_t* sig_bm = nullptr;
 };
 
-// ws: where the call's counters, query keys and sort storage live (null: the context's own buffers).
+// scratch_base: the fixed region that holds the call's workspace (null: the context's own buffers).
 void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch* q, Mode mode, RunOut o,
               upbp_memory out_mem, upbp_eval_stats* stats, const AdjointOut* adj_ph, const AdjointOut* adj_bm,
-              bool force_sync, const MisDev* mis = nullptr, const Workspace* ws = nullptr) {
+              bool force_sync, const MisDev* mis = nullptr, void* scratch_base = nullptr) {
     check_batch(ctx, q);
     if (bre) UPBP_REQUIRE(bre->ctx == &ctx, UPBP_EINVAL, "photon structure belongs to another context");
     if (bm) UPBP_REQUIRE(bm->ctx == &ctx, UPBP_EINVAL, "beam structure belongs to another context");
@@ -320,13 +332,18 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     if (timing) UPBP_HIP(hipEventRecord(ctx.ev[0], ctx.stream));
     float lo[3], hi[3];
     scene_bounds(bre, bm, lo, hi);
-    Workspace own;
-    if (!ws) {
-        own = context_workspace(ctx, q);
-        ws = &own;
-    }
+    const uint32_t parts[2] = {want_ph ? split_parts(Q, bre->n) : 1, want_bm ? split_parts(Q, bm->pieces) : 1};
+    uint32_t blocks[2] = {1, 1};  // the adjoint adds atomically
+    if (mode != Mode::Adjoint)
+        for (int e = 0; e < 2; ++e) blocks[e] = split_blocks(parts[e]);
+    const Workspace own = scratch_base ? scratch_workspace(scratch_base, Q, blocks) : context_workspace(ctx, q, blocks);
+    const Workspace* ws = &own;
     QueryView v = make_view(ctx, q, lo, hi, !want_bm, *ws);
-    launch_clear_u64(ctx, (uint64_t*)ws->stats, kStatSlots);
+    for (int e = 0; e < 2; ++e) {
+        v.parts[e] = parts[e];
+        v.partial[e] = ws->partial[e];
+    }
+    launch_clear_u64(ctx, (uint64_t*)ws->stats, kStatWords);
     // the UPBP light walks read per-vertex tails, built once here for both estimators
     MisDev mis_t;
     if (mis && mode == Mode::Upbp && Q > 0) {
@@ -391,6 +408,13 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     }
     if (timing) UPBP_HIP(hipEventRecord(ctx.ev[3], ctx.stream));
     if (overlap) UPBP_HIP(hipStreamWaitEvent(ctx.stream, ctx.join, 0));
+    if (blocks[0] > 1 || blocks[1] > 1) {
+        const bool ph = want_ph && bre->n > 0, bmv = want_bm && bm->pieces > 0;
+        if (mode == Mode::Signature)
+            launch_sum_parts_sig(ctx, v, ph ? sph : nullptr, bmv ? sbm : nullptr);
+        else
+            launch_sum_parts(ctx, v, ph ? dph : nullptr, bmv ? dbm : nullptr);
+    }
     if (out_mem == UPBP_MEM_HOST && Q > 0) {
         if (o.out_ph && want_ph) UPBP_HIP(hipMemcpyAsync(o.out_ph, dph, Q * 12, hipMemcpyDeviceToHost, ctx.stream));
         if (o.out_bm && want_bm) UPBP_HIP(hipMemcpyAsync(o.out_bm, dbm, Q * 12, hipMemcpyDeviceToHost, ctx.stream));
@@ -399,9 +423,10 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     }
     const bool do_sync = ctx.sync || timing || force_sync || out_mem == UPBP_MEM_HOST || q->memory == UPBP_MEM_HOST;
     if (!do_sync) return;
-    uint64_t st[kStatSlots];
-    UPBP_HIP(hipMemcpyAsync(st, ws->stats, sizeof(st), hipMemcpyDeviceToHost, ctx.stream));
+    uint64_t rows[kStatWords], st[kStatSlots];
+    UPBP_HIP(hipMemcpyAsync(rows, ws->stats, sizeof(rows), hipMemcpyDeviceToHost, ctx.stream));
     UPBP_HIP(hipStreamSynchronize(ctx.stream));
+    sum_stats(rows, st);
     float ms_other = 0.f, ms_ph = 0.f, ms_bm = 0.f;
     if (timing) {
         UPBP_HIP(hipEventElapsedTime(&ms_other, ctx.ev[0], ctx.ev[1]));
@@ -440,7 +465,7 @@ upbp_status upbp_ctx_create(int device, upbp_ctx** out_ctx) {
         UPBP_HIP(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
         UPBP_HIP(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming));
         UPBP_HIP(hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming));
-        ctx->stats.ensure(kStatSlots * 8);
+        ctx->stats.ensure(kStatWords * 8);
         ctx->scratch = scratch_address(device, ctx->scratch_error);
         *out_ctx = ctx;
         return UPBP_OK;
@@ -758,9 +783,8 @@ upbp_status upbp_eval_noalloc(upbp_ctx* ctx, const upbp_bre* bre, const upbp_bea
         RunOut o;
         o.out_ph = bre ? out_photons : nullptr;
         o.out_bm = beams ? out_beams : nullptr;
-        const Workspace ws = scratch_workspace(ctx->scratch);
         run_eval(*ctx, bre, beams, queries, Mode::Forward, o, UPBP_MEM_DEVICE, stats, nullptr, nullptr, false, nullptr,
-                 &ws);
+                 ctx->scratch);
     });
 }
 
@@ -941,7 +965,7 @@ void run_vm_eval(Ctx* ctx, const HashGrid* grid, uint32_t type, const Query* que
             dsig = ctx->staging[6].as<uint32_t>();
         }
     }
-    launch_clear_u64(*ctx, ctx->stats.as<uint64_t>(), kStatSlots);
+    launch_clear_u64(*ctx, ctx->stats.as<uint64_t>(), kStatWords);
     if (timing) UPBP_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
     if (use_mis && count > 0) launch_light_tails(*ctx, d);
     launch(dq, d, dout, dsig);
@@ -951,9 +975,10 @@ void run_vm_eval(Ctx* ctx, const HashGrid* grid, uint32_t type, const Query* que
         if (sig) UPBP_HIP(hipMemcpyAsync(sig, dsig, count * 8, hipMemcpyDeviceToHost, ctx->stream));
     }
     // the staged inputs are freed on return, so the call always completes here
-    uint64_t st[kStatSlots];
-    UPBP_HIP(hipMemcpyAsync(st, ctx->stats.p, sizeof(st), hipMemcpyDeviceToHost, ctx->stream));
+    uint64_t rows[kStatWords], st[kStatSlots];
+    UPBP_HIP(hipMemcpyAsync(rows, ctx->stats.p, sizeof(rows), hipMemcpyDeviceToHost, ctx->stream));
     UPBP_HIP(hipStreamSynchronize(ctx->stream));
+    sum_stats(rows, st);
     float ms_other = 0.f, ms_k = 0.f;
     if (timing) {
         UPBP_HIP(hipEventElapsedTime(&ms_other, ctx->ev[0], ctx->ev[1]));
@@ -1122,8 +1147,8 @@ upbp_status upbp_adjoint(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* b
         const float* gph = do_ph ? stage_q(*ctx, 4, grad_out_photons, 3 * Q, memory) : nullptr;
         const float* gbm = do_bm ? stage_q(*ctx, 5, grad_out_beams, 3 * Q, memory) : nullptr;
         DevBuf gmedia, items_ph, items_bm, gs_d, ga_d;
-        gmedia.ensure((size_t)M * 6 * 4);
-        launch_clear_f32(*ctx, gmedia.as<float>(), (int64_t)M * 6);
+        gmedia.ensure((size_t)kGradRows * M * 6 * 4);
+        launch_clear_f32(*ctx, gmedia.as<float>(), (int64_t)kGradRows * M * 6);
         float* dpp = grad_photon_power;
         float* dbp = grad_beam_power;
         if (memory == UPBP_MEM_HOST) {
@@ -1160,8 +1185,9 @@ upbp_status upbp_adjoint(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* b
                                        grad_absorption);
             UPBP_HIP(hipStreamSynchronize(ctx->stream));
         } else {
-            std::vector<float> gm((size_t)M * 6);
-            UPBP_HIP(hipMemcpy(gm.data(), gmedia.p, gm.size() * 4, hipMemcpyDeviceToHost));
+            std::vector<float> rows((size_t)kGradRows * M * 6), gm((size_t)M * 6, 0.f);
+            UPBP_HIP(hipMemcpy(rows.data(), gmedia.p, rows.size() * 4, hipMemcpyDeviceToHost));
+            for (size_t i = 0; i < rows.size(); ++i) gm[i % gm.size()] += rows[i];
             const std::vector<float>& sg = ctx->media_sign_host;
             for (int m = 0; m < M; ++m)
                 for (int c = 0; c < 3; ++c) {
@@ -1357,7 +1383,7 @@ upbp_status upbp_batch_plan_destroy(upbp_batch_plan* plan) {
 // capture records as edges), so the beam kernel's blocks fill the CUs the photon
 // kernel frees as its queue drains.
 static void enqueue_batch(Ctx& ctx, upbp_batch_plan* plan, int blocks) {
-    launch_clear_u64(ctx, ctx.stats.as<uint64_t>(), kStatSlots);
+    launch_clear_u64(ctx, ctx.stats.as<uint64_t>(), kStatWords);
     launch_fill_u32(ctx, plan->counters.as<uint32_t>(), 0u, 2);
     hipStream_t main_stream = ctx.stream;
     UPBP_HIP(hipEventRecord(ctx.fork, main_stream));
@@ -1426,9 +1452,10 @@ upbp_status upbp_batch_run(upbp_ctx* ctx, upbp_batch_plan* plan, int use_graph, 
         }
         if (stats) UPBP_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
         if (!ctx->sync && !stats) return;
-        uint64_t st[kStatSlots];
-        UPBP_HIP(hipMemcpyAsync(st, ctx->stats.p, sizeof(st), hipMemcpyDeviceToHost, ctx->stream));
+        uint64_t rows[kStatWords], st[kStatSlots];
+        UPBP_HIP(hipMemcpyAsync(rows, ctx->stats.p, sizeof(rows), hipMemcpyDeviceToHost, ctx->stream));
         UPBP_HIP(hipStreamSynchronize(ctx->stream));
+        sum_stats(rows, st);
         float ms = 0.f;
         if (stats) UPBP_HIP(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
         fill_stats(stats, st, ms, 0.f, 0.f, 2);

@@ -468,9 +468,10 @@ __global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __res
         he |= __shfl_xor(he, off, 64);
     }
     if ((threadIdx.x & 63) == 0 && A.count_stats) {
-        if (hp) atomicAdd(A.stats + kStatPhotonHits, (unsigned long long)hp);
-        if (ht) atomicAdd(A.stats + kStatPhotonCands, (unsigned long long)ht);
-        if (he) atomicOr(A.stats + kStatError, (unsigned long long)he);
+        unsigned long long* stats = A.stats + (slot / 64) % kStatRows * kStatSlots;
+        if (hp) atomicAdd(stats + kStatPhotonHits, (unsigned long long)hp);
+        if (ht) atomicAdd(stats + kStatPhotonCands, (unsigned long long)ht);
+        if (he) atomicOr(stats + kStatError, (unsigned long long)he);
     }
 }
 

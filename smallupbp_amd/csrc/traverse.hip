@@ -60,7 +60,7 @@ struct EvalArgs {
     unsigned long long* __restrict__ stats;
     // adjoint
     const float* __restrict__ grad_out;
-    float* __restrict__ grad_media;  // [M][6]
+    float* __restrict__ grad_media;  // [kGradRows][M][6]: a wave adds to its block's row
     float* __restrict__ grad_items;  // [items][3]
     // UPBP mode
     const upbp_query_mis* __restrict__ qmis;
@@ -71,6 +71,33 @@ struct EvalArgs {
     uint32_t frustum_leaf;
     // per-cell beam reduction of the beam estimators (red.max == 0: none)
     RedDev red;
+    // a tile's items split over `parts` waves (a power of two): the waves of a block, parts of one
+    // tile, add their sums up in LDS, and each block's go to the outputs, or with several blocks per
+    // tile to partial[block of the tile][slot][3] (partial_sig: [2]), which k_sum_parts adds up
+    uint32_t parts;
+    uint32_t part_shift;
+    float* __restrict__ partial;
+    uint32_t* __restrict__ partial_sig;
+};
+
+// The items a wave gathers: the blocks of 2^shift items of leaf order whose index is p modulo
+// mask + 1. Blocks are dealt out in turn, because the items that one tile meets often lie close
+// together in that order (the beams that leave one light).
+struct ItemPart {
+    uint32_t p, mask, shift;
+    // whether some of the n items from s on are this part's
+    __device__ __forceinline__ bool meets(uint32_t s, uint32_t n) const {
+        const uint32_t b = s >> shift;
+        return ((p - b) & mask) <= ((s + n - 1u) >> shift) - b;
+    }
+    // which of the n <= 64 items from s on are (they lie in at most two blocks, of 64 items or more)
+    __device__ __forceinline__ uint64_t items(uint32_t s, uint32_t n) const {
+        const uint64_t all = n >= 64u ? ~0ull : ((1ull << n) - 1ull);
+        const uint32_t b = s >> shift, first = ((b + 1u) << shift) - s;  // items left in the first block
+        const uint64_t low = first >= 64u ? ~0ull : ((1ull << first) - 1ull);
+        const uint64_t mine = (((p - b) & mask) == 0u ? low : 0ull) | (((p - b - 1u) & mask) == 0u ? ~low : 0ull);
+        return all & mine;
+    }
 };
 
 __device__ __forceinline__ float guard_inv(float d) {
@@ -115,6 +142,25 @@ __device__ __forceinline__ uint64_t uni_u64(uint64_t v) {
     return ((uint64_t)hi << 32) | (uint64_t)lo;
 }
 
+// The kernel's arguments read again from memory (KARG: A is k_eval's only argument; else A itself), for
+// the code around the traversal: values the compiler would otherwise load once and keep in scalar
+// registers through the traversal loop, or spill into lanes of vector registers there. `after` is a
+// scalar that the reads must wait for. (Not volatile: that would count as a write to memory, and the
+// traversal's node and item reads would no longer be scalar loads.)
+template <bool KARG, class Args>
+__device__ __forceinline__ const Args* reread(const Args& A, uint32_t after) {
+    if (!KARG) return &A;
+    auto p = (const __attribute__((address_space(4))) Args*)(uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm("" : "+s"(p) : "s"(after));
+    return (const Args*)p;
+}
+
+// A pointer to global memory, however it was read.
+template <class T>
+__device__ __forceinline__ T* as_global(T* p) {
+    return (T*)(__attribute__((address_space(1))) T*)p;
+}
+
 template <class T>
 __device__ __forceinline__ T* uni_global(T* p) {
     return (T*)(__attribute__((address_space(1))) T*)uni_u64((uint64_t)p);
@@ -142,6 +188,8 @@ struct SegState {
 // A MODE of Forward or Signature with this bit set applies the per-cell beam reduction
 // (a separate instantiation: the plain kernels keep their registers).
 constexpr int kReduced = 8;
+// With this bit a tile's items are split over several waves (the others keep their registers too).
+constexpr int kSplit = 16;
 
 template <int MODE>
 struct LaneOut {
@@ -895,30 +943,30 @@ __device__ __forceinline__ void beam_leaf(const EvalArgs& A, const Ray& r, SegSt
 // The items [start, start + cnt) (cnt <= 64) of a leaf, culled against the wave's frustum first
 // when it has one.
 template <int EST, int MODE>
-__device__ __forceinline__ void visit_leaf(const EvalArgs& A, const Frustum& F, bool fr, const Ray& r, SegState& s,
-                                           LaneOut<MODE>& lo, uint32_t start, uint32_t cnt, bool short_q,
-                                           uint32_t active, uint64_t& tests) {
-    const uint64_t all = cnt >= 64u ? ~0ull : ((1ull << cnt) - 1ull);
+__device__ __forceinline__ void visit_leaf(const EvalArgs& A, const Frustum& F, bool fr, ItemPart part,
+                                           const Ray& r, SegState& s, LaneOut<MODE>& lo, uint32_t start,
+                                           uint32_t cnt, bool short_q, uint32_t& tested) {
+    const uint64_t all = (MODE & kSplit) ? part.items(start, cnt) : cnt >= 64u ? ~0ull : ((1ull << cnt) - 1ull);
     if (EST == kEstPhotons) {
         const uint64_t items = fr ? frustum_photons(A, F, start, cnt) & all : all;
-        tests += (uint64_t)__popcll(items) * active;
+        tested += (uint32_t)__popcll(items);
         photon_leaf<MODE>(A, r, s, lo, start, items, short_q);
     } else {
         const uint64_t items = fr ? frustum_items(A, F, start, cnt) & all : all;
-        tests += (uint64_t)__popcll(items) * active;
+        tested += (uint32_t)__popcll(items);
         beam_leaf<MODE>(A, r, s, lo, start, items, short_q);
     }
 }
 
 template <int EST, int MODE>
-__device__ __forceinline__ void traverse(const EvalArgs& A, const Ray& r, SegState& s, LaneOut<MODE>& lo,
-                                         bool short_q, uint64_t& nodes_visited, uint64_t& tests,
+__device__ __forceinline__ void traverse(const EvalArgs& A, ItemPart part, const Ray& r, SegState& s,
+                                         LaneOut<MODE>& lo, bool short_q, uint32_t& nodes_visited, uint64_t& tests,
                                          uint32_t& overflow) {
     const int lane = threadIdx.x & (kWave - 1);
     uint32_t stk0 = 0, stk1 = 0;
     int sp = 0;
     uint32_t node = A.root;
-    const uint32_t active = (uint32_t)__popcll(__ballot(s.tmin <= s.tmax));
+    uint32_t tested = 0;
     Frustum F;
     const bool fr = make_frustum(r, s, F);
     while (true) {
@@ -932,21 +980,20 @@ __device__ __forceinline__ void traverse(const EvalArgs& A, const Ray& r, SegSta
         nodes_visited++;
         const uint64_t m0 = slab_mask(r, s.tmin, s.tmax, a.x, a.y, a.z, a.w, b.x, b.y);
         const uint64_t m1 = slab_mask(r, s.tmin, s.tmax, b.z, b.w, c.x, c.y, c.z, c.w);
-        // the wave-uniform child references are tested on the scalar side
-        const bool any0 = m0 != 0 && rr.z != kInvalid;
-        const bool any1 = m1 != 0 && rr.w != kInvalid;
+        // the wave-uniform child references and the items their subtrees hold (this wave's part
+        // or not) are tested on the scalar side
+        const uint32_t n0 = rr.z & kSpanMask, n1 = rr.w & kSpanMask;
+        const uint32_t s0 = (rr.z & kSpanEnds) ? rr.x + 1u - n0 : rr.x;
+        const uint32_t s1 = (rr.w & kSpanEnds) ? rr.y + 1u - n1 : rr.y;
+        const bool any0 = m0 != 0 && rr.z != kInvalid && (!(MODE & kSplit) || part.meets(s0, n0));
+        const bool any1 = m1 != 0 && rr.w != kInvalid && (!(MODE & kSplit) || part.meets(s1, n1));
         // A leaf; or, for a wave with a frustum, an inner node whose subtree holds at most
         // frustum_leaf items: the frustum check takes a whole leaf in one pass, so a small
         // subtree costs less as one leaf than as nodes (leaves stay small for the other waves).
-        const uint32_t n0 = rr.z & kSpanMask, n1 = rr.w & kSpanMask;
         const bool leaf0 = any0 && (!(rr.z & kInner) || (fr && n0 <= A.frustum_leaf));
         const bool leaf1 = any1 && (!(rr.w & kInner) || (fr && n1 <= A.frustum_leaf));
-        if (leaf0)
-            visit_leaf<EST, MODE>(A, F, fr, r, s, lo, (rr.z & kSpanEnds) ? rr.x + 1u - n0 : rr.x, n0, short_q,
-                                  active, tests);
-        if (leaf1)
-            visit_leaf<EST, MODE>(A, F, fr, r, s, lo, (rr.w & kSpanEnds) ? rr.y + 1u - n1 : rr.y, n1, short_q,
-                                  active, tests);
+        if (leaf0) visit_leaf<EST, MODE>(A, F, fr, part, r, s, lo, s0, n0, short_q, tested);
+        if (leaf1) visit_leaf<EST, MODE>(A, F, fr, part, r, s, lo, s1, n1, short_q, tested);
         const bool go0 = any0 && !leaf0;
         const bool go1 = any1 && !leaf1;
         if (go0 && go1) {
@@ -971,38 +1018,46 @@ __device__ __forceinline__ void traverse(const EvalArgs& A, const Ray& r, SegSta
                               : (uint32_t)__builtin_amdgcn_readlane((int)stk1, sp - kWave);
         }
     }
+    tests += (uint64_t)tested * (uint32_t)__popcll(__ballot(s.tmin <= s.tmax));
 }
 
 __device__ __forceinline__ bool finite3(float x, float y, float z) {
     return __builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z);
 }
 
-__device__ __forceinline__ float s_tmin_of(const EvalArgs& A, int64_t i) { return A.segments[i].dist_min; }
-__device__ __forceinline__ float s_tmax_of(const EvalArgs& A, int64_t i) { return A.segments[i].dist_max; }
+// The block's row of the medium gradients (media_base is 0 outside batched plans, which have no adjoint).
+__device__ __forceinline__ float* grad_row(const EvalArgs& A) {
+    return as_global(A.grad_media) + (size_t)(blockIdx.x % kGradRows) * A.n_media * 6;
+}
 
-// Processes the 64 queries of one tile (wave). `slot0` is the first lane slot.
-template <int EST, int MODE>
-__device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* local_stats,
+__shared__ float g_part[4][3][kWave];  // a split tile's sums per wave of the block
+
+// Processes the 64 queries of one tile (wave) against its part of the items. `slot0` is the first
+// lane slot.
+template <int EST, int MODE, bool KARG>
+__device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsigned long long* local_stats,
                          float* lds_media /* adjoint: [lds_media_n][6][64] for this wave or null */) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t slot = slot0 + lane;
     const bool valid = slot < A.count;
-    int64_t qi = 0;
-    if (valid) qi = A.perm ? (int64_t)A.perm[slot] : slot;
+    uint32_t qi = 0;  // fewer than 2^32 queries
+    if (valid) qi = A.perm ? A.perm[slot] : (uint32_t)slot;
     uint32_t err = 0;
     Ray r = {};
-    int64_t s0 = 0, s1 = 0;
+    int nseg = 0;
     bool alive = false;
     if (valid) {
-        r.ox = A.origin[3 * qi];
-        r.oy = A.origin[3 * qi + 1];
-        r.oz = A.origin[3 * qi + 2];
-        r.dx = A.direction[3 * qi];
-        r.dy = A.direction[3 * qi + 1];
-        r.dz = A.direction[3 * qi + 2];
-        s0 = A.offsets[qi];
-        s1 = A.offsets[qi + 1];
+        const float* o = A.origin + 3 * (int64_t)qi;
+        const float* d = A.direction + 3 * (int64_t)qi;
+        r.ox = o[0];
+        r.oy = o[1];
+        r.oz = o[2];
+        r.dx = d[0];
+        r.dy = d[1];
+        r.dz = d[2];
+        const int64_t s0 = A.offsets[qi], s1 = A.offsets[(int64_t)qi + 1];
         const int64_t sq = A.offsets[A.count];
+        nseg = (int)(s1 - s0);
         alive = true;
         if (!(s0 >= 0 && s0 <= s1 && s1 <= sq)) {
             err |= kErrBadOffsets;
@@ -1025,7 +1080,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                                   __float_as_uint(r.dx), __float_as_uint(r.dy), __float_as_uint(r.dz)};
         r.qkey = red_query_key(bits);
     }
-    int nseg = alive ? (int)(s1 - s0) : 0;
+    if (!alive) nseg = 0;
     int maxseg = nseg;
     for (int off = 32; off > 0; off >>= 1) maxseg = max(maxseg, __shfl_xor(maxseg, off, kWave));
     maxseg = (int)uni((uint32_t)maxseg);
@@ -1035,9 +1090,9 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
     float R0 = 0.f, R1 = 0.f, R2 = 0.f;
     float W0 = 0.f, W1 = 0.f, W2 = 0.f;
     if ((MODE & 7) == (int)Mode::Adjoint && valid) {
-        W0 = A.grad_out[3 * qi];
-        W1 = A.grad_out[3 * qi + 1];
-        W2 = A.grad_out[3 * qi + 2];
+        W0 = A.grad_out[3 * (int64_t)qi];
+        W1 = A.grad_out[3 * (int64_t)qi + 1];
+        W2 = A.grad_out[3 * (int64_t)qi + 2];
     }
     LaneOut<MODE> lo;
     if ((MODE & 7) == (int)Mode::Upbp) {
@@ -1071,8 +1126,8 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
         g_hacc[w][1][lane] = 0.f;
         g_hacc[w][2][lane] = 0.f;
     }
-    uint64_t nodes_visited = 0, tests = 0;
-    uint32_t overflow = 0;
+    uint64_t tests = 0;
+    uint32_t nodes_visited = 0, overflow = 0;
     for (int k = 0; k < maxseg; ++k) {
         bool has = alive && k < nseg;
         SegState s;
@@ -1088,19 +1143,18 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
         s.w0 = s.w1 = s.w2 = 0.f;
         s.gs0 = s.gs1 = s.gs2 = 0.f;
         s.gt0 = s.gt1 = s.gt2 = 0.f;
-        const MediumDev* m = nullptr;
-        float a0 = 1.f, a1 = 1.f, a2 = 1.f, pdf = 1.f;
+        const EvalArgs& C = *reread<KARG>(A, (uint32_t)k);
+        const upbp_volume_segment* segments = as_global(C.segments);
+        const MediumDev* media = as_global(C.media);
         bool scatter = false;
         if (has) {
-            const upbp_volume_segment* sg = A.segments + (s0 + k);
+            const upbp_volume_segment* sg = segments + (as_global(C.offsets)[qi] + k);
             const float tmin = sg->dist_min, tmax = sg->dist_max;
             const int32_t mid = sg->medium_id;
-            a0 = sg->attenuation[0];
-            a1 = sg->attenuation[1];
-            a2 = sg->attenuation[2];
-            pdf = sg->ray_sample_pdf;
-            // A.n_media counts the media from A.media_base on (the whole table outside batched plans)
-            if (mid < 0 || mid >= A.n_media) {
+            const float a0 = sg->attenuation[0], a1 = sg->attenuation[1], a2 = sg->attenuation[2];
+            const float pdf = sg->ray_sample_pdf;
+            // n_media counts the media from media_base on (the whole table outside batched plans)
+            if (mid < 0 || mid >= C.n_media) {
                 err |= kErrBadMedium;
                 has = false;
                 alive = false;
@@ -1114,7 +1168,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                 has = false;
                 alive = false;
             } else {
-                m = A.media + (A.media_base + mid);
+                const MediumDev* m = media + (C.media_base + mid);
                 scatter = m->has_scattering != 0;
                 s.medium = mid;
                 if (scatter) {
@@ -1135,12 +1189,6 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                 }
                 if ((MODE & 7) == (int)Mode::Upbp)
                     lo.ml.seg_flags = UPBP_END_IN_MEDIUM | (k == 0 ? lo.ml.ray_flags : 0u);
-                if (A.lite) {
-                    const float len = tmax - tmin;
-                    a0 = fast_exp(-m->st[0] * len);
-                    a1 = fast_exp(-m->st[1] * len);
-                    a2 = fast_exp(-m->st[2] * len);
-                }
             }
         }
         if ((MODE & 7) == (int)Mode::Adjoint) {
@@ -1149,17 +1197,18 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
             s.w2 = W2 * P2;
         }
         if (__ballot(scatter)) {
-            traverse<EST, MODE>(A, r, s, lo, short_q, nodes_visited, tests, overflow);
+            traverse<EST, MODE>(A, part, r, s, lo, short_q, nodes_visited, tests, overflow);
             if ((MODE & 7) == (int)Mode::Upbp) upbp_segment_end<EST, MODE>(A, r, s, lo, short_q);
         }
+        const EvalArgs& D = *reread<KARG>(A, nodes_visited);
         if (has) {
             R0 += P0 * s.acc0;
             R1 += P1 * s.acc1;
             R2 += P2 * s.acc2;
             if ((MODE & 7) == (int)Mode::Adjoint && scatter) {
                 // medium gradients of this segment plus the prefix terms of earlier segments
-                const int mloc = A.media_base + s.medium;
-                float* slab_m = (lds_media && s.medium < A.lds_media_n) ? lds_media : nullptr;
+                const int mloc = D.media_base + s.medium;
+                float* slab_m = (lds_media && s.medium < D.lds_media_n) ? lds_media : nullptr;
                 if (slab_m) {
                     float* base = slab_m + (size_t)s.medium * 6 * kWave + lane;
                     base[0 * kWave] += s.gs0;
@@ -1169,7 +1218,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                     base[4 * kWave] += s.gt1;
                     base[5 * kWave] += s.gt2;
                 } else {
-                    float* gm = A.grad_media + (size_t)mloc * 6;
+                    float* gm = grad_row(D) + (size_t)mloc * 6;
                     unsafeAtomicAdd(&gm[0], s.gs0);
                     unsafeAtomicAdd(&gm[1], s.gs1);
                     unsafeAtomicAdd(&gm[2], s.gs2);
@@ -1179,14 +1228,14 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                 }
                 // s.acc = sum_hits w * C for this segment (w already includes P)
                 for (int j = 0; j < k; ++j) {
-                    const upbp_volume_segment* sp = A.segments + (s0 + j);
+                    const upbp_volume_segment* sp = as_global(D.segments) + (as_global(D.offsets)[qi] + j);
                     const float len = sp->dist_max - sp->dist_min;
                     const int32_t mj = sp->medium_id;
                     float d0 = -s.acc0 * len, d1 = -s.acc1 * len, d2 = -s.acc2 * len;
                     // SHORT query: the segment's factor is attenuation over its pass-through pdf
                     // exp(-sigma_t_k len) when the medium samples distances (Media.hxx:294-323)
-                    if (short_q && !A.lite) {
-                        const MediumDev* mm = A.media + (A.media_base + mj);
+                    if (short_q && !D.lite) {
+                        const MediumDev* mm = as_global(D.media) + (D.media_base + mj);
                         if (mm->min_comp > 0.f && mm->has_scattering) {
                             const float sum = ((s.acc0 + s.acc1) + s.acc2) * len;
                             if (mm->min_idx == 0) d0 += sum;
@@ -1194,20 +1243,31 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                             else d2 += sum;
                         }
                     }
-                    if (lds_media && mj < A.lds_media_n) {
+                    if (lds_media && mj < D.lds_media_n) {
                         float* base = lds_media + (size_t)mj * 6 * kWave + lane;
                         base[3 * kWave] += d0;
                         base[4 * kWave] += d1;
                         base[5 * kWave] += d2;
                     } else {
-                        float* gm = A.grad_media + (size_t)(A.media_base + mj) * 6;
+                        float* gm = grad_row(D) + (size_t)(D.media_base + mj) * 6;
                         unsafeAtomicAdd(&gm[3], d0);
                         unsafeAtomicAdd(&gm[4], d1);
                         unsafeAtomicAdd(&gm[5], d2);
                     }
                 }
             }
-            if (A.lite || !short_q) {
+            // the segment's record is read again here instead of held through the traversal
+            const upbp_volume_segment* sg = as_global(D.segments) + (as_global(D.offsets)[qi] + k);
+            const MediumDev* m = as_global(D.media) + (D.media_base + s.medium);
+            float a0 = sg->attenuation[0], a1 = sg->attenuation[1], a2 = sg->attenuation[2];
+            const float pdf = sg->ray_sample_pdf;
+            if (D.lite) {
+                const float len = sg->dist_max - sg->dist_min;
+                a0 = fast_exp(-m->st[0] * len);
+                a1 = fast_exp(-m->st[1] * len);
+                a2 = fast_exp(-m->st[2] * len);
+            }
+            if (D.lite || !short_q) {
                 P0 *= a0;
                 P1 *= a1;
                 P2 *= a2;
@@ -1219,10 +1279,10 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
             if (!(P0 > 1e-20f && P1 > 1e-20f && P2 > 1e-20f)) alive = false;
             if ((MODE & 7) == (int)Mode::Upbp) {
                 // ray-sampling pdf prefixes of the segment loop (Bre.cxx:871-873, lite :955-958)
-                if (A.lite) {
+                if (D.lite) {
                     float rev = 1.f, spdf = 1.f;
                     if (m->min_comp != 0.f && m->has_scattering) {
-                        float att = fmaxf(__expf(-m->min_comp * (s_tmax_of(A, s0 + k) - s_tmin_of(A, s0 + k))), 1e-35f);
+                        float att = fmaxf(__expf(-m->min_comp * (sg->dist_max - sg->dist_min)), 1e-35f);
                         const float minatt = m->min_comp * att;
                         const uint32_t f = k == 0 ? lo.ml.ray_flags : 0u;
                         spdf = (f & UPBP_END_IN_MEDIUM) ? minatt : att;
@@ -1232,20 +1292,33 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
                     lo.ml.pref_rev *= rev;
                 } else {
                     lo.ml.pref_pdf *= pdf;
-                    lo.ml.pref_rev *= A.segments[s0 + k].ray_sample_rev_pdf;
+                    lo.ml.pref_rev *= sg->ray_sample_rev_pdf;
                 }
             }
         }
     }
     err |= lo.err;
+    const EvalArgs& E = *reread<KARG>(A, nodes_visited);
     if (valid && (MODE & 7) != (int)Mode::Adjoint) {
-        if ((MODE & 7) == (int)Mode::Signature) {
-            A.sig[2 * qi] = lo.sig_n;
-            A.sig[2 * qi + 1] = lo.sig_h;
+        if (MODE & kSplit) {  // the block adds its waves' parts up (block_sum)
+            const int w = threadIdx.x / kWave;
+            if ((MODE & 7) == (int)Mode::Signature) {
+                g_part[w][0][lane] = __uint_as_float(lo.sig_n);
+                g_part[w][1][lane] = __uint_as_float(lo.sig_h);
+            } else {
+                g_part[w][0][lane] = R0;
+                g_part[w][1][lane] = R1;
+                g_part[w][2][lane] = R2;
+            }
+        } else if ((MODE & 7) == (int)Mode::Signature) {
+            uint32_t* sig = as_global(E.sig);
+            sig[2 * (int64_t)qi] = lo.sig_n;
+            sig[2 * (int64_t)qi + 1] = lo.sig_h;
         } else {
-            A.out[3 * qi] = R0;
-            A.out[3 * qi + 1] = R1;
-            A.out[3 * qi + 2] = R2;
+            float* out = as_global(E.out) + 3 * (int64_t)qi;
+            out[0] = R0;
+            out[1] = R1;
+            out[2] = R2;
         }
     }
     // per-wave counters
@@ -1257,18 +1330,20 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, unsigned long long* l
     for (int off = 32; off > 0; off >>= 1) e |= __shfl_xor(e, off, kWave);
     local_stats[EST == kEstPhotons ? kStatPhotonHits : kStatBeamHits] += uni(h);
     local_stats[EST == kEstPhotons ? kStatPhotonCands : kStatBeamCands] += uni_u64(tests);
-    local_stats[kStatNodes] += uni_u64(nodes_visited);
+    local_stats[kStatNodes] += uni(nodes_visited);
     local_stats[kStatError] |= uni(e);
     local_stats[kStatOverflow] += uni(overflow);
 }
 
+// One wave's counters, in a row of its block's.
 __device__ __forceinline__ void flush_stats(const EvalArgs& A, const unsigned long long* ls) {
     if ((threadIdx.x & (kWave - 1)) == 0) {
+        unsigned long long* stats = as_global(A.stats) + blockIdx.x % kStatRows * kStatSlots;
         for (int k = 0; k < kStatSlots; ++k) {
             if (k == kStatError) {
-                if (ls[k]) atomicOr(&A.stats[k], ls[k]);
+                if (ls[k]) atomicOr(&stats[k], ls[k]);
             } else if (ls[k]) {
-                atomicAdd(&A.stats[k], ls[k]);
+                atomicAdd(&stats[k], ls[k]);
             }
         }
     }
@@ -1292,7 +1367,7 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
     const int wave_in_block = threadIdx.x / kWave;
     const int waves_per_block = blockDim.x / kWave;
     const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const int64_t wave = blk * waves_per_block + wave_in_block;
+    const int64_t wave = blk * waves_per_block + wave_in_block;  // parts of a tile are neighbours
     unsigned long long ls[kStatSlots] = {0, 0, 0, 0, 0, 0, 0, 0};
     // adjoint: per-lane medium gradient slabs, [lds_media_n][6][64] floats per wave, sized at launch
     extern __shared__ float lds_dyn[];
@@ -1302,17 +1377,44 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
         my_lds = lds_dyn + (size_t)wave_in_block * slab;
         for (int k = threadIdx.x & (kWave - 1); k < slab; k += kWave) my_lds[k] = 0.f;
     }
-    if (wave * kWave < A.count) run_tile<EST, MODE>(A, wave * kWave, ls, my_lds);
+    // wave-uniform (fewer than 2^32 waves: at most 2^26 tiles, and parts > 1 only for small batches)
+    const uint32_t w = uni((uint32_t)wave);
+    const uint32_t tile = (MODE & kSplit) ? w / A.parts : w;
+    const ItemPart part = {(MODE & kSplit) ? w % A.parts : 0u, A.parts - 1u, A.part_shift};
+    const int64_t slot0 = (int64_t)tile * kWave;
+    if (slot0 < A.count) run_tile<EST, MODE, true>(A, slot0, part, ls, my_lds);
+    const EvalArgs& E = *reread<true>(A, (uint32_t)ls[kStatNodes]);
+    if ((MODE & 7) != (int)Mode::Adjoint && (MODE & kSplit)) {
+        // every wave of the block holds a part of this tile: lane l of wave c sums channel c of its slot
+        __syncthreads();
+        constexpr int kN = (MODE & 7) == (int)Mode::Signature ? 2 : 3;
+        const uint32_t blocks = E.parts / (uint32_t)waves_per_block, b = part.p / (uint32_t)waves_per_block;
+        const int lane = threadIdx.x & (kWave - 1);
+        const int64_t slot = slot0 + lane;
+        if (slot < E.count)
+            for (int c = wave_in_block; c < kN; c += waves_per_block) {
+                const int64_t at = blocks > 1 ? (int64_t)b * E.count + slot : E.perm ? (int64_t)as_global(E.perm)[slot] : slot;
+                if ((MODE & 7) == (int)Mode::Signature) {
+                    uint32_t v = 0;
+                    for (int k = 0; k < waves_per_block; ++k) v += __float_as_uint(g_part[k][c][lane]);
+                    as_global(blocks > 1 ? E.partial_sig : E.sig)[kN * at + c] = v;
+                } else {
+                    float v = 0.f;
+                    for (int k = 0; k < waves_per_block; ++k) v += g_part[k][c][lane];
+                    as_global(blocks > 1 ? E.partial : E.out)[kN * at + c] = v;
+                }
+            }
+    }
     if ((MODE & 7) == (int)Mode::Adjoint) {
         // reduce the per-lane medium slabs of this wave and add them once
         const int lane = threadIdx.x & (kWave - 1);
-        const int nm = A.lds_media_n;
+        const int nm = E.lds_media_n;
         for (int e = 0; e < nm * 6; ++e) {
             const float v = wave_sum_dpp(my_lds[(size_t)e * kWave + lane]);
-            if (lane == 0 && v != 0.f) unsafeAtomicAdd(&A.grad_media[(size_t)(A.media_base) * 6 + e], v);
+            if (lane == 0 && v != 0.f) unsafeAtomicAdd(&grad_row(E)[(size_t)(E.media_base) * 6 + e], v);
         }
     }
-    flush_stats(A, ls);
+    flush_stats(E, ls);
 }
 
 // Persistent batched kernel: waves take (instance, tile) items from a device
@@ -1356,7 +1458,7 @@ __global__ __launch_bounds__(256, 6) void k_eval_batched(EvalArgs A, const Insta
         B.n_media = A.n_media - B.media_base;
         B.out = uni_global(EST == kEstPhotons ? I.out_photons : I.out_beams);
         const int64_t tile_begin = uni64(I.tile_begin);
-        run_tile<EST, (int)Mode::Forward>(B, ((int64_t)item - tile_begin) * kWave, ls, nullptr);
+        run_tile<EST, (int)Mode::Forward, false>(B, ((int64_t)item - tile_begin) * kWave, ItemPart{0u, 0u, 6u}, ls, nullptr);
     }
     flush_stats(A, ls);
 }
@@ -1369,6 +1471,27 @@ __global__ void k_rebase_nodes(NodeDev* nodes, int64_t n, uint32_t node_off, uin
     if (r.z != kInvalid) r.x += (r.z & kInner) ? node_off : item_off;
     if (r.w != kInvalid) r.y += (r.w & kInner) ? node_off : item_off;
     nodes[i].r = r;
+}
+
+// Adds up the blocks' sums of a split evaluation in block order (one thread per value in slot order;
+// an output that is null was written by its blocks).
+template <class T, int N>
+__global__ void k_sum_parts(int64_t n, const uint32_t* __restrict__ perm, uint32_t blocks_a, const T* __restrict__ pa,
+                            T* __restrict__ a, uint32_t blocks_b, const T* __restrict__ pb, T* __restrict__ b) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= N * n) return;
+    const int64_t slot = i / N, c = i % N;
+    const int64_t at = N * (perm ? (int64_t)perm[slot] : slot) + c;
+    if (a) {
+        T v = 0;
+        for (uint32_t k = 0; k < blocks_a; ++k) v += pa[N * n * k + i];
+        a[at] = v;
+    }
+    if (b) {
+        T v = 0;
+        for (uint32_t k = 0; k < blocks_b; ++k) v += pb[N * n * k + i];
+        b[at] = v;
+    }
 }
 
 __global__ void k_clear_u64(unsigned long long* p, int64_t n) {
@@ -1388,7 +1511,11 @@ __global__ void k_combine_media(const float* gm, const float* sign, int n, float
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 3 * n) return;
     const int m = i / 3, c = i % 3;
-    const float direct = gm[6 * m + c], dt = gm[6 * m + 3 + c];
+    float direct = 0.f, dt = 0.f;
+    for (int r = 0; r < kGradRows; ++r) {
+        direct += gm[6 * ((size_t)r * n + m) + c];
+        dt += gm[6 * ((size_t)r * n + m) + 3 + c];
+    }
     if (gs) gs[i] += sign[6 * m + 3 + c] * (direct + dt);
     if (ga) ga[i] += sign[6 * m + c] * dt;
 }
@@ -1484,54 +1611,34 @@ inline unsigned grid_for(int64_t n, int block = 256) {
     return (unsigned)std::max<int64_t>(1, (n + block - 1) / block);
 }
 
+template <int EST, int MODE>
+void launch_kernel(Ctx& ctx, const EvalArgs& A, unsigned blocks, unsigned threads, size_t lds) {
+    if (A.parts > 1)
+        hipLaunchKernelGGL((k_eval<EST, MODE | kSplit>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
+    else
+        hipLaunchKernelGGL((k_eval<EST, MODE>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
+    UPBP_HIP(hipGetLastError());
+}
+
+template <int EST, int MODE>
+void launch_reduced(Ctx& ctx, const EvalArgs& A, unsigned blocks, unsigned threads, size_t lds = 0) {
+    if constexpr (EST == kEstBeams) {
+        if (A.red.max != 0) return launch_kernel<EST, MODE | kReduced>(ctx, A, blocks, threads, lds);
+    }
+    launch_kernel<EST, MODE>(ctx, A, blocks, threads, lds);
+}
+
 template <int EST>
 void launch_mode(Ctx& ctx, Mode mode, const EvalArgs& A, unsigned blocks, unsigned threads) {
     switch (mode) {
-        case Mode::Forward:
-            if constexpr (EST == kEstBeams) {
-                if (A.red.max != 0) {
-                    hipLaunchKernelGGL((k_eval<EST, (int)Mode::Forward | kReduced>), dim3(blocks), dim3(threads), 0,
-                                       ctx.stream, A);
-                    break;
-                }
-            }
-            hipLaunchKernelGGL((k_eval<EST, (int)Mode::Forward>), dim3(blocks), dim3(threads), 0, ctx.stream, A);
-            break;
-        case Mode::Signature:
-            if constexpr (EST == kEstBeams) {
-                if (A.red.max != 0) {
-                    hipLaunchKernelGGL((k_eval<EST, (int)Mode::Signature | kReduced>), dim3(blocks), dim3(threads), 0,
-                                       ctx.stream, A);
-                    break;
-                }
-            }
-            hipLaunchKernelGGL((k_eval<EST, (int)Mode::Signature>), dim3(blocks), dim3(threads), 0, ctx.stream, A);
-            break;
-        case Mode::Adjoint: {
+        case Mode::Forward: return launch_reduced<EST, (int)Mode::Forward>(ctx, A, blocks, threads);
+        case Mode::Signature: return launch_reduced<EST, (int)Mode::Signature>(ctx, A, blocks, threads);
+        case Mode::Adjoint:
             // LDS gradient slabs for the media actually present: fewer bytes, more resident waves
-            const size_t lds = (size_t)(threads / kWave) * A.lds_media_n * 6 * kWave * sizeof(float);
-            if constexpr (EST == kEstBeams) {
-                if (A.red.max != 0) {
-                    hipLaunchKernelGGL((k_eval<EST, (int)Mode::Adjoint | kReduced>), dim3(blocks), dim3(threads), lds,
-                                       ctx.stream, A);
-                    break;
-                }
-            }
-            hipLaunchKernelGGL((k_eval<EST, (int)Mode::Adjoint>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
-            break;
-        }
-        case Mode::Upbp:
-            if constexpr (EST == kEstBeams) {
-                if (A.red.max != 0) {
-                    hipLaunchKernelGGL((k_eval<EST, (int)Mode::Upbp | kReduced>), dim3(blocks), dim3(threads), 0,
-                                       ctx.stream, A);
-                    break;
-                }
-            }
-            hipLaunchKernelGGL((k_eval<EST, (int)Mode::Upbp>), dim3(blocks), dim3(threads), 0, ctx.stream, A);
-            break;
+            return launch_reduced<EST, (int)Mode::Adjoint>(
+                ctx, A, blocks, threads, (size_t)(threads / kWave) * A.lds_media_n * 6 * kWave * sizeof(float));
+        case Mode::Upbp: return launch_reduced<EST, (int)Mode::Upbp>(ctx, A, blocks, threads);
     }
-    UPBP_HIP(hipGetLastError());
 }
 
 EvalArgs base_args(Ctx& ctx, const QueryView& q) {
@@ -1706,6 +1813,48 @@ static void set_mis(EvalArgs& A, const MisDev* mis) {
     A.mis.p = mis->params;
 }
 
+uint32_t split_parts(int64_t count, int64_t items) {
+    const int64_t tiles = (count + kWave - 1) / kWave;
+    uint32_t parts = 1;
+    if (items < kSplitFrom) return parts;
+    while (parts < kSplitMost && 2 * parts * tiles <= kSplitWaves && 2 * parts * kSplitItems <= items) parts *= 2;
+    return parts;
+}
+
+uint32_t split_blocks(uint32_t parts) { return parts > 4 ? parts / 4 : 1; }
+
+// 2^shift items per block of a split, 64 or more (ItemPart::items): 32 to 64 blocks per part where there
+// are enough. Fewer balance worse (8: 22.0 against 20.0 ms on 200k rays without a common origin, 7.9
+// against 7.0 ms on traced beams), more make every part walk more of the tree.
+static uint32_t part_shift(int64_t items, uint32_t parts) {
+    uint32_t shift = 6;
+    while (parts > 1 && ((int64_t)parts * 32 << (shift + 1)) <= items) ++shift;
+    return shift;
+}
+
+template <class T, int N>
+static void sum_parts(Ctx& ctx, const QueryView& q, T* ph, T* bm) {
+    const uint32_t a = split_blocks(q.parts[kEstPhotons]), b = split_blocks(q.parts[kEstBeams]);
+    if (a == 1) ph = nullptr;
+    if (b == 1) bm = nullptr;
+    if (!ph && !bm) return;
+    hipLaunchKernelGGL((k_sum_parts<T, N>), dim3(grid_for(N * q.count)), dim3(256), 0, ctx.stream, q.count, q.perm, a,
+                       reinterpret_cast<const T*>(q.partial[kEstPhotons]), ph, b,
+                       reinterpret_cast<const T*>(q.partial[kEstBeams]), bm);
+    UPBP_HIP(hipGetLastError());
+}
+
+void launch_sum_parts(Ctx& ctx, const QueryView& q, float* ph, float* bm) { sum_parts<float, 3>(ctx, q, ph, bm); }
+void launch_sum_parts_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* bm) {
+    sum_parts<uint32_t, 2>(ctx, q, ph, bm);
+}
+
+// Waves per block: the tuned number, or for split tiles (whose blocks hold parts of one tile) up to 4.
+static int block_waves(Mode mode, uint32_t parts, int tuned) {
+    if (parts > 1) return (int)std::min(parts, 4u);
+    return mode == Mode::Adjoint ? 4 : std::min(std::max(tuned, 1), 4);
+}
+
 void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& q, float* out, uint32_t* sig,
                     const AdjointOut* adj, const MisDev* mis, unsigned long long* stats) {
     if (q.count == 0) return;
@@ -1718,8 +1867,12 @@ void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& 
     A.inc = ph.inc;
     A.orig = ph.orig;
     A.red = ph.sel;
+    A.parts = q.parts[kEstPhotons];
+    A.part_shift = part_shift(ph.n, A.parts);
     A.out = out;
     A.sig = sig;
+    A.partial = q.partial[kEstPhotons];
+    A.partial_sig = reinterpret_cast<uint32_t*>(q.partial[kEstPhotons]);
     if (adj) {
         A.grad_out = adj->grad_out;
         A.grad_media = adj->grad_media;
@@ -1727,8 +1880,8 @@ void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& 
     }
     const int want = ctx.tuning.photon_waves_per_block > 0 ? ctx.tuning.photon_waves_per_block
                                                            : ctx.tuning.waves_per_block;
-    const int wpb = mode == Mode::Adjoint ? 4 : std::min(std::max(want, 1), 4);
-    const int64_t waves = (q.count + kWave - 1) / kWave;
+    const int wpb = block_waves(mode, A.parts, want);
+    const int64_t waves = (q.count + kWave - 1) / kWave * A.parts;
     launch_mode<kEstPhotons>(ctx, mode, A, (unsigned)((waves + wpb - 1) / wpb), (unsigned)(wpb * kWave));
 }
 
@@ -1743,15 +1896,19 @@ void launch_beams(Ctx& ctx, Mode mode, const BeamArgs& bm, const QueryView& q, f
     A.piece_flux = bm.piece_flux;
     A.orig = bm.piece_beam;
     A.red = bm.red;
+    A.parts = q.parts[kEstBeams];
+    A.part_shift = part_shift(bm.pieces_n, A.parts);
     A.out = out;
     A.sig = sig;
+    A.partial = q.partial[kEstBeams];
+    A.partial_sig = reinterpret_cast<uint32_t*>(q.partial[kEstBeams]);
     if (adj) {
         A.grad_out = adj->grad_out;
         A.grad_media = adj->grad_media;
         A.grad_items = adj->grad_items;
     }
-    const int wpb = mode == Mode::Adjoint ? 4 : std::min(std::max(ctx.tuning.waves_per_block, 1), 4);
-    const int64_t waves = (q.count + kWave - 1) / kWave;
+    const int wpb = block_waves(mode, A.parts, ctx.tuning.waves_per_block);
+    const int64_t waves = (q.count + kWave - 1) / kWave * A.parts;
     launch_mode<kEstBeams>(ctx, mode, A, (unsigned)((waves + wpb - 1) / wpb), (unsigned)(wpb * kWave));
 }
 
@@ -1777,6 +1934,8 @@ void prepare_batched(Ctx& ctx, int waves_per_block) {
 void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, uint32_t* counters,
                     const MergedDev& merged, int which, int grid_blocks, int waves_per_block) {
     EvalArgs A = {};
+    A.parts = 1;
+    A.part_shift = 6;
     A.media = ctx.media.as<MediumDev>();
     A.n_media = ctx.n_media;
     A.stats = ctx.stats.as<unsigned long long>();

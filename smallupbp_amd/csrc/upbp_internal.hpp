@@ -103,6 +103,20 @@ enum StatSlot : int {
     kStatOverflow = 6,  // traversal stack overflow count
     kStatSlots = 8
 };
+// The counters are kept in kStatRows rows of kStatSlots (one 64-byte line each) that the waves
+// spread over, added up by the host (sum_stats): with one row every wave of a launch queued for
+// the same few words. 131072 waves that had almost nothing else to do took 1.9 ms.
+constexpr int kStatRows = 64;
+constexpr int kStatWords = kStatRows * kStatSlots;
+
+inline void sum_stats(const uint64_t* rows, uint64_t* st) {
+    for (int k = 0; k < kStatSlots; ++k) st[k] = 0;
+    for (int r = 0; r < kStatRows; ++r)
+        for (int k = 0; k < kStatSlots; ++k) {
+            const uint64_t v = rows[r * kStatSlots + k];
+            st[k] = k == kStatError ? (st[k] | v) : st[k] + v;
+        }
+}
 constexpr uint32_t kErrBadOffsets = 1u, kErrBadMedium = 2u, kErrBadSegment = 4u, kErrNonFinite = 8u;
 
 struct Tuning {
@@ -132,7 +146,7 @@ struct Ctx {
     // bumped by every upbp_set_media: a batched plan whose captured graph froze an older table
     // re-validates its instances and captures again
     uint64_t media_gen = 0;
-    DevBuf stats;       // kStatSlots x uint64
+    DevBuf stats;       // kStatWords x uint64
     DevBuf sort_tmp;    // hipcub temporary storage
     TmpPool tmp;        // build temporaries
     DevBuf qkeys, qkeys2, qperm, qperm2;
@@ -141,6 +155,7 @@ struct Ctx {
     DevBuf photon_recs;  // 64-byte MIS record per light vertex of the current UPBP call
     DevBuf vm_rec;       // merge records (4 float4 per grid slot) of the current PP3D / SURF call
     DevBuf lt_slots[8];  // light tracing: per-path vertex, position and beam slots, counts, offsets, lights
+    DevBuf partial[2];  // sums of a split evaluation's parts, per estimator
     DevBuf staging[8];  // host-input staging copies
     hipEvent_t ev[6] = {};
     // second stream: the photon and beam kernels of one eval call run concurrently
@@ -201,11 +216,12 @@ struct Beams {
 // context's own growable buffers by default; the allocation-free entry point passes a fixed
 // region instead.
 struct Workspace {
-    unsigned long long* stats = nullptr;  // kStatSlots counters
+    unsigned long long* stats = nullptr;  // kStatWords counters
     uint32_t *keys = nullptr, *keys2 = nullptr, *perm = nullptr, *perm2 = nullptr;  // [max_sorted] each
     int64_t max_sorted = 0;
     void* sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
+    float* partial[2] = {nullptr, nullptr};  // per estimator, the sums of a split evaluation's parts
 };
 
 // Device-resident view of a query batch.
@@ -218,7 +234,25 @@ struct QueryView {
     uint32_t beam_type = UPBP_LONG_BEAM;
     uint32_t lite = 0;
     const uint32_t* perm = nullptr;  // lane slot -> query index, or null (identity)
+    // per estimator, a tile's items split over this many waves (split_parts); with several blocks per
+    // tile each block's sums go to partial ([split_blocks][count][3] floats) for k_sum_parts
+    uint32_t parts[2] = {1, 1};
+    float* partial[2] = {nullptr, nullptr};
 };
+
+// A tile of 64 queries is one wave, and the GPU holds 8192 of them: a batch of fewer tiles leaves it
+// partly idle, and one of a few times more waits for the waves that meet most of the items. So a
+// tile's items are split over as many waves as bring the launch to kSplitWaves, at most kSplitMost, each
+// for at least kSplitItems items. Structures of fewer than kSplitFrom items stay whole: little is left to
+// split there, and their sums stay the same bits as a batched plan's, which splits nothing. Measured unsplit / at 8192 / 16384 / 32768 / 65536 waves:
+//   64x36 rays x 20k photons + 2k beams       907 /  211 /  215 /  211 /  205 us
+//   512x512 rays, forward and adjoint       11.58 / 10.5 / 10.4 / 11.5 / 13.9 ms
+//   640x360 rays x 40k traced beams         24.59 / 14.9 /  9.2 /  6.7 /  5.6 ms
+//   200k rays without a common origin       36.95 / 23.3 / 20.9 / 19.9 / 20.6 ms
+// Above kSplitWaves tiles nothing is split: 1920x1080 rays took 12.4 ms either way at 2 parts, 13.7 at 4.
+constexpr int64_t kSplitWaves = 32768;
+constexpr int64_t kSplitItems = 256, kSplitFrom = 16384;
+constexpr uint32_t kSplitMost = 64;
 
 // ---- lbvh.hip -------------------------------------------------------------
 // Builds an LBVH over n item boxes (lo/hi as float4 .xyz). On return
@@ -303,9 +337,12 @@ struct BeamArgs {
     int64_t pieces_n;
     RedDev red;
 };
+// Rows of medium gradients that the adjoint's waves spread their atomics over (each wave adds 6 values
+// per medium: on one row they queue for the same words).
+constexpr int kGradRows = 64;
 struct AdjointOut {
     const float* grad_out;  // [Q][3]
-    float* grad_media;      // [M][6]: dsigma_s direct (0..2), dsigma_t (3..5)
+    float* grad_media;      // [kGradRows][M][6]: dsigma_s direct (0..2), dsigma_t (3..5)
     float* grad_items;      // photon [n_in][3] or beam [n][3]
 };
 
@@ -325,7 +362,7 @@ struct MisDev {
     const void* photon_recs = nullptr;  // per light vertex, launch_photon_records
 };
 
-// stats: the kStatSlots counters the kernels add to (null: the context's own)
+// stats: the kStatWords counters the kernels add to (null: the context's own)
 void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& q, float* out,
                     uint32_t* sig, const AdjointOut* adj, const MisDev* mis = nullptr,
                     unsigned long long* stats = nullptr);
@@ -343,10 +380,17 @@ void launch_light_tails(Ctx& ctx, MisDev& mis);
 void launch_beam_records(Ctx& ctx, MisDev& mis, int64_t n_beams);
 // The same per light vertex for the PB2D hits into ctx.photon_recs (mis.photon_recs).
 void launch_photon_records(Ctx& ctx, MisDev& mis);
+// How many waves share a tile's items in an evaluation of count queries against items items (a power
+// of two), and how many blocks they form.
+uint32_t split_parts(int64_t count, int64_t items);
+uint32_t split_blocks(uint32_t parts);
+// Adds up a split evaluation's parts into the outputs (null: not evaluated), in query order.
+void launch_sum_parts(Ctx& ctx, const QueryView& q, float* ph, float* bm);
+void launch_sum_parts_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* bm);
 void launch_clear_u64(Ctx& ctx, uint64_t* p, int64_t n);
 void launch_clear_f32(Ctx& ctx, float* p, int64_t n);
-// gs += sign_s * (direct + d/d sigma_t), ga += sign_a * d/d sigma_t per medium and channel
-// (sign: [M][6] of ctx.media_sign).
+// gs += sign_s * (direct + d/d sigma_t), ga += sign_a * d/d sigma_t per medium and channel, summed
+// over the kGradRows rows of gm (sign: [M][6] of ctx.media_sign).
 void launch_combine_media_grads(Ctx& ctx, const float* gm, const float* sign, int n_media, float* gs, float* ga);
 
 // ---- hashgrid.hip: vertex-merging hashed grid (PP3D, SURF) --------------------
