@@ -255,11 +255,10 @@ __device__ __forceinline__ bool vm_take(const VmArgs& A, uint32_t k, uint32_t ca
 // the camera / light continuation probabilities. Both walks are linear in their first
 // reverse pdf 1 / factor: the light walk is last * (k0 + k1 * dir_pdf) from the slot's
 // record, the camera walk last * ((a0 + bb0 * s * b) + cn * rev_pdf) from the query's split.
-__device__ __forceinline__ void vm_accumulate(const VmArgs& A, uint32_t k, uint32_t v, const CamSplit& cs,
+__device__ __forceinline__ void vm_accumulate(const VmArgs& A, uint32_t k, const float4& r1, const CamSplit& cs,
                                               float factor, float sin_t, float dir_pdf, float rev_pdf,
                                               uint32_t evaluated, float f0, float f1, float f2, float acc[3],
                                               uint32_t& err) {
-    const float4 r1 = A.rec[kRecWords * (int64_t)k + 1];
     float w = 1.f;
     if (!(A.flags & UPBP_VM_NO_MIS)) {
         const MisGlobals& G = A.mis;
@@ -273,21 +272,28 @@ __device__ __forceinline__ void vm_accumulate(const VmArgs& A, uint32_t k, uint3
         if (!__builtin_isnan(r2.y)) {
             w_light = inv * (r2.x + r2.y * dir_pdf);
         } else {
-            const upbp_light_vertex* __restrict__ lv = G.lv + v;
+            const upbp_light_vertex* __restrict__ lv = G.lv + __float_as_uint(A.slots[k].w);
             LightView lview{&G, nullptr, -1, 0.f};
             w_light = light_path_weight(lview, lv->path_idx, (int)lv->path_length, inv, dir_pdf, evaluated,
                                         P.query_beam_type, P.photon_beam_type, P.techniques, err);
         }
         w = 1.f / (w_light + w_cam);
     }
-    acc[0] += w * (f0 * r1.x);
-    acc[1] += w * (f1 * r1.y);
-    acc[2] += w * (f2 * r1.z);
+    acc[0] = w * (f0 * r1.x);
+    acc[1] = w * (f1 * r1.y);
+    acc[2] = w * (f2 * r1.z);
 }
+
+// What a camera vertex's merges read of it, kWords words per lane in LDS rows of 64: an entry of
+// the wave's hit queue is evaluated by whichever lane draws it, and that lane reads its owner's.
+// Words 0..3 are the path length (bits) and the camera walk's split.
+constexpr int kCamWords = 4;
 
 // ---- PP3D: camera vertex in a medium -------------------------------------
 struct Pp3dCam {
-    MediumDev m;
+    static constexpr int kWords = kCamWords + 9;
+    float dir[3], ss[3], g, cont;
+    uint32_t info;  // bit 0 scattering, bit 1 isotropic
 };
 
 __device__ __forceinline__ bool query_ok(const VmArgs& A, const upbp_pp3d_query& q, uint32_t& err) {
@@ -308,29 +314,40 @@ __device__ __forceinline__ bool query_ok(const VmArgs& A, const upbp_pp3d_query&
 }
 
 __device__ __forceinline__ Pp3dCam camera_of(const VmArgs& A, const upbp_pp3d_query& q) {
-    return Pp3dCam{A.media[q.medium]};
+    const MediumDev& m = A.media[q.medium];
+    return Pp3dCam{{q.dir_fix[0], q.dir_fix[1], q.dir_fix[2]},
+                   {m.ss[0], m.ss[1], m.ss[2]},
+                   m.g,
+                   m.cont,
+                   (m.has_scattering ? 1u : 0u) | (m.isotropic ? 2u : 0u)};
 }
 
 // RangeQuery::Process with a medium camera BSDF (Bsdf.hxx:216-230): sigma_s * phase
-// (fix = camera WorldDirFix, gen = light WorldDirFix), zero without scattering.
-__device__ void vm_process(const VmArgs& A, const upbp_pp3d_query& q, const Pp3dCam& c, const CamSplit& cs,
-                           uint32_t k, uint32_t v, float acc[3], uint32_t& err) {
+// (fix = camera WorldDirFix, gen = light WorldDirFix), zero without scattering. False: no merge.
+__device__ __forceinline__ bool vm_process(const VmArgs& A, const Pp3dCam& c, uint32_t len, const CamSplit& cs,
+                                           uint32_t k, float acc[3], uint32_t& err) {
     float4 r0, r3;
-    if (!vm_take(A, k, q.camera_path_length, r0, r3, err)) return;
-    const MediumDev& m = c.m;
-    if (!m.has_scattering) return;
-    const float cos_t = -dot3(r0.x, r0.y, r0.z, q.dir_fix[0], q.dir_fix[1], q.dir_fix[2]);
+    if (!vm_take(A, k, len, r0, r3, err)) return false;
+    if (!(c.info & 1u)) return false;
+    const float cos_t = -dot3(r0.x, r0.y, r0.z, c.dir[0], c.dir[1], c.dir[2]);
     const float sin_t = __builtin_sqrtf(fmaxf(0.f, 1.f - cos_t * cos_t));
-    const float pdf = phase_pdf(m.g, m.isotropic != 0, cos_t);
-    const float f0 = m.ss[0] * pdf, f1 = m.ss[1] * pdf, f2 = m.ss[2] * pdf;
-    if (f0 <= 0.f && f1 <= 0.f && f2 <= 0.f) return;
-    const float cont_l = A.rec[kRecWords * (int64_t)k + 1].w;
+    const float pdf = phase_pdf(c.g, (c.info & 2u) != 0, cos_t);
+    const float f0 = c.ss[0] * pdf, f1 = c.ss[1] * pdf, f2 = c.ss[2] * pdf;
+    if (f0 <= 0.f && f1 <= 0.f && f2 <= 0.f) return false;
+    const float4 r1 = A.rec[kRecWords * (int64_t)k + 1];
     // camera continuation on the direct pdf (UPBP.hxx:110), light continuation on the reverse (:116)
-    vm_accumulate(A, k, v, cs, r3.x, sin_t, pdf * m.cont, pdf * cont_l, UPBP_PP3D, f0, f1, f2, acc, err);
+    vm_accumulate(A, k, r1, cs, r3.x, sin_t, pdf * c.cont, pdf * r1.w, UPBP_PP3D, f0, f1, f2, acc, err);
+    return true;
 }
 
 // ---- SURF: camera vertex on a surface ------------------------------------
-struct SurfCam {};
+struct SurfCam {
+    static constexpr int kWords = kCamWords + 22;
+    float frame[9];  // x, y, z axes
+    float fix[3];
+    float diffuse[3], phong[3];
+    float diff_prob, phong_prob, exponent, cont;
+};
 
 __device__ __forceinline__ bool query_ok(const VmArgs& A, const upbp_surf_query& q, uint32_t& err) {
     bool ok = true;
@@ -346,23 +363,38 @@ __device__ __forceinline__ bool query_ok(const VmArgs& A, const upbp_surf_query&
     return ok;
 }
 
-__device__ __forceinline__ SurfCam camera_of(const VmArgs&, const upbp_surf_query&) { return SurfCam{}; }
+__device__ __forceinline__ SurfCam camera_of(const VmArgs&, const upbp_surf_query& q) {
+    SurfCam c;
+    for (int a = 0; a < 3; ++a) {
+        c.frame[a] = q.frame_x[a];
+        c.frame[3 + a] = q.frame_y[a];
+        c.frame[6 + a] = q.frame_z[a];
+        c.fix[a] = q.local_dir_fix[a];
+        c.diffuse[a] = q.diffuse[a];
+        c.phong[a] = q.phong[a];
+    }
+    c.diff_prob = q.diff_prob;
+    c.phong_prob = q.phong_prob;
+    c.exponent = q.phong_exponent;
+    c.cont = q.continuation_prob;
+    return c;
+}
 
 // RangeQuery::Process with a surface camera BSDF: Bsdf::Evaluate on a surface
 // (Bsdf.hxx:176-215) = EvaluateDiffuse (:542-561) + EvaluatePhong (:563-600), with the
-// light's WorldDirFix as the generated direction; sin(theta) is 0 on surfaces.
-__device__ void vm_process(const VmArgs& A, const upbp_surf_query& q, const SurfCam&, const CamSplit& cs, uint32_t k,
-                           uint32_t v, float acc[3], uint32_t& err) {
+// light's WorldDirFix as the generated direction; sin(theta) is 0 on surfaces. False: no merge.
+__device__ __forceinline__ bool vm_process(const VmArgs& A, const SurfCam& q, uint32_t len, const CamSplit& cs,
+                                           uint32_t k, float acc[3], uint32_t& err) {
     float4 r0, r3;
-    if (!vm_take(A, k, q.camera_path_length, r0, r3, err)) return;
+    if (!vm_take(A, k, len, r0, r3, err)) return false;
     const float gx = r0.x, gy = r0.y, gz = r0.z;
     // Frame::ToLocal (Frame.hxx:69-72)
-    const float lx = dot3(gx, gy, gz, q.frame_x[0], q.frame_x[1], q.frame_x[2]);
-    const float ly = dot3(gx, gy, gz, q.frame_y[0], q.frame_y[1], q.frame_y[2]);
-    const float lz = dot3(gx, gy, gz, q.frame_z[0], q.frame_z[1], q.frame_z[2]);
-    const float fx = q.local_dir_fix[0], fy = q.local_dir_fix[1], fz = q.local_dir_fix[2];
-    if (fabsf(lz) < kEpsCosine) return;  // too parallel with the tangent plane
-    if (lz * fz < 0.f) return;           // the other side of the surface
+    const float lx = dot3(gx, gy, gz, q.frame[0], q.frame[1], q.frame[2]);
+    const float ly = dot3(gx, gy, gz, q.frame[3], q.frame[4], q.frame[5]);
+    const float lz = dot3(gx, gy, gz, q.frame[6], q.frame[7], q.frame[8]);
+    const float fx = q.fix[0], fy = q.fix[1], fz = q.fix[2];
+    if (fabsf(lz) < kEpsCosine) return false;  // too parallel with the tangent plane
+    if (lz * fz < 0.f) return false;           // the other side of the surface
     float f0 = 0.f, f1 = 0.f, f2 = 0.f, dir_pdf = 0.f, rev_pdf = 0.f;
     const bool lobes = !(fz < kEpsCosine || lz < kEpsCosine);
     if (q.diff_prob != 0.f && lobes) {
@@ -376,7 +408,7 @@ __device__ void vm_process(const VmArgs& A, const upbp_surf_query& q, const Surf
         // ReflectLocal(mLocalDirFix) = (-x, -y, z) (Utils2.hxx:374-377)
         const float dot_r = dot3(-fx, -fy, fz, lx, ly, lz);
         if (dot_r > kEpsPhong) {
-            const float e = q.phong_exponent;
+            const float e = q.exponent;
             const float pw = powf(dot_r, e);
             if (pw > 1e-20f) {  // Float::isPositive (Utils.hxx:109-111)
                 // PowerCosHemispherePdfW (Utils2.hxx:78-86), symmetric
@@ -390,25 +422,81 @@ __device__ void vm_process(const VmArgs& A, const upbp_surf_query& q, const Surf
             }
         }
     }
-    if (f0 <= 0.f && f1 <= 0.f && f2 <= 0.f) return;
-    const float cont_l = A.rec[kRecWords * (int64_t)k + 1].w;
-    vm_accumulate(A, k, v, cs, r3.x, 0.f, dir_pdf * q.continuation_prob, rev_pdf * cont_l, UPBP_SURF, f0, f1, f2,
-                  acc, err);
+    if (f0 <= 0.f && f1 <= 0.f && f2 <= 0.f) return false;
+    const float4 r1 = A.rec[kRecWords * (int64_t)k + 1];
+    vm_accumulate(A, k, r1, cs, r3.x, 0.f, dir_pdf * q.cont, rev_pdf * r1.w, UPBP_SURF, f0, f1, f2, acc, err);
+    return true;
 }
 
-// HashGrid::Process (HashGrid.hxx:130-186) over one lane's camera vertex.
+template <class Query>
+struct CameraOf;
+template <>
+struct CameraOf<upbp_pp3d_query> {
+    using type = Pp3dCam;
+};
+template <>
+struct CameraOf<upbp_surf_query> {
+    using type = SurfCam;
+};
+
+// A wave's hit queue (slot, owner lane), its lanes' camera state and their sums. The slots that a wave's
+// lanes test together are found within the radius by few of them (6 % of the tests on 1M camera
+// vertices x 2.5M in-medium vertices, 19 % on 3.5M surface vertices), and a merge costs ten times a
+// test, so it is not evaluated in place but 64 queued hits at a time.
+constexpr int kWaves = kBlock / 64;
+constexpr int kHitRing = 128;  // a ballot adds at most 64 to fewer than 64 queued
+template <class Cam>
+struct VmLds {
+    uint32_t slot[kWaves][kHitRing];
+    uint32_t owner[kWaves][kHitRing];
+    float cam[kWaves][Cam::kWords][64];
+    float acc[kWaves][3][64];
+};
+
+// Evaluates n (1..64) queued hits from ring position head on. The sums are LDS atomics of one wave, in
+// lane and so in queue order: each owner's terms are added in the order it found them.
+template <class Cam>
+__device__ __forceinline__ void vm_drain(const VmArgs& A, VmLds<Cam>& L, uint32_t head, uint32_t n, uint32_t& err) {
+    const int w = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u;
+    if (lane >= n) return;
+    const uint32_t at = (head + lane) & (kHitRing - 1);
+    const uint32_t k = L.slot[w][at], o = L.owner[w][at];
+    Cam c;
+    float* words = reinterpret_cast<float*>(&c);
+    for (int i = 0; i < Cam::kWords - kCamWords; ++i) words[i] = L.cam[w][kCamWords + i][o];
+    const CamSplit cs = {L.cam[w][1][o], L.cam[w][2][o], L.cam[w][3][o]};
+    float v[3];
+    if (!vm_process(A, c, __float_as_uint(L.cam[w][0][o]), cs, k, v, err)) return;
+    atomicAdd(&L.acc[w][0][o], v[0]);
+    atomicAdd(&L.acc[w][1][o], v[1]);
+    atomicAdd(&L.acc[w][2][o], v[2]);
+}
+
+// HashGrid::Process (HashGrid.hxx:130-186), one lane per camera vertex: the eight buckets' ranges are
+// read at once, then each bucket is walked kStep slots at a time, so that its loads are in flight
+// together. 1M camera vertices: PP3D 1.28 -> 0.00 ms, SURF 12.05 -> 0.00 ms.
 template <class Query, bool SIG>
 __global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __restrict__ queries) {
+    using Cam = typename CameraOf<Query>::type;
+    static_assert(sizeof(Cam) == (Cam::kWords - kCamWords) * 4, "camera state words");
+    constexpr int kStep = 4;
+    __shared__ VmLds<Cam> L;  // unused with SIG
+    const int w = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u;
     const int64_t slot = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const bool valid = slot < A.count;
     uint32_t err = 0, processed = 0, sig_h = 0;
     uint64_t tested = 0;
-    float acc[3] = {0.f, 0.f, 0.f};
-    int64_t qi = 0;
+    const int64_t qi = !valid ? 0 : A.perm ? (int64_t)A.perm[slot] : slot;
+    float x = 0.f, y = 0.f, z = 0.f;
+    uint32_t first[8] = {}, end[8] = {};  // no slots for a lane without a query
     if (valid) {
-        qi = A.perm ? (int64_t)A.perm[slot] : slot;
         const Query q = queries[qi];
         const bool ok = query_ok(A, q, err);
+        x = q.position[0];
+        y = q.position[1];
+        z = q.position[2];
         float dmin[3], dmax[3];
         for (int a = 0; a < 3; ++a) {
             dmin[a] = q.position[a] - A.g.lo[a];
@@ -416,12 +504,6 @@ __global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __res
         }
         if (ok && A.n_sel > 0 && !(dmin[0] < 0.f) && !(dmax[0] < 0.f) && !(dmin[1] < 0.f) && !(dmax[1] < 0.f) &&
             !(dmin[2] < 0.f) && !(dmax[2] < 0.f)) {
-            const auto cam = camera_of(A, q);
-            const CamSplit cs =
-                (SIG || (A.flags & UPBP_VM_NO_MIS))
-                    ? CamSplit{0.f, 0.f, 0.f}
-                    : camera_split(A.mis.camera + q.camera_offset, (int)q.camera_path_length,
-                                   A.mis.p.query_beam_type, A.mis.p.photon_beam_type, A.mis.p.techniques);
             int32_t p[3], po[3];
             for (int a = 0; a < 3; ++a) {
                 const float cp = A.g.inv_cell * dmin[a];
@@ -429,34 +511,92 @@ __global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __res
                 p[a] = (int32_t)cf;
                 po[a] = p[a] + ((cp - cf) < 0.5f ? -1 : 1);
             }
+#pragma unroll
             for (int j = 0; j < 8; ++j) {
                 // case order of HashGrid.hxx:163-172: x slowest, z fastest
                 const uint32_t c = bucket_of((j & 4) ? po[0] : p[0], (j & 2) ? po[1] : p[1], (j & 1) ? po[2] : p[2],
                                              A.g.cells);
-                uint32_t k = c == 0 ? 0u : A.ends[c - 1];
-                const uint32_t e = A.ends[c];
-                tested += e - k;
-                for (; k < e; ++k) {
-                    const float4 s = A.slots[k];
-                    const float dx = q.position[0] - s.x, dy = q.position[1] - s.y, dz = q.position[2] - s.z;
-                    if ((dx * dx + dy * dy) + dz * dz <= A.g.r2) {
-                        const uint32_t v = __float_as_uint(s.w);
+                first[j] = c == 0 ? 0u : A.ends[c - 1];
+                end[j] = A.ends[c];
+            }
+            if (!SIG) {
+                const Cam cam = camera_of(A, q);
+                const CamSplit cs = (A.flags & UPBP_VM_NO_MIS)
+                                        ? CamSplit{0.f, 0.f, 0.f}
+                                        : camera_split(A.mis.camera + q.camera_offset, (int)q.camera_path_length,
+                                                       A.mis.p.query_beam_type, A.mis.p.photon_beam_type,
+                                                       A.mis.p.techniques);
+                L.cam[w][0][lane] = __uint_as_float(q.camera_path_length);
+                L.cam[w][1][lane] = cs.a0;
+                L.cam[w][2][lane] = cs.bb0;
+                L.cam[w][3][lane] = cs.cn;
+                const float* words = reinterpret_cast<const float*>(&cam);
+                for (int i = 0; i < Cam::kWords - kCamWords; ++i) L.cam[w][kCamWords + i][lane] = words[i];
+            }
+        }
+    }
+    if (!SIG)
+        for (int c = 0; c < 3; ++c) L.acc[w][c][lane] = 0.f;
+    uint32_t head = 0, tail = 0;  // of the wave's ring (wave-uniform)
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) {
+        uint32_t k = first[0];
+        const uint32_t e = end[0];
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {  // the next bucket moves to the front: no indexed registers
+            first[i] = first[i + 1];
+            end[i] = end[i + 1];
+        }
+        tested += e - k;
+        for (; __ballot(k < e); k += kStep) {
+            bool hit[kStep];
+            uint32_t v[kStep];
+#pragma unroll
+            for (int i = 0; i < kStep; ++i) {
+                const uint32_t at = k + (uint32_t)i;
+                hit[i] = at < e;
+                v[i] = 0;
+                if (hit[i]) {
+                    const float4 s = A.slots[at];
+                    const float dx = x - s.x, dy = y - s.y, dz = z - s.z;
+                    hit[i] = (dx * dx + dy * dy) + dz * dz <= A.g.r2;
+                    v[i] = __float_as_uint(s.w);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kStep; ++i) {
+                if (SIG) {
+                    if (hit[i]) {
                         processed++;
-                        if (SIG)
-                            sig_h += hash32(v);
-                        else
-                            vm_process(A, q, cam, cs, k, v, acc, err);
+                        sig_h += hash32(v[i]);
                     }
+                    continue;
+                }
+                const uint64_t m = __ballot(hit[i]);
+                if (!m) continue;
+                if (hit[i]) {
+                    processed++;
+                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    const uint32_t at = (tail + rank) & (kHitRing - 1);
+                    L.slot[w][at] = k + (uint32_t)i;
+                    L.owner[w][at] = lane;
+                }
+                tail += (uint32_t)__popcll(m);
+                if (tail - head >= 64u) {
+                    vm_drain(A, L, head, 64u, err);
+                    head += 64u;
                 }
             }
         }
+    }
+    if (!SIG && tail != head) vm_drain(A, L, head, tail - head, err);
+    if (valid) {
         if (SIG) {
             A.sig[2 * qi] = processed;
             A.sig[2 * qi + 1] = sig_h;
         } else {
-            A.out[3 * qi] = acc[0];
-            A.out[3 * qi + 1] = acc[1];
-            A.out[3 * qi + 2] = acc[2];
+            for (int c = 0; c < 3; ++c) A.out[3 * qi + c] = L.acc[w][c][lane];
         }
     }
     // one atomic per wave for each counter
@@ -467,7 +607,7 @@ __global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __res
         ht += __shfl_xor(ht, off, 64);
         he |= __shfl_xor(he, off, 64);
     }
-    if ((threadIdx.x & 63) == 0 && A.count_stats) {
+    if (lane == 0 && A.count_stats) {
         unsigned long long* stats = A.stats + (slot / 64) % kStatRows * kStatSlots;
         if (hp) atomicAdd(stats + kStatPhotonHits, (unsigned long long)hp);
         if (ht) atomicAdd(stats + kStatPhotonCands, (unsigned long long)ht);
