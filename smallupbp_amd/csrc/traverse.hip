@@ -171,11 +171,11 @@ __device__ __forceinline__ int64_t uni64(int64_t x) { return (int64_t)uni_u64((u
 // Lane state of one segment being gathered.
 struct SegState {
     float tmin, tmax;
-    float st0, st1, st2;
+    float e0, e1, e2;  // sigma_t log2(e) per channel: transmittances are exp2(-e t)
+    float ek;          // the smallest sigma_t's (what SHORT beams are normalised by)
     float ss0, ss1, ss2;
-    float g;
-    int32_t iso;
-    int32_t kidx;
+    float g;           // 0 for isotropic media, where phase_pdf gives the constant exactly
+    int32_t kidx;      // the smallest sigma_t's channel (adjoint)
     int32_t medium;     // medium id (instance-local, for the beam medium test)
     float min_comp, mfp, cont;  // UPBP mode: min sigma_t component, mean free path, continuation
     float acc0, acc1, acc2;
@@ -196,6 +196,7 @@ struct LaneOut {
     uint32_t hits = 0;
     uint32_t sig_n = 0, sig_h = 0;
     uint32_t err = 0;
+    bool aniso = false;       // whether some lane's medium of the segment is anisotropic (wave-uniform)
     MisLane ml;               // UPBP mode only
     uint32_t qh = 0, qt = 0;  // UPBP mode: head and tail of the wave's hit queue (wave-uniform)
 };
@@ -228,20 +229,28 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
 }
 
 // ---- leaf visitors ---------------------------------------------------------
-// Exponent of the transmittance of channel c along `dist` with the SHORT
-// normalisation T_c / T_k folded in: exp(-st_c d + st_k d) = T_c(d) / T_k(d).
-__device__ __forceinline__ float neg_tau(float st_c, float st_k, float d, bool short_norm) {
-    return short_norm ? (st_k * d - st_c * d) : -(st_c * d);
+// One fused multiply-add and one exp2 per channel: the exponents with their products, differences and
+// selections, and the per-lane choice of phase function, were 50 of the 80 vector instructions of a beam
+// hit, which made 1920x1080 rays x 200k SHORT beams 11.8 ms; 10.9 ms with these and the record read
+// in one go (test_beam_beam).
+// exp2 of the channels' transmittance exponents along `dist` with the SHORT normalisations folded in:
+// exp2(-e_c dist + ek norm) = T_c(dist) / T_k(norm), norm the part of dist that is SHORT.
+struct Trans {
+    float c0, c1, c2;
+};
+__device__ __forceinline__ Trans transmittance(const SegState& s, float dist, float norm) {
+    const float k = s.ek * norm;
+    return {__builtin_amdgcn_exp2f(__builtin_fmaf(-s.e0, dist, k)), __builtin_amdgcn_exp2f(__builtin_fmaf(-s.e1, dist, k)),
+            __builtin_amdgcn_exp2f(__builtin_fmaf(-s.e2, dist, k))};
 }
 
-// Sums the three channels' item gradients over the wave (DPP) and adds them once.
+// Sums the three channels' item gradients over the wave (DPP) and adds them once: lanes 0 to 2 add one
+// channel each in one instruction, to neighbouring words (512x512 forward and adjoint: 10.6 ms with one
+// lane adding all three, 10.0 ms).
 __device__ __forceinline__ void add_item_gradient(float* grad, uint32_t o, float g0, float g1, float g2) {
     const float r0 = wave_sum_dpp(g0), r1 = wave_sum_dpp(g1), r2 = wave_sum_dpp(g2);
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        unsafeAtomicAdd(&grad[3 * o + 0], r0);
-        unsafeAtomicAdd(&grad[3 * o + 1], r1);
-        unsafeAtomicAdd(&grad[3 * o + 2], r2);
-    }
+    const int lane = threadIdx.x & (kWave - 1);
+    if (lane < 3) unsafeAtomicAdd(&grad[3 * o + lane], lane == 0 ? r0 : lane == 1 ? r1 : r2);
 }
 
 __device__ __forceinline__ MisF merge_vertex_mis(const upbp_mis_params& P, float pdf_a_inv, float ray_pdf_inv,
@@ -280,14 +289,9 @@ __device__ void photon_hit_mis(const EvalArgs& A, const Ray& r, SegState& s, con
     // rounding (hit decisions are all made before this point), so reciprocals and square
     // roots are the single hardware instructions.
     const float dt = t - s.tmin;
-    float a0 = fast_exp(-s.st0 * dt), a1 = fast_exp(-s.st1 * dt), a2 = fast_exp(-s.st2 * dt);
-    const float pdf = pick3(s.kidx, a0, a1, a2);
-    if (short_q) {
-        const float ip = __builtin_amdgcn_rcpf(pdf);
-        a0 *= ip;
-        a1 *= ip;
-        a2 *= ip;
-    }
+    const float pdf = __builtin_amdgcn_exp2f(-s.ek * dt);
+    const Trans tr = transmittance(s, dt, short_q ? dt : 0.f);
+    const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
     float ray_pdf = s.min_comp * pdf;
     float ray_rev = (ml.seg_flags & UPBP_ORIGIN_IN_MEDIUM) ? ray_pdf : pdf;
     const float ratio = __builtin_amdgcn_rcpf(s.min_comp);
@@ -297,7 +301,7 @@ __device__ void photon_hit_mis(const EvalArgs& A, const Ray& r, SegState& s, con
     // PhaseFunction::Evaluate(-ray.dir, lightDirection): cos = -dot(gen, fix) = dot(dir_fix, d)
     const float lx = rec.b.x, ly = rec.b.y, lz = rec.b.z;
     const float cos_t = -dot3(lx, ly, lz, -r.dx, -r.dy, -r.dz);
-    const float bsdf = phase_pdf(s.g, s.iso != 0, cos_t);
+    const float bsdf = phase_pdf(s.g, false, cos_t);
     const float sin_t = __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - cos_t * cos_t));
     if (bsdf <= 0.f) return;
     const float dir_pdf = bsdf * s.cont;
@@ -358,11 +362,9 @@ __device__ void beam_hit_mis(const EvalArgs& A, const Ray& r, SegState& s, const
     // 1e-4 budget: hardware reciprocals, and one exponential per channel for the query and
     // beam transmittances together (with the SHORT normalisations folded into the exponent).
     const float dq = t1 - s.tmin;
-    const float stk = pick3(s.kidx, s.st0, s.st1, s.st2);
-    const float pq = fast_exp(-stk * dq), pb = fast_exp(-stk * t2);
-    const float a0 = fast_exp(neg_tau(s.st0, stk, dq, short_q) + neg_tau(s.st0, stk, t2, short_b));
-    const float a1 = fast_exp(neg_tau(s.st1, stk, dq, short_q) + neg_tau(s.st1, stk, t2, short_b));
-    const float a2 = fast_exp(neg_tau(s.st2, stk, dq, short_q) + neg_tau(s.st2, stk, t2, short_b));
+    const float pq = __builtin_amdgcn_exp2f(-s.ek * dq), pb = __builtin_amdgcn_exp2f(-s.ek * t2);
+    const Trans tr = transmittance(s, dq + t2, (short_q ? dq : 0.f) + (short_b ? t2 : 0.f));
+    const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
     float rsp_q = s.min_comp * pq;
     float rsr_q = (ml.seg_flags & UPBP_ORIGIN_IN_MEDIUM) ? rsp_q : pq;
     float rsp_b = s.min_comp * pb;
@@ -375,7 +377,7 @@ __device__ void beam_hit_mis(const EvalArgs& A, const Ray& r, SegState& s, const
     rsr_b *= rec.ray_sample_rev_pdf;
     // PhaseFunction::Evaluate(-ray.direction, -beam.direction): cos = -dot(-d2, -d1)
     const float cos_t = -dot3(-d2x, -d2y, -d2z, -r.dx, -r.dy, -r.dz);
-    const float bsdf = phase_pdf(s.g, s.iso != 0, cos_t);
+    const float bsdf = phase_pdf(s.g, false, cos_t);
     if (bsdf <= 0.f) return;
     const float dir_pdf = bsdf * s.cont;
     const float rev_pdf = bsdf * s.cont;
@@ -455,15 +457,14 @@ __device__ __forceinline__ void owner_state(const Ray& r, const SegState& s, con
     ro.dy = from_lane(r.dy, owner);
     ro.dz = from_lane(r.dz, owner);
     so.tmin = from_lane(s.tmin, owner);
-    so.st0 = from_lane(s.st0, owner);
-    so.st1 = from_lane(s.st1, owner);
-    so.st2 = from_lane(s.st2, owner);
+    so.e0 = from_lane(s.e0, owner);
+    so.e1 = from_lane(s.e1, owner);
+    so.e2 = from_lane(s.e2, owner);
+    so.ek = from_lane(s.ek, owner);
     so.ss0 = from_lane(s.ss0, owner);
     so.ss1 = from_lane(s.ss1, owner);
     so.ss2 = from_lane(s.ss2, owner);
     so.g = from_lane(s.g, owner);
-    so.iso = from_lane(s.iso, owner);
-    so.kidx = from_lane(s.kidx, owner);
     so.min_comp = from_lane(s.min_comp, owner);
     so.mfp = from_lane(s.mfp, owner);
     so.cont = from_lane(s.cont, owner);
@@ -599,14 +600,10 @@ __device__ __forceinline__ void photon_leaf(const EvalArgs& A, const Ray& r, Seg
             float gp0 = 0.f, gp1 = 0.f, gp2 = 0.f;
             if (hit) {
                 const float dt = t - s.tmin;
-                const float stk = pick3(s.kidx, s.st0, s.st1, s.st2);
-                const float a0 = fast_exp(neg_tau(s.st0, stk, dt, short_q));
-                const float a1 = fast_exp(neg_tau(s.st1, stk, dt, short_q));
-                const float a2 = fast_exp(neg_tau(s.st2, stk, dt, short_q));
-                float ph;
-                if (s.iso) {
-                    ph = kInvPi * 0.25f;
-                } else {
+                const Trans tr = transmittance(s, dt, short_q ? dt : 0.f);
+                const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
+                float ph = kInvPi * 0.25f;
+                if (lo.aniso) {
                     const float4 in = A.inc[i];
                     ph = phase_pdf(s.g, false, dot3(in.x, in.y, in.z, r.dx, r.dy, r.dz));
                 }
@@ -834,10 +831,9 @@ __device__ __forceinline__ void beam_leaf(const EvalArgs& A, const Ray& r, SegSt
         const int32_t bmed = (int32_t)(word & kMediumMask);
         float dist, st, t1, t2, radius;
         // radius = mStartRadius (p1.w) + t2 * mRadiusChange (p3.y)
-        const bool hit = (bmed == s.medium) &&
-                         test_beam_beam(r.ox, r.oy, r.oz, r.dx, r.dy, r.dz, r.d1o1, s.tmin, s.tmax, pc.p0.x, pc.p0.y,
-                                        pc.p0.z, pc.p1.x, pc.p1.y, pc.p1.z, pc.p3.x, pc.p0.w, pc.p2.w, pc.p2.x,
-                                        pc.p2.y, pc.p1.w, pc.p3.y, dist, st, t1, t2, radius);
+        const bool hit = test_beam_beam(bmed == s.medium, r.ox, r.oy, r.oz, r.dx, r.dy, r.dz, r.d1o1, s.tmin, s.tmax,
+                                        pc.p0.x, pc.p0.y, pc.p0.z, pc.p1.x, pc.p1.y, pc.p1.z, pc.p3.x, pc.p0.w,
+                                        pc.p2.w, pc.p2.x, pc.p2.y, pc.p1.w, pc.p3.y, dist, st, t1, t2, radius);
         if ((MODE & 7) == (int)Mode::Upbp) {
             // per-cell reduction: a hit is queued with the times its cell tests it and the
             // cell's pdf, in place of the radius (recomputed from the piece when drained)
@@ -884,14 +880,14 @@ __device__ __forceinline__ void beam_leaf(const EvalArgs& A, const Ray& r, SegSt
             if (hit && red_n != 0) {
                 const bool short_b = (word & kShortBeamBit) != 0;
                 const float dq = t1 - s.tmin;
-                const float stk = pick3(s.kidx, s.st0, s.st1, s.st2);
-                // T(t1 - tmin) [/ T_k] * T(t2) [/ T_k(t2)], one exponential per channel
-                const float a0 = fast_exp(neg_tau(s.st0, stk, dq, short_q) + neg_tau(s.st0, stk, t2, short_b));
-                const float a1 = fast_exp(neg_tau(s.st1, stk, dq, short_q) + neg_tau(s.st1, stk, t2, short_b));
-                const float a2 = fast_exp(neg_tau(s.st2, stk, dq, short_q) + neg_tau(s.st2, stk, t2, short_b));
+                // T(t1 - tmin) [/ T_k] * T(t2) [/ T_k(t2)], one exponential per channel; the two
+                // normalised lengths are selected by scalar factors
+                const float kq = short_q ? 1.f : 0.f, kb = short_b ? 1.f : 0.f;
+                const Trans tr = transmittance(s, dq + t2, __builtin_fmaf(kq, dq, kb * t2));
+                const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
                 // phase: Evaluate(ray.direction, beam direction), cos = -dot(d2, d1)
-                const float ph = s.iso ? kInvPi * 0.25f
-                                       : phase_pdf(s.g, false, -dot3(pc.p1.x, pc.p1.y, pc.p1.z, r.dx, r.dy, r.dz));
+                const float ph = lo.aniso ? phase_pdf(s.g, false, -dot3(pc.p1.x, pc.p1.y, pc.p1.z, r.dx, r.dy, r.dz))
+                                          : kInvPi * 0.25f;
                 // 1D kernel (1 - dist^2/r^2) * 3 / (4 r sin(theta)), PhotonBeam.hxx:364-365
                 const float kern = radial_kernel(dist * dist, radius * radius);
                 float scale = (ph * kern * 3.0f) * __builtin_amdgcn_rcpf((4.0f * radius) * st);
@@ -1133,10 +1129,9 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
         SegState s;
         s.tmin = __builtin_inff();
         s.tmax = -__builtin_inff();
-        s.st0 = s.st1 = s.st2 = 0.f;
+        s.e0 = s.e1 = s.e2 = s.ek = 0.f;
         s.ss0 = s.ss1 = s.ss2 = 0.f;
         s.g = 0.f;
-        s.iso = 1;
         s.kidx = 0;
         s.medium = -1;
         s.acc0 = s.acc1 = s.acc2 = 0.f;
@@ -1174,14 +1169,14 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
                 if (scatter) {
                     s.tmin = tmin;
                     s.tmax = tmax;
-                    s.st0 = m->st[0];
-                    s.st1 = m->st[1];
-                    s.st2 = m->st[2];
+                    s.e0 = m->st[0] * kLog2e;
+                    s.e1 = m->st[1] * kLog2e;
+                    s.e2 = m->st[2] * kLog2e;
+                    s.ek = pick3(m->min_idx, s.e0, s.e1, s.e2);
                     s.ss0 = m->ss[0];
                     s.ss1 = m->ss[1];
                     s.ss2 = m->ss[2];
-                    s.g = m->g;
-                    s.iso = m->isotropic;
+                    s.g = m->isotropic ? 0.f : m->g;
                     s.kidx = m->min_idx;
                     s.min_comp = m->min_comp;
                     s.mfp = m->mfp;
@@ -1197,6 +1192,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
             s.w2 = W2 * P2;
         }
         if (__ballot(scatter)) {
+            lo.aniso = __ballot(s.g != 0.f) != 0;
             traverse<EST, MODE>(A, part, r, s, lo, short_q, nodes_visited, tests, overflow);
             if ((MODE & 7) == (int)Mode::Upbp) upbp_segment_end<EST, MODE>(A, r, s, lo, short_q);
         }

@@ -116,8 +116,9 @@ __device__ __forceinline__ float radial_kernel(float num, float den) {
 // reference's, on its own t2. d1o1 = dot3(d1, o1) and d2o2 = dot3(d2, o2) are passed in
 // precomputed (same operations, same values). The radius test decides with the exact
 // dist = |ad| / sqrt(s2) of the reference; dist and sin_theta are returned from the
-// reciprocal square root unless the test needed the exact values.
-__device__ __forceinline__ bool test_beam_beam(float o1x, float o1y, float o1z, float d1x, float d1y,
+// reciprocal square root unless the test needed the exact values. same_medium is not tested before the
+// line distance: a branch on it made the record's reads wait for one another.
+__device__ __forceinline__ bool test_beam_beam(bool same_medium, float o1x, float o1y, float o1z, float d1x, float d1y,
                                                float d1z, float d1o1, float min_t1, float max_t1, float o2x,
                                                float o2y, float o2z, float d2x, float d2y, float d2z,
                                                float d2o2, float len, float max_dist_sqr, float t_lo,
@@ -128,7 +129,7 @@ __device__ __forceinline__ bool test_beam_beam(float o1x, float o1y, float o1z, 
     const float cz = d1x * d2y - d1y * d2x;
     const float s2 = dot3(cx, cy, cz, cx, cy, cz);
     const float ad = dot3(o2x - o1x, o2y - o1y, o2z - o1z, cx, cy, cz);
-    if (ad * ad >= max_dist_sqr * s2) return false;
+    if (!((int)same_medium & (int)!(ad * ad >= max_dist_sqr * s2))) return false;
     const float q = dot3(d1x, d1y, d1z, d2x, d2y, d2z);
     const float q2m1 = q * q - 1.0f;
     if (q2m1 < 1e-5f && q2m1 > -1e-5f) return false;
@@ -163,8 +164,9 @@ __device__ __forceinline__ bool test_beam_beam(float o1x, float o1y, float o1z, 
     return ok;
 }
 
+constexpr float kLog2e = 1.4426950408889634f;
 // exp(x) for x <= 0 through the hardware base-2 exponential.
-__device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
+__device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
 // PhaseFunction::Pdf (PhaseFunction.hxx:52-80); cos_theta = -dot(gen, fix). It only
 // scales contributions and weights (no hit decision), so dd^(-3/2) is the hardware
