@@ -191,13 +191,21 @@ __global__ void k_beam_pieces(int64_t n, BeamIn b, const uint32_t* count, const 
 }
 
 __global__ void k_piece_gather(int64_t n, const uint32_t* order, const PieceDev* in, const float4* in_flux,
-                               const uint32_t* in_beam, PieceDev* out, float4* out_flux, uint32_t* out_beam) {
+                               const uint32_t* in_beam, PieceDev* out, float4* out_flux, uint32_t* out_beam,
+                               uint64_t* end_bits) {
     int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    uint32_t k = order[s];
-    out[s] = in[k];
-    out_flux[s] = in_flux[k];
-    out_beam[s] = in_beam[k];
+    bool end = false;
+    if (s < n) {
+        const uint32_t k = order[s];
+        const PieceDev pc = in[k];
+        out[s] = pc;
+        out_flux[s] = in_flux[k];
+        out_beam[s] = in_beam[k];
+        end = !(__builtin_isfinite(pc.p2.x) && __builtin_isfinite(pc.p2.y));
+    }
+    // one word per wave of 64 pieces (and the word after the last, when the grid has a wave for it)
+    const uint64_t m = __ballot(end);
+    if ((threadIdx.x & 63) == 0 && s <= n) end_bits[s >> 6] = m;
 }
 
 // Copy host arrays to device staging buffers when needed.
@@ -393,9 +401,10 @@ void beams_build(Ctx& ctx, const upbp_beam_input& in, const upbp_build_params& p
     out.piece.ensure(total * sizeof(PieceDev));
     out.piece_flux.ensure(total * 16);
     out.piece_beam.ensure(total * 4);
-    hipLaunchKernelGGL(k_piece_gather, dim3(grid_for(total)), dim3(kBlock), 0, st, total, order.as<uint32_t>(),
+    out.end_bits.ensure((size_t)(total / 64 + 2) * 8);
+    hipLaunchKernelGGL(k_piece_gather, dim3(grid_for(total + 64)), dim3(kBlock), 0, st, total, order.as<uint32_t>(),
                        pieces.as<PieceDev>(), flux.as<float4>(), piece_beam.as<uint32_t>(), out.piece.as<PieceDev>(),
-                       out.piece_flux.as<float4>(), out.piece_beam.as<uint32_t>());
+                       out.piece_flux.as<float4>(), out.piece_beam.as<uint32_t>(), out.end_bits.as<uint64_t>());
     UPBP_HIP(hipGetLastError());
     beam_reduction_build(ctx, n, b.origin, b.direction, b.length, out.r_start.as<float>(), out.r_end.as<float>(),
                          params, out);

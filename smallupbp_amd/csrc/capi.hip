@@ -305,6 +305,7 @@ BeamArgs beam_args(const Beams* b) {
     a.pieces = b->piece.as<PieceDev>();
     a.piece_flux = b->piece_flux.as<float4>();
     a.piece_beam = b->piece_beam.as<uint32_t>();
+    a.end_bits = b->end_bits.as<uint64_t>();
     a.pieces_n = b->pieces;
     a.red = b->red;
     return a;

@@ -38,6 +38,7 @@ struct EvalArgs {
     const float4* __restrict__ power;
     const float4* __restrict__ inc;
     const uint32_t* __restrict__ orig;  // photon original index / piece -> beam index
+    const uint64_t* __restrict__ end_bits;  // a bit per piece: a beam's first or last (one more word after)
     const PieceDev* __restrict__ pieces;
     const float4* __restrict__ piece_flux;
     // queries
@@ -190,6 +191,13 @@ struct SegState {
 constexpr int kReduced = 8;
 // With this bit a tile's items are split over several waves (the others keep their registers too).
 constexpr int kSplit = 16;
+// The plain modes evaluate the waves whose rays share their origin; with this bit (a launch of its own,
+// since its registers would cost the others) they evaluate the other waves.
+constexpr int kSparse = 32;
+// Whether a mode comes in those two launches.
+constexpr bool in_two(int mode) {
+    return ((mode & 7) == (int)Mode::Forward || (mode & 7) == (int)Mode::Signature) && !(mode & kReduced);
+}
 
 template <int MODE>
 struct LaneOut {
@@ -198,7 +206,7 @@ struct LaneOut {
     uint32_t err = 0;
     bool aniso = false;       // whether some lane's medium of the segment is anisotropic (wave-uniform)
     MisLane ml;               // UPBP mode only
-    uint32_t qh = 0, qt = 0;  // UPBP mode: head and tail of the wave's hit queue (wave-uniform)
+    uint32_t qh = 0, qt = 0;  // UPBP, kSparse: head and tail of the wave's queue (wave-uniform)
 };
 
 __device__ __forceinline__ float pick3(int k, float a, float b, float c) { return k == 0 ? a : (k == 1 ? b : c); }
@@ -935,15 +943,153 @@ __device__ __forceinline__ void beam_leaf(const EvalArgs& A, const Ray& r, SegSt
     }
 }
 
+// ---- pair queue of waves without a common origin -----------------------------
+// The rays of scattered paths share a wave but no direction: of 64 lanes only one or two meet the box of
+// a visited leaf (200k rays from points of the media: 47 million pieces with a ray within the radius
+// of their line, 1.9 rays each), so testing an item with the whole wave leaves nearly all lanes idle.
+// Where at most kSparseLanes lanes meet a leaf's box, its (lane, item) pairs are queued instead and
+// tested 64 at a time, a lane taking any ray and any item. An item is accepted only by rays that meet
+// its box (the boxes are widened for that), but for the pairs that a beam's first and last piece own
+// beyond its ends: those pieces are tested by the whole wave as ever.
+constexpr int kSparseLanes = 16;
+constexpr int kPq = 128;  // a leaf adds at most 64 pairs per lane to fewer than 64 queued
+__shared__ uint32_t g_pq[kHqWaves][2][kPq];
+
+// Tests the first n (1..64) queued pairs: [0] item, [1] lane.
+template <int EST, int MODE>
+__device__ __forceinline__ void drain_pairs(const EvalArgs& A, const Ray& r, const SegState& s, LaneOut<MODE>& lo,
+                                            uint32_t n, bool short_q) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const uint32_t pos = (lo.qh + (uint32_t)lane) & (kPq - 1);
+    const bool act = (uint32_t)lane < n;
+    const int owner = act ? (int)(g_pq[w][1][pos] & (kWave - 1)) : lane;
+    const uint32_t i = g_pq[w][0][pos];
+    const float ox = from_lane(r.ox, owner), oy = from_lane(r.oy, owner), oz = from_lane(r.oz, owner);
+    const float dx = from_lane(r.dx, owner), dy = from_lane(r.dy, owner), dz = from_lane(r.dz, owner);
+    const float tmin = from_lane(s.tmin, owner), tmax = from_lane(s.tmax, owner);
+    SegState so;
+    so.e0 = from_lane(s.e0, owner);
+    so.e1 = from_lane(s.e1, owner);
+    so.e2 = from_lane(s.e2, owner);
+    so.ek = from_lane(s.ek, owner);
+    const float ss0 = from_lane(s.ss0, owner), ss1 = from_lane(s.ss1, owner), ss2 = from_lane(s.ss2, owner);
+    const float g = from_lane(s.g, owner);
+    bool hit;
+    float c0 = 0.f, c1 = 0.f, c2 = 0.f;
+    if (EST == kEstPhotons) {
+        float t, sq;
+        const float4 p = A.pos_r2[act ? i : 0u];
+        hit = act && test_bre(ox, oy, oz, dx, dy, dz, tmin, tmax, p.x, p.y, p.z, p.w, t, sq);
+        if (hit && (MODE & 7) == (int)Mode::Forward) {
+            const float4 pw = A.power[i];
+            const float dt = t - tmin;
+            const Trans tr = transmittance(so, dt, short_q ? dt : 0.f);
+            float ph = kInvPi * 0.25f;
+            if (lo.aniso) {
+                const float4 in = A.inc[i];
+                ph = phase_pdf(g, false, dot3(in.x, in.y, in.z, dx, dy, dz));
+            }
+            const float scale = (ph * radial_kernel(sq, p.w)) * pw.w;
+            c0 = pw.x * (tr.c0 * scale) * ss0;
+            c1 = pw.y * (tr.c1 * scale) * ss1;
+            c2 = pw.z * (tr.c2 * scale) * ss2;
+        }
+    } else {
+        const float d1o1 = from_lane(r.d1o1, owner);
+        const int32_t medium = from_lane(s.medium, owner);
+        const PieceDev pc = A.pieces[act ? i : 0u];
+        const uint32_t word = __float_as_uint(pc.p2.z);
+        float dist, st, t1, t2, radius;
+        hit = test_beam_beam(act && (int32_t)(word & kMediumMask) == medium, ox, oy, oz, dx, dy, dz, d1o1, tmin, tmax,
+                             pc.p0.x, pc.p0.y, pc.p0.z, pc.p1.x, pc.p1.y, pc.p1.z, pc.p3.x, pc.p0.w, pc.p2.w, pc.p2.x,
+                             pc.p2.y, pc.p1.w, pc.p3.y, dist, st, t1, t2, radius);
+        if (hit && (MODE & 7) == (int)Mode::Forward) {
+            const float4 flux = A.piece_flux[i];
+            const float dq = t1 - tmin;
+            const Trans tr = transmittance(so, dq + t2, (short_q ? dq : 0.f) + ((word & kShortBeamBit) ? t2 : 0.f));
+            const float ph = lo.aniso ? phase_pdf(g, false, -dot3(pc.p1.x, pc.p1.y, pc.p1.z, dx, dy, dz))
+                                      : kInvPi * 0.25f;
+            const float kern = radial_kernel(dist * dist, radius * radius);
+            const float scale = (ph * kern * 3.0f) * __builtin_amdgcn_rcpf((4.0f * radius) * st);
+            c0 = flux.x * ss0 * (tr.c0 * scale);
+            c1 = flux.y * ss1 * (tr.c1 * scale);
+            c2 = flux.z * ss2 * (tr.c2 * scale);
+        }
+    }
+    if (hit) {
+        lo.hits++;
+        if ((MODE & 7) == (int)Mode::Signature) {
+            uint32_t* sums = reinterpret_cast<uint32_t*>(&g_hacc[w][0][0]);
+            atomicAdd(&sums[owner], 1u);
+            atomicAdd(&sums[kWave + owner], hash32(A.orig[i]));
+        } else {
+            atomicAdd(&g_hacc[w][0][owner], c0);
+            atomicAdd(&g_hacc[w][1][owner], c1);
+            atomicAdd(&g_hacc[w][2][owner], c2);
+        }
+    }
+    lo.qh += n;
+}
+
+// Queues the pairs of the lanes of `lanes` with the items start + j, j the bits of items.
+template <int EST, int MODE>
+__device__ __forceinline__ void queue_pairs(const EvalArgs& A, const Ray& r, const SegState& s, LaneOut<MODE>& lo,
+                                            uint64_t lanes, uint32_t start, uint64_t items, bool short_q) {
+    if (!items) return;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const uint32_t n = (uint32_t)__popcll(items), rank = lane_rank(items);
+    while (lanes) {
+        const uint32_t owner = (uint32_t)__builtin_ctzll(lanes);
+        lanes &= lanes - 1;
+        if ((items >> lane) & 1u) {
+            const uint32_t pos = (lo.qt + rank) & (kPq - 1);
+            g_pq[w][0][pos] = start + (uint32_t)lane;
+            g_pq[w][1][pos] = owner;
+        }
+        lo.qt = uni(lo.qt + n);
+        if (lo.qt - lo.qh >= (uint32_t)kWave) drain_pairs<EST, MODE>(A, r, s, lo, kWave, short_q);
+    }
+}
+
+// End of a segment: tests what is still queued and moves the owners' sums to their lanes.
+template <int EST, int MODE>
+__device__ __forceinline__ void sparse_segment_end(const EvalArgs& A, const Ray& r, SegState& s, LaneOut<MODE>& lo,
+                                                   bool short_q) {
+    const uint32_t n = uni(lo.qt - lo.qh);
+    if (n) drain_pairs<EST, MODE>(A, r, s, lo, n, short_q);
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    if ((MODE & 7) == (int)Mode::Signature) {
+        lo.sig_n += __float_as_uint(g_hacc[w][0][lane]);
+        lo.sig_h += __float_as_uint(g_hacc[w][1][lane]);
+    } else {
+        s.acc0 += g_hacc[w][0][lane];
+        s.acc1 += g_hacc[w][1][lane];
+        s.acc2 += g_hacc[w][2][lane];
+    }
+    for (int c = 0; c < 3; ++c) g_hacc[w][c][lane] = 0.f;
+}
+
+// Bits j of the pieces start + j (j < 64) that are a beam's first or last.
+__device__ __forceinline__ uint64_t end_pieces(const EvalArgs& A, uint32_t start) {
+    const uint64_t lo = A.end_bits[start >> 6], hi = A.end_bits[(start >> 6) + 1u];
+    const uint32_t sh = start & 63u;
+    return sh ? (lo >> sh) | (hi << (64u - sh)) : lo;
+}
+
 // ---- wave-cooperative traversal ------------------------------------------
-// The items [start, start + cnt) (cnt <= 64) of a leaf, culled against the wave's frustum first
-// when it has one.
+// The items [start, start + cnt) (cnt <= 64) of a leaf that the rays of `lanes` meet the box of, culled
+// against the wave's frustum first when it has one.
 template <int EST, int MODE>
 __device__ __forceinline__ void visit_leaf(const EvalArgs& A, const Frustum& F, bool fr, ItemPart part,
-                                           const Ray& r, SegState& s, LaneOut<MODE>& lo, uint32_t start,
-                                           uint32_t cnt, bool short_q, uint32_t& tested) {
+                                           uint64_t lanes, const Ray& r, SegState& s, LaneOut<MODE>& lo,
+                                           uint32_t start, uint32_t cnt, bool short_q, uint32_t& tested) {
     const uint64_t all = (MODE & kSplit) ? part.items(start, cnt) : cnt >= 64u ? ~0ull : ((1ull << cnt) - 1ull);
-    if (EST == kEstPhotons) {
+    if ((MODE & kSparse) && __popcll(lanes) <= kSparseLanes) {
+        const uint64_t ends = EST == kEstPhotons ? 0ull : end_pieces(A, start) & all;
+        tested += (uint32_t)__popcll(all);
+        if (EST == kEstBeams) beam_leaf<MODE>(A, r, s, lo, start, ends, short_q);
+        queue_pairs<EST, MODE>(A, r, s, lo, lanes, start, all & ~ends, short_q);
+    } else if (EST == kEstPhotons) {
         const uint64_t items = fr ? frustum_photons(A, F, start, cnt) & all : all;
         tested += (uint32_t)__popcll(items);
         photon_leaf<MODE>(A, r, s, lo, start, items, short_q);
@@ -964,7 +1110,7 @@ __device__ __forceinline__ void traverse(const EvalArgs& A, ItemPart part, const
     uint32_t node = A.root;
     uint32_t tested = 0;
     Frustum F;
-    const bool fr = make_frustum(r, s, F);
+    const bool fr = !(MODE & kSparse) && make_frustum(r, s, F);
     while (true) {
         node = uni(node);
         // One 64-byte scalar load for the whole node, then both slab tests without
@@ -988,8 +1134,8 @@ __device__ __forceinline__ void traverse(const EvalArgs& A, ItemPart part, const
         // subtree costs less as one leaf than as nodes (leaves stay small for the other waves).
         const bool leaf0 = any0 && (!(rr.z & kInner) || (fr && n0 <= A.frustum_leaf));
         const bool leaf1 = any1 && (!(rr.w & kInner) || (fr && n1 <= A.frustum_leaf));
-        if (leaf0) visit_leaf<EST, MODE>(A, F, fr, part, r, s, lo, s0, n0, short_q, tested);
-        if (leaf1) visit_leaf<EST, MODE>(A, F, fr, part, r, s, lo, s1, n1, short_q, tested);
+        if (leaf0) visit_leaf<EST, MODE>(A, F, fr, part, m0, r, s, lo, s0, n0, short_q, tested);
+        if (leaf1) visit_leaf<EST, MODE>(A, F, fr, part, m1, r, s, lo, s1, n1, short_q, tested);
         const bool go0 = any0 && !leaf0;
         const bool go1 = any1 && !leaf1;
         if (go0 && go1) {
@@ -1029,9 +1175,9 @@ __device__ __forceinline__ float* grad_row(const EvalArgs& A) {
 __shared__ float g_part[4][3][kWave];  // a split tile's sums per wave of the block
 
 // Processes the 64 queries of one tile (wave) against its part of the items. `slot0` is the first
-// lane slot.
+// lane slot. False: the tile is the other launch's (in_two), nothing was done.
 template <int EST, int MODE, bool KARG>
-__device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsigned long long* local_stats,
+__device__ bool run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsigned long long* local_stats,
                          float* lds_media /* adjoint: [lds_media_n][6][64] for this wave or null */) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t slot = slot0 + lane;
@@ -1063,6 +1209,13 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
             err |= kErrNonFinite;
             alive = false;
         }
+    }
+    if (KARG && in_two(MODE)) {
+        const uint64_t am = __ballot(alive);
+        const int fl = am ? __builtin_ctzll(am) : 0;
+        const float ox = __shfl(r.ox, fl, kWave), oy = __shfl(r.oy, fl, kWave), oz = __shfl(r.oz, fl, kWave);
+        const bool one = __ballot(alive && !(r.ox == ox && r.oy == oy && r.oz == oz)) == 0;
+        if (one == ((MODE & kSparse) != 0)) return false;
     }
     r.ix = guard_inv(r.dx);
     r.iy = guard_inv(r.dy);
@@ -1116,7 +1269,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
             }
         }
     }
-    if ((MODE & 7) == (int)Mode::Upbp) {
+    if ((MODE & 7) == (int)Mode::Upbp || (MODE & kSparse)) {
         const int w = threadIdx.x / kWave;
         g_hacc[w][0][lane] = 0.f;
         g_hacc[w][1][lane] = 0.f;
@@ -1195,6 +1348,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
             lo.aniso = __ballot(s.g != 0.f) != 0;
             traverse<EST, MODE>(A, part, r, s, lo, short_q, nodes_visited, tests, overflow);
             if ((MODE & 7) == (int)Mode::Upbp) upbp_segment_end<EST, MODE>(A, r, s, lo, short_q);
+            if (MODE & kSparse) sparse_segment_end<EST, MODE>(A, r, s, lo, short_q);
         }
         const EvalArgs& D = *reread<KARG>(A, nodes_visited);
         if (has) {
@@ -1329,6 +1483,7 @@ __device__ void run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
     local_stats[kStatNodes] += uni(nodes_visited);
     local_stats[kStatError] |= uni(e);
     local_stats[kStatOverflow] += uni(overflow);
+    return true;
 }
 
 // One wave's counters, in a row of its block's.
@@ -1358,7 +1513,7 @@ __device__ __forceinline__ int64_t xcd_block(int64_t bid, int64_t nblk) {
 // register spill cost less than the latency the extra wave hides (measured 3-4 %).
 // UPBP kernels ask for 4 (128 VGPRs), which both fit without spilling.
 template <int EST, int MODE>
-__global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7) == (int)Mode::Adjoint ? 1 : (MODE & kReduced) ? 6 : (MODE & 7) == (int)Mode::Forward ? 8 : 1)) void k_eval(
+__global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7) == (int)Mode::Adjoint ? 1 : (MODE & kReduced) ? 6 : (MODE & kSparse) ? 5 : (MODE & 7) == (int)Mode::Forward ? 8 : 1)) void k_eval(
     EvalArgs A) {
     const int wave_in_block = threadIdx.x / kWave;
     const int waves_per_block = blockDim.x / kWave;
@@ -1378,7 +1533,8 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
     const uint32_t tile = (MODE & kSplit) ? w / A.parts : w;
     const ItemPart part = {(MODE & kSplit) ? w % A.parts : 0u, A.parts - 1u, A.part_shift};
     const int64_t slot0 = (int64_t)tile * kWave;
-    if (slot0 < A.count) run_tile<EST, MODE, true>(A, slot0, part, ls, my_lds);
+    const bool ran = slot0 < A.count && run_tile<EST, MODE, true>(A, slot0, part, ls, my_lds);
+    if (in_two(MODE) && !ran) return;  // a block's waves agree: with kSplit they hold one tile, else none waits
     const EvalArgs& E = *reread<true>(A, (uint32_t)ls[kStatNodes]);
     if ((MODE & 7) != (int)Mode::Adjoint && (MODE & kSplit)) {
         // every wave of the block holds a part of this tile: lane l of wave c sums channel c of its slot
@@ -1614,6 +1770,14 @@ void launch_kernel(Ctx& ctx, const EvalArgs& A, unsigned blocks, unsigned thread
     else
         hipLaunchKernelGGL((k_eval<EST, MODE>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
     UPBP_HIP(hipGetLastError());
+    if constexpr (in_two(MODE)) {
+        if (A.count <= 1) return;  // one ray has one origin
+        if (A.parts > 1)
+            hipLaunchKernelGGL((k_eval<EST, MODE | kSplit | kSparse>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
+        else
+            hipLaunchKernelGGL((k_eval<EST, MODE | kSparse>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
+        UPBP_HIP(hipGetLastError());
+    }
 }
 
 template <int EST, int MODE>
@@ -1891,6 +2055,7 @@ void launch_beams(Ctx& ctx, Mode mode, const BeamArgs& bm, const QueryView& q, f
     A.pieces = bm.pieces;
     A.piece_flux = bm.piece_flux;
     A.orig = bm.piece_beam;
+    A.end_bits = bm.end_bits;
     A.red = bm.red;
     A.parts = q.parts[kEstBeams];
     A.part_shift = part_shift(bm.pieces_n, A.parts);

@@ -200,6 +200,7 @@ struct Beams {
     DevBuf piece;         // PieceDev [pieces]
     DevBuf piece_flux;    // float4 [pieces] throughput (rgb, 0)
     DevBuf piece_beam;    // uint32 [pieces] original beam index
+    DevBuf end_bits;      // a bit per piece, in uint64 words and one more: a beam's first or last
     DevBuf r_start, r_end;  // float [n] start / end radius the build gave each beam
     // per-cell beam reduction (max_beams_in_cell > 0): the reference grid's cell lists
     RedDev red;            // device view; red.max == 0 without reduction
@@ -334,6 +335,7 @@ struct BeamArgs {
     const PieceDev* pieces;
     const float4* piece_flux;
     const uint32_t* piece_beam;
+    const uint64_t* end_bits;
     int64_t pieces_n;
     RedDev red;
 };
