@@ -333,7 +333,8 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     if (timing) UPBP_HIP(hipEventRecord(ctx.ev[0], ctx.stream));
     float lo[3], hi[3];
     scene_bounds(bre, bm, lo, hi);
-    const uint32_t parts[2] = {want_ph ? split_parts(Q, bre->n) : 1, want_bm ? split_parts(Q, bm->pieces) : 1};
+    const uint32_t parts[2] = {want_ph ? split_parts(Q, bre->n, 0, mode) : 1,
+                               want_bm ? split_parts(Q, bm->pieces, 1, mode) : 1};
     uint32_t blocks[2] = {1, 1};  // the adjoint adds atomically
     if (mode != Mode::Adjoint)
         for (int e = 0; e < 2; ++e) blocks[e] = split_blocks(parts[e]);

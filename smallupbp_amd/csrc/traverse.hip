@@ -1973,11 +1973,12 @@ static void set_mis(EvalArgs& A, const MisDev* mis) {
     A.mis.p = mis->params;
 }
 
-uint32_t split_parts(int64_t count, int64_t items) {
+uint32_t split_parts(int64_t count, int64_t items, int est, Mode mode) {
     const int64_t tiles = (count + kWave - 1) / kWave;
     uint32_t parts = 1;
     if (items < kSplitFrom) return parts;
-    while (parts < kSplitMost && 2 * parts * tiles <= kSplitWaves && 2 * parts * kSplitItems <= items) parts *= 2;
+    const int64_t waves = mode == Mode::Upbp || est == kEstPhotons ? kSplitWavesLight : kSplitWaves;
+    while (parts < kSplitMost && 2 * parts * tiles <= waves && 2 * parts * kSplitItems <= items) parts *= 2;
     return parts;
 }
 

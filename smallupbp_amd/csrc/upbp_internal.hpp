@@ -245,13 +245,19 @@ struct QueryView {
 // partly idle, and one of a few times more waits for the waves that meet most of the items. So a
 // tile's items are split over as many waves as bring the launch to kSplitWaves, at most kSplitMost, each
 // for at least kSplitItems items. Structures of fewer than kSplitFrom items stay whole: little is left to
-// split there, and their sums stay the same bits as a batched plan's, which splits nothing. Measured unsplit / at 8192 / 16384 / 32768 / 65536 waves:
-//   64x36 rays x 20k photons + 2k beams       907 /  211 /  215 /  211 /  205 us
-//   512x512 rays, forward and adjoint       11.58 / 10.5 / 10.4 / 11.5 / 13.9 ms
-//   640x360 rays x 40k traced beams         24.59 / 14.9 /  9.2 /  6.7 /  5.6 ms
-//   200k rays without a common origin       36.95 / 23.3 / 20.9 / 19.9 / 20.6 ms
-// Above kSplitWaves tiles nothing is split: 1920x1080 rays took 12.4 ms either way at 2 parts, 13.7 at 4.
-constexpr int64_t kSplitWaves = 32768;
+// split there, and their sums stay the same bits as a batched plan's, which splits nothing. Every part
+// walks the top of the tree again, so photons, which are tested in less time than beams, and the UPBP
+// kernels, of which the GPU holds half as many waves, stop at kSplitWavesLight. Measured unsplit / at
+// 4096 / 8192 / 16384 / 32768 waves for every estimator:
+//   64x36 rays x 20k photons + 2k beams       820 /  206 /  220 /  212 /  213 us
+//   256x256 rays x 100k photons               282 /  216 /  231 /  250 /  326 us
+//   512x512 rays, forward and adjoint        9.73 / 9.80 / 9.99 / 9.00 / 10.1 ms
+//   640x360 rays x 40k traced beams          21.6 / 21.9 / 14.8 /  8.6 /  6.6 ms
+//   60k rays x 300k beams                    13.0 /  6.9 /  4.7 /  4.4 /  3.8 ms
+//   200k rays without a common origin        17.2 / 16.9 / 16.8 / 14.5 / 14.6 ms
+//   300x168 rays, UPBP                        699 /  445 /  504 /  637 /  892 us
+// Above that many tiles nothing is split: 1920x1080 rays took 12.4 ms either way at 2 parts, 13.7 at 4.
+constexpr int64_t kSplitWaves = 16384, kSplitWavesLight = 4096;
 constexpr int64_t kSplitItems = 256, kSplitFrom = 16384;
 constexpr uint32_t kSplitMost = 64;
 
@@ -384,7 +390,7 @@ void launch_beam_records(Ctx& ctx, MisDev& mis, int64_t n_beams);
 void launch_photon_records(Ctx& ctx, MisDev& mis);
 // How many waves share a tile's items in an evaluation of count queries against items items (a power
 // of two), and how many blocks they form.
-uint32_t split_parts(int64_t count, int64_t items);
+uint32_t split_parts(int64_t count, int64_t items, int estimator, Mode mode);
 uint32_t split_blocks(uint32_t parts);
 // Adds up a split evaluation's parts into the outputs (null: not evaluated), in query order.
 void launch_sum_parts(Ctx& ctx, const QueryView& q, float* ph, float* bm);
