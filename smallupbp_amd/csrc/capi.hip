@@ -54,9 +54,9 @@ struct upbp_batch_plan {
 // ends. In host code `scratch` names a host-side stand-in: only the address that
 // hipGetSymbolAddress returns for the current device (kept per device below) is ever used.
 constexpr size_t kScratchBytes = (size_t)UPBP_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kScratchStatsBytes = 4096;
+constexpr size_t kScratchStatsBytes = 8192;
 constexpr int64_t kScratchMaxSorted = UPBP_NOALLOC_MAX_SORTED_QUERIES;
-static_assert(kStatWords * 8 <= kScratchStatsBytes, "counters fit the scratch header");
+static_assert(kStatAll * 8 <= kScratchStatsBytes, "counters fit the scratch header");
 static_assert(kScratchStatsBytes + 4 * (size_t)kScratchMaxSorted * 4 < kScratchBytes, "scratch keeps room for the sort");
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -86,10 +86,10 @@ void* scratch_address(int device, std::string& why) {
     return g_scratch_ptr[device];
 }
 
-// The workspace carved out of a device's scratch region for a batch of `count` queries whose tiles
-// are split over `blocks` blocks per estimator: counters first, then the four key / permutation arrays, then the
-// sort storage in what remains below the blocks' sums at the end (none with one block).
-Workspace scratch_workspace(void* base, int64_t count, const uint32_t blocks[2]) {
+// The workspace carved out of a device's scratch region for a batch of `count` queries split as
+// `split` says per estimator: counters first, then the four key / permutation arrays, then the
+// sort storage in what remains below the splits' plans at the end.
+Workspace scratch_workspace(void* base, int64_t count, const Split split[2]) {
     Workspace w;
     char* p = static_cast<char*>(base);
     w.stats = reinterpret_cast<unsigned long long*>(p);
@@ -103,9 +103,9 @@ Workspace scratch_workspace(void* base, int64_t count, const uint32_t blocks[2])
     w.sort_tmp = p;
     char* end = static_cast<char*>(base) + kScratchBytes;
     for (int e = 0; e < 2; ++e)
-        if (blocks[e] > 1) {
-            end -= ((size_t)blocks[e] * count * 12 + 255) / 256 * 256;
-            w.partial[e] = reinterpret_cast<float*>(end);
+        if (const size_t bytes = TilePlan::bytes(split[e])) {
+            end -= (bytes + 255) / 256 * 256;
+            w.plan[e] = TilePlan::at(split[e], end);
         }
     w.sort_tmp_bytes = (size_t)(end - p);
     return w;
@@ -187,15 +187,15 @@ void check_batch(const Ctx& ctx, const upbp_query_batch* q) {
 }
 
 // The context's own workspace: its counters, for a sorted batch of Q queries its key and
-// permutation buffers and sort storage, and the sums of a split evaluation's parts, grown to fit.
-Workspace context_workspace(Ctx& ctx, const upbp_query_batch* q, const uint32_t blocks[2]) {
+// permutation buffers and sort storage, and the plans of a split evaluation, grown to fit.
+Workspace context_workspace(Ctx& ctx, const upbp_query_batch* q, const Split split[2]) {
     Workspace w;
     w.stats = ctx.stats.as<unsigned long long>();
     const int64_t Q = q->count;
     for (int e = 0; e < 2; ++e)
-        if (blocks[e] > 1) {
-            ctx.partial[e].ensure((size_t)blocks[e] * Q * 12);
-            w.partial[e] = ctx.partial[e].as<float>();
+        if (const size_t bytes = TilePlan::bytes(split[e])) {
+            ctx.plan[e].ensure(bytes);
+            w.plan[e] = TilePlan::at(split[e], ctx.plan[e].as<char>());
         }
     if (q->order == UPBP_ORDER_SORTED && Q > 64) {
         for (DevBuf* b : {&ctx.qkeys, &ctx.qkeys2, &ctx.qperm, &ctx.qperm2}) b->ensure((size_t)Q * 4);
@@ -333,19 +333,17 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     if (timing) UPBP_HIP(hipEventRecord(ctx.ev[0], ctx.stream));
     float lo[3], hi[3];
     scene_bounds(bre, bm, lo, hi);
-    const uint32_t parts[2] = {want_ph ? split_parts(Q, bre->n, 0, mode) : 1,
-                               want_bm ? split_parts(Q, bm->pieces, 1, mode) : 1};
-    uint32_t blocks[2] = {1, 1};  // the adjoint adds atomically
-    if (mode != Mode::Adjoint)
-        for (int e = 0; e < 2; ++e) blocks[e] = split_blocks(parts[e]);
-    const Workspace own = scratch_base ? scratch_workspace(scratch_base, Q, blocks) : context_workspace(ctx, q, blocks);
+    const Split split[2] = {want_ph ? split_of(Q, bre->n, 0, mode) : Split(),
+                            want_bm ? split_of(Q, bm->pieces, 1, mode) : Split()};
+    const Workspace own = scratch_base ? scratch_workspace(scratch_base, Q, split) : context_workspace(ctx, q, split);
     const Workspace* ws = &own;
     QueryView v = make_view(ctx, q, lo, hi, !want_bm, *ws);
     for (int e = 0; e < 2; ++e) {
-        v.parts[e] = parts[e];
-        v.partial[e] = ws->partial[e];
+        v.split[e] = split[e];
+        v.plan[e] = ws->plan[e];
+        v.plan[e].words = reinterpret_cast<PlanWords*>(ws->stats + kStatWords) + e;
     }
-    launch_clear_u64(ctx, (uint64_t*)ws->stats, kStatWords);
+    launch_clear_u64(ctx, (uint64_t*)ws->stats, kStatAll);
     // the UPBP light walks read per-vertex tails, built once here for both estimators
     MisDev mis_t;
     if (mis && mode == Mode::Upbp && Q > 0) {
@@ -410,12 +408,12 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     }
     if (timing) UPBP_HIP(hipEventRecord(ctx.ev[3], ctx.stream));
     if (overlap) UPBP_HIP(hipStreamWaitEvent(ctx.stream, ctx.join, 0));
-    if (blocks[0] > 1 || blocks[1] > 1) {
+    if (split[0].rows > 0 || split[1].rows > 0) {
         const bool ph = want_ph && bre->n > 0, bmv = want_bm && bm->pieces > 0;
         if (mode == Mode::Signature)
-            launch_sum_parts_sig(ctx, v, ph ? sph : nullptr, bmv ? sbm : nullptr);
+            launch_sum_rows_sig(ctx, v, ph ? sph : nullptr, bmv ? sbm : nullptr);
         else
-            launch_sum_parts(ctx, v, ph ? dph : nullptr, bmv ? dbm : nullptr);
+            launch_sum_rows(ctx, v, ph ? dph : nullptr, bmv ? dbm : nullptr);
     }
     if (out_mem == UPBP_MEM_HOST && Q > 0) {
         if (o.out_ph && want_ph) UPBP_HIP(hipMemcpyAsync(o.out_ph, dph, Q * 12, hipMemcpyDeviceToHost, ctx.stream));
@@ -467,7 +465,7 @@ upbp_status upbp_ctx_create(int device, upbp_ctx** out_ctx) {
         UPBP_HIP(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
         UPBP_HIP(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming));
         UPBP_HIP(hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming));
-        ctx->stats.ensure(kStatWords * 8);
+        ctx->stats.ensure(kStatAll * 8);
         ctx->scratch = scratch_address(device, ctx->scratch_error);
         *out_ctx = ctx;
         return UPBP_OK;

@@ -72,13 +72,14 @@ struct EvalArgs {
     uint32_t frustum_leaf;
     // per-cell beam reduction of the beam estimators (red.max == 0: none)
     RedDev red;
-    // a tile's items split over `parts` waves (a power of two): the waves of a block, parts of one
-    // tile, add their sums up in LDS, and each block's go to the outputs, or with several blocks per
-    // tile to partial[block of the tile][slot][3] (partial_sig: [2]), which k_sum_parts adds up
-    uint32_t parts;
-    uint32_t part_shift;
-    float* __restrict__ partial;
-    uint32_t* __restrict__ partial_sig;
+    // split tiles: wave w gathers part w % 2^log_parts of tile w / 2^log_parts into row row0 + w, or does
+    // tasks[w] (of plan->n_tasks; tile_task); a part's sums go to rows[row][3][64] (signatures: [2][64]),
+    // which k_sum_rows adds up
+    const uint2* __restrict__ tasks;
+    PlanWords* __restrict__ plan;
+    uint32_t shift;  // ItemPart::shift of one part; half the items per block for twice the parts, at least 64
+    uint32_t log_parts, row0;
+    float* __restrict__ rows;
 };
 
 // The items a wave gathers: the blocks of 2^shift items of leaf order whose index is p modulo
@@ -100,6 +101,32 @@ struct ItemPart {
         return all & mine;
     }
 };
+
+// The work of wave w of a split launch.
+struct TileTask {
+    uint32_t tile, row, log_parts;
+    ItemPart part;
+};
+constexpr uint32_t kTaskPartBits = 8, kTaskLogBits = 4;  // of a task's second word, then the row
+__device__ __forceinline__ TileTask tile_task(const uint2* tasks, uint32_t log_parts, uint32_t row0, uint32_t shift,
+                                              uint32_t w) {
+    TileTask t;
+    uint32_t p;
+    if (tasks) {
+        const uint2 v = tasks[w];
+        t.tile = v.x;
+        p = v.y & ((1u << kTaskPartBits) - 1u);
+        t.log_parts = (v.y >> kTaskPartBits) & ((1u << kTaskLogBits) - 1u);
+        t.row = v.y >> (kTaskPartBits + kTaskLogBits);
+    } else {
+        t.tile = w >> log_parts;
+        p = w & ((1u << log_parts) - 1u);
+        t.log_parts = log_parts;
+        t.row = row0 + w;
+    }
+    t.part = {p, (1u << t.log_parts) - 1u, (uint32_t)max((int)shift - (int)t.log_parts, 6)};
+    return t;
+}
 
 __device__ __forceinline__ float guard_inv(float d) {
     const float a = __builtin_fabsf(d) < 1e-20f ? __builtin_copysignf(1e-20f, d) : d;
@@ -1172,7 +1199,7 @@ __device__ __forceinline__ float* grad_row(const EvalArgs& A) {
     return as_global(A.grad_media) + (size_t)(blockIdx.x % kGradRows) * A.n_media * 6;
 }
 
-__shared__ float g_part[4][3][kWave];  // a split tile's sums per wave of the block
+__shared__ float g_part[4][3][kWave];  // the sums of a split launch's waves
 
 // Processes the 64 queries of one tile (wave) against its part of the items. `slot0` is the first
 // lane slot. False: the tile is the other launch's (in_two), nothing was done.
@@ -1450,7 +1477,7 @@ __device__ bool run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
     err |= lo.err;
     const EvalArgs& E = *reread<KARG>(A, nodes_visited);
     if (valid && (MODE & 7) != (int)Mode::Adjoint) {
-        if (MODE & kSplit) {  // the block adds its waves' parts up (block_sum)
+        if (MODE & kSplit) {  // k_eval stores them
             const int w = threadIdx.x / kWave;
             if ((MODE & 7) == (int)Mode::Signature) {
                 g_part[w][0][lane] = __uint_as_float(lo.sig_n);
@@ -1529,10 +1556,12 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
     EvalArgs A) {
     const int wave_in_block = threadIdx.x / kWave;
     const int waves_per_block = blockDim.x / kWave;
-    // the parts of a split tile are spread over the blocks already
-    const int64_t blk = (MODE & kSplit) ? xcd_block(blockIdx.x, gridDim.x)
-                                        : xcd_round_block(blockIdx.x, gridDim.x, kXcdChunk);
-    const int64_t wave = blk * waves_per_block + wave_in_block;  // parts of a tile are neighbours
+    // the parts of a split without a plan are spread over the blocks already
+    const int64_t blk = (MODE & kSplit) && !A.tasks ? xcd_block(blockIdx.x, gridDim.x)
+                                                    : xcd_round_block(blockIdx.x, gridDim.x, kXcdChunk);
+    // wave-uniform (fewer than 2^32 waves: at most 2^26 tiles, and splits only of small batches)
+    const uint32_t w = uni((uint32_t)(blk * waves_per_block + wave_in_block));
+    if ((MODE & kSplit) && A.tasks && w >= as_global(A.plan)->n_tasks) return;
     unsigned long long ls[kStatSlots] = {0, 0, 0, 0, 0, 0, 0, 0};
     // adjoint: per-lane medium gradient slabs, [lds_media_n][6][64] floats per wave, sized at launch
     extern __shared__ float lds_dyn[];
@@ -1542,34 +1571,34 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
         my_lds = lds_dyn + (size_t)wave_in_block * slab;
         for (int k = threadIdx.x & (kWave - 1); k < slab; k += kWave) my_lds[k] = 0.f;
     }
-    // wave-uniform (fewer than 2^32 waves: at most 2^26 tiles, and parts > 1 only for small batches)
-    const uint32_t w = uni((uint32_t)wave);
-    const uint32_t tile = (MODE & kSplit) ? w / A.parts : w;
-    const ItemPart part = {(MODE & kSplit) ? w % A.parts : 0u, A.parts - 1u, A.part_shift};
+    ItemPart part = {0u, 0u, 6u};
+    uint32_t tile = w;
+    if (MODE & kSplit) {
+        const TileTask t = tile_task(as_global(A.tasks), A.log_parts, A.row0, A.shift, w);
+        tile = t.tile;
+        part = t.part;
+    }
     const int64_t slot0 = (int64_t)tile * kWave;
     const bool ran = slot0 < A.count && run_tile<EST, MODE, true>(A, slot0, part, ls, my_lds);
-    if (in_two(MODE) && !ran) return;  // a block's waves agree: with kSplit they hold one tile, else none waits
+    if (in_two(MODE) && !ran) return;
     const EvalArgs& E = *reread<true>(A, (uint32_t)ls[kStatNodes]);
     if ((MODE & 7) != (int)Mode::Adjoint && (MODE & kSplit)) {
-        // every wave of the block holds a part of this tile: lane l of wave c sums channel c of its slot
-        __syncthreads();
         constexpr int kN = (MODE & 7) == (int)Mode::Signature ? 2 : 3;
-        const uint32_t blocks = E.parts / (uint32_t)waves_per_block, b = part.p / (uint32_t)waves_per_block;
+        const TileTask t = tile_task(as_global(E.tasks), E.log_parts, E.row0, E.shift, w);
         const int lane = threadIdx.x & (kWave - 1);
-        const int64_t slot = slot0 + lane;
-        if (slot < E.count)
-            for (int c = wave_in_block; c < kN; c += waves_per_block) {
-                const int64_t at = blocks > 1 ? (int64_t)b * E.count + slot : E.perm ? (int64_t)as_global(E.perm)[slot] : slot;
-                if ((MODE & 7) == (int)Mode::Signature) {
-                    uint32_t v = 0;
-                    for (int k = 0; k < waves_per_block; ++k) v += __float_as_uint(g_part[k][c][lane]);
-                    as_global(blocks > 1 ? E.partial_sig : E.sig)[kN * at + c] = v;
-                } else {
-                    float v = 0.f;
-                    for (int k = 0; k < waves_per_block; ++k) v += g_part[k][c][lane];
-                    as_global(blocks > 1 ? E.partial : E.out)[kN * at + c] = v;
-                }
+        const int64_t slot = (int64_t)t.tile * kWave + lane;
+        if (slot < E.count) {
+            float* out;
+            int64_t step = 1;
+            if (t.log_parts == 0) {
+                out = (kN == 2 ? (float*)as_global(E.sig) : as_global(E.out)) +
+                      kN * (E.perm ? (int64_t)as_global(E.perm)[slot] : slot);
+            } else {
+                out = as_global(E.rows) + (size_t)t.row * kN * kWave + lane;
+                step = kWave;
             }
+            for (int c = 0; c < kN; ++c) out[c * step] = g_part[wave_in_block][c][lane];
+        }
     }
     if ((MODE & 7) == (int)Mode::Adjoint) {
         // reduce the per-lane medium slabs of this wave and add them once
@@ -1639,24 +1668,266 @@ __global__ void k_rebase_nodes(NodeDev* nodes, int64_t n, uint32_t node_off, uin
     nodes[i].r = r;
 }
 
-// Adds up the blocks' sums of a split evaluation in block order (one thread per value in slot order;
-// an output that is null was written by its blocks).
+// Adds up the rows of split tiles in the order of their parts: one block per tile, whose waves take
+// every fourth row. Row 0 of the grid's y is the photons', row 1 the beams' (null out: nothing to add).
+template <class T>
+struct SumRows {
+    const uint2* info;  // a planned tile's {log2 of its parts, first row}
+    uint32_t log_parts;
+    const T* rows;
+    T* out;
+};
 template <class T, int N>
-__global__ void k_sum_parts(int64_t n, const uint32_t* __restrict__ perm, uint32_t blocks_a, const T* __restrict__ pa,
-                            T* __restrict__ a, uint32_t blocks_b, const T* __restrict__ pb, T* __restrict__ b) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= N * n) return;
-    const int64_t slot = i / N, c = i % N;
-    const int64_t at = N * (perm ? (int64_t)perm[slot] : slot) + c;
-    if (a) {
-        T v = 0;
-        for (uint32_t k = 0; k < blocks_a; ++k) v += pa[N * n * k + i];
-        a[at] = v;
+__global__ __launch_bounds__(256) void k_sum_rows(int64_t n, const uint32_t* __restrict__ perm, SumRows<T> a,
+                                                  SumRows<T> b) {
+    __shared__ T part[4][N][kWave];
+    const SumRows<T> s = blockIdx.y ? b : a;
+    if (!s.out) return;
+    const uint32_t tile = blockIdx.x;
+    const uint2 info = s.info ? s.info[tile] : make_uint2(s.log_parts, tile << s.log_parts);
+    if (info.x == 0) return;  // written by its wave
+    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const int64_t slot = (int64_t)tile * kWave + lane;
+    T v[N] = {};
+    if (slot < n)
+        for (uint32_t k = w; k < (1u << info.x); k += 4)
+            for (int c = 0; c < N; ++c) v[c] += s.rows[((size_t)(info.y + k) * N + c) * kWave + lane];
+    for (int c = 0; c < N; ++c) part[w][c][lane] = v[c];
+    __syncthreads();
+    if (w < N && slot < n)
+        s.out[N * (perm ? (int64_t)perm[slot] : slot) + w] =
+            ((part[0][w][lane] + part[1][w][lane]) + part[2][w][lane]) + part[3][w][lane];
+}
+
+// ---- tile plans ----------------------------------------------------------------
+// What a tile costs is estimated before a split launch, so that expensive tiles are split into more parts
+// than cheap ones and start first. Parts of equal number left a launch waiting for a few waves: of
+// 640x360 rays on traced beams the longest wave took 5.8 ms, 20 times the average.
+//
+// Estimate, one wave per tile: the subtrees of at most frustum_leaf items whose boxes meet the cone
+// around the tile's rays within the segments that scatter, 64 nodes at a time (a lane tests a node, where
+// the gather tests one node with all rays), weighed as the gather's instruction counts are. Nothing but
+// the order and the number of the parts depends on it.
+constexpr int kCostQueue = 1024;            // nodes that wait; what does not fit counts without being opened
+constexpr int kCostSteps = 64;              // as does what is left after so many steps, or a 128th of the tiles
+constexpr uint32_t kCostOther = 0xFFFFFFFFu;  // a wave without a common origin
+
+template <int EST>
+__global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, int steps, uint32_t* __restrict__ cost) {
+    __shared__ uint32_t queue[4][kCostQueue];
+    constexpr float kNode = 46.f, kLeaf = 73.f, kItem = EST == kEstPhotons ? 8.f : 20.f, kTile = 500.f;
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t tile = uni(blockIdx.x * 4u + threadIdx.x / kWave);
+    const int64_t slot = (int64_t)tile * kWave + lane;
+    if ((int64_t)tile * kWave >= A.count) return;
+    uint32_t* const nodes = queue[threadIdx.x / kWave];
+    float ox = 0.f, oy = 0.f, oz = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
+    float t0 = __builtin_inff(), t1 = -__builtin_inff();
+    if (slot < A.count) {
+        const int64_t q = A.perm ? (int64_t)A.perm[slot] : slot;
+        ox = A.origin[3 * q], oy = A.origin[3 * q + 1], oz = A.origin[3 * q + 2];
+        dx = A.direction[3 * q], dy = A.direction[3 * q + 1], dz = A.direction[3 * q + 2];
+        const int64_t s0 = A.offsets[q], s1 = A.offsets[q + 1];
+        if (s0 >= 0 && s0 <= s1 && s1 <= A.offsets[A.count] && finite3(ox, oy, oz) && finite3(dx, dy, dz))
+            for (int64_t k = s0; k < s1; ++k) {
+                const upbp_volume_segment* sg = A.segments + k;
+                const int32_t m = sg->medium_id;
+                if (m < 0 || m >= A.n_media) break;
+                if (A.media[m].has_scattering) {
+                    t0 = fminf(t0, sg->dist_min);
+                    t1 = fmaxf(t1, sg->dist_max);
+                }
+            }
     }
-    if (b) {
-        T v = 0;
-        for (uint32_t k = 0; k < blocks_b; ++k) v += pb[N * n * k + i];
-        b[at] = v;
+    const uint64_t am = __ballot(t0 <= t1);
+    float c = 0.f;
+    bool one = true;
+    if (am) {
+        const int fl = __builtin_ctzll(am);
+        const bool on = t0 <= t1;
+        const float px = __shfl(ox, fl, kWave), py = __shfl(oy, fl, kWave), pz = __shfl(oz, fl, kWave);
+        one = __ballot(on && !(ox == px && oy == py && oz == pz)) == 0;
+        const float len = __builtin_sqrtf((dx * dx + dy * dy) + dz * dz);
+        const float il = on && len > 0.f ? 1.f / len : 0.f;
+        const float ux = dx * il, uy = dy * il, uz = dz * il;
+        float ax = ux, ay = uy, az = uz, lo = on ? t0 * len : __builtin_inff(), hi = on ? t1 * len : 0.f;
+        for (int off = 32; off > 0; off >>= 1) {
+            ax += __shfl_xor(ax, off, kWave);
+            ay += __shfl_xor(ay, off, kWave);
+            az += __shfl_xor(az, off, kWave);
+            lo = fminf(lo, __shfl_xor(lo, off, kWave));
+            hi = fmaxf(hi, __shfl_xor(hi, off, kWave));
+        }
+        const float al = __builtin_sqrtf((ax * ax + ay * ay) + az * az);
+        const float ia = al > 0.f ? 1.f / al : 0.f;
+        ax *= ia, ay *= ia, az *= ia;
+        float cs = on ? (ux * ax + uy * ay) + uz * az : 1.f;
+        for (int off = 32; off > 0; off >>= 1) cs = fminf(cs, __shfl_xor(cs, off, kWave));
+        const float tn = cs > 0.1f ? __builtin_sqrtf(fmaxf(1.f - cs * cs, 0.f)) / cs : 10.f;
+        const float ix = guard_inv(ax), iy = guard_inv(ay), iz = guard_inv(az);
+        int head = 0, size = one ? 1 : 0;
+        if (lane == 0) nodes[0] = A.root;
+        for (int step = 0; size > 0; ++step) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int n = min(size, kWave), from = head;
+            head = (head + n) % kCostQueue;
+            size -= n;
+            bool go[2] = {false, false};
+            uint32_t ref[2] = {0u, 0u};
+            float skipped[2] = {0.f, 0.f};
+            if (lane < n) {
+                const NodeDev nd = A.nodes[nodes[(from + lane) % kCostQueue]];
+                const float bl[2][3] = {{nd.a.x, nd.a.y, nd.a.z}, {nd.b.z, nd.b.w, nd.c.x}};
+                const float bh[2][3] = {{nd.a.w, nd.b.x, nd.b.y}, {nd.c.y, nd.c.z, nd.c.w}};
+                const uint32_t kind[2] = {nd.r.z, nd.r.w};
+                ref[0] = nd.r.x, ref[1] = nd.r.y;
+                c += kNode;
+                for (int k = 0; k < 2; ++k) {
+                    if (kind[k] == kInvalid) continue;
+                    // the axis against the box, widened by the cone's radius at the box's far side
+                    const float mx = 0.5f * (bl[k][0] + bh[k][0]) - px, my = 0.5f * (bl[k][1] + bh[k][1]) - py,
+                                mz = 0.5f * (bl[k][2] + bh[k][2]) - pz;
+                    const float hx = 0.5f * (bh[k][0] - bl[k][0]), hy = 0.5f * (bh[k][1] - bl[k][1]),
+                                hz = 0.5f * (bh[k][2] - bl[k][2]);
+                    const float rad = __builtin_amdgcn_sqrtf((hx * hx + hy * hy) + hz * hz);
+                    const float far = __builtin_amdgcn_sqrtf((mx * mx + my * my) + mz * mz) + rad;
+                    const float e = fmaxf(tn * fminf(far, hi), 1e-30f);
+                    const float wx = (hx + e) * __builtin_fabsf(ix), wy = (hy + e) * __builtin_fabsf(iy),
+                                wz = (hz + e) * __builtin_fabsf(iz);
+                    const float cx = mx * ix, cy = my * iy, cz = mz * iz;
+                    const float near = fmaxf(fmaxf(cx - wx, cy - wy), fmaxf(cz - wz, lo));
+                    const float past = fminf(fminf(cx + wx, cy + wy), fminf(cz + wz, hi));
+                    if (!(near <= past)) continue;
+                    const uint32_t items = kind[k] & kSpanMask;
+                    float cost = kLeaf + (kLeaf / 64.f + kItem) * (float)items;
+                    if ((kind[k] & kInner) && items > A.frustum_leaf) {
+                        // of a larger subtree, the runs of 64 items that the cone crosses
+                        const float part = __builtin_amdgcn_exp2f(
+                            __builtin_amdgcn_logf((float)A.frustum_leaf / (float)items) * (1.f / 3.f));
+                        const float f = (e + part * rad) * __builtin_amdgcn_rcpf(e + rad);
+                        cost *= f * f;
+                        go[k] = step < steps;
+                    }
+                    if (go[k])
+                        skipped[k] = cost;
+                    else
+                        c += cost;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();  // the popped entries are read before others take their place
+            for (int k = 0; k < 2; ++k) {
+                const uint64_t m = __ballot(go[k]);
+                const int at = size + __builtin_popcountll(m & ((1ull << lane) - 1ull));
+                if (go[k]) {
+                    if (at < kCostQueue)
+                        nodes[(head + at) % kCostQueue] = ref[k];
+                    else
+                        c += skipped[k];
+                }
+                size = min(size + __builtin_popcountll(m), kCostQueue);
+            }
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);
+    if (lane == 0) {
+        const uint32_t v = (uint32_t)fminf(c + kTile, 4e9f);
+        cost[tile] = one ? v : kCostOther;
+        if (one) {
+            PlanWords* p = A.plan;
+            atomicAdd(&p->total[blockIdx.x % 64][0], (unsigned long long)v);
+            atomicAdd(&p->total[blockIdx.x % 64][1], 1ull);
+        }
+    }
+}
+
+// Parts per tile: the share of `waves` that its cost is of the whole, rounded down to a power of two, so
+// that all parts together are no more than `waves`. Then a counting sort of the parts by what one costs,
+// in quarter octaves, dearest first.
+constexpr uint32_t kNoTask = 64;
+struct PlanArgs {
+    int64_t tiles;
+    uint32_t waves, log_most, log_other;  // log_other: of tiles without an estimate
+    bool other_apart;                     // those are another launch's, with their rows after the plan's
+    const uint32_t* cost;
+    uint2* info;  // {log2 of the parts, first row}; k_plan_parts leaves the bucket in y
+    uint2* tasks;
+    PlanWords* words;
+};
+
+__global__ __launch_bounds__(256) void k_plan_parts(PlanArgs P) {
+    __shared__ uint32_t hist[64];
+    __shared__ float share;
+    if (threadIdx.x < 64) {
+        hist[threadIdx.x] = 0;
+        unsigned long long t = P.words->total[threadIdx.x][0], n = P.words->total[threadIdx.x][1];
+        for (int off = 32; off > 0; off >>= 1) {
+            t += __shfl_xor(t, off, kWave);
+            n += __shfl_xor(n, off, kWave);
+        }
+        if (threadIdx.x == 0)
+            share = (float)((double)P.waves * (double)n / ((double)P.tiles * (double)(t > 0 ? t : 1)));
+    }
+    __syncthreads();
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < P.tiles) {
+        const uint32_t c = P.cost[i];
+        uint32_t lg = P.log_other, bucket = 0;
+        if (c != kCostOther) {
+            const float want = (float)c * share;
+            lg = 0;
+            while (lg < P.log_most && want >= (float)(2u << lg)) ++lg;
+            const int q = (int)(__float_as_uint(want / (float)(1u << lg)) >> 21) - (int)(__float_as_uint(1.f) >> 21);
+            bucket = (uint32_t)min(max(24 - q, 0), 63);
+        }
+        if (c == kCostOther && P.other_apart) bucket = kNoTask;
+        P.info[i] = make_uint2(lg, bucket);
+        if (bucket != kNoTask) atomicAdd(&hist[bucket], 1u << lg);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64 && hist[threadIdx.x]) atomicAdd(&P.words->hist[threadIdx.x], hist[threadIdx.x]);
+}
+
+__global__ __launch_bounds__(256) void k_plan_tasks(PlanArgs P) {
+    __shared__ uint32_t base[64], taken[64], rows, row_base;
+    if (threadIdx.x < 64) {
+        const uint32_t h = P.words->hist[threadIdx.x];
+        uint32_t x = h;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t y = __shfl_up(x, off, kWave);
+            x += (int)threadIdx.x >= off ? y : 0u;
+        }
+        base[threadIdx.x] = x - h;
+        taken[threadIdx.x] = 0;
+        if (threadIdx.x == 63 && blockIdx.x == 0) P.words->n_tasks = x;
+        if (threadIdx.x == 0) rows = 0;
+    }
+    __syncthreads();
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    uint2 info = make_uint2(0u, kNoTask);
+    uint32_t at = 0, row = 0;
+    if (i < P.tiles) info = P.info[i];
+    if (info.y != kNoTask) {
+        at = atomicAdd(&taken[info.y], 1u << info.x);
+        if (info.x) row = atomicAdd(&rows, 1u << info.x);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64 && taken[threadIdx.x])
+        base[threadIdx.x] += atomicAdd(&P.words->cursor[threadIdx.x], taken[threadIdx.x]);
+    if (threadIdx.x == 64) row_base = atomicAdd(&P.words->n_rows, rows);
+    __syncthreads();
+    const bool task = info.y != kNoTask;
+    at += task ? base[info.y] : 0u;
+    row = task ? row + row_base : P.waves + ((uint32_t)i << info.x);
+    if (i < P.tiles) P.info[i] = make_uint2(info.x, row);
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t first = (uint32_t)(i - lane);
+    for (uint64_t m = __ballot(task); m; m &= m - 1) {  // the wave writes each tile's tasks together
+        const int k = __builtin_ctzll(m);
+        const uint32_t lg = __shfl(info.x, k, kWave), to = __shfl(at, k, kWave), r = __shfl(row, k, kWave);
+        for (uint32_t j = lane; j < (1u << lg); j += kWave)
+            P.tasks[to + j] =
+                make_uint2(first + k, j | (lg << kTaskPartBits) | ((r + j) << (kTaskPartBits + kTaskLogBits)));
     }
 }
 
@@ -1777,41 +2048,77 @@ inline unsigned grid_for(int64_t n, int block = 256) {
     return (unsigned)std::max<int64_t>(1, (n + block - 1) / block);
 }
 
-template <int EST, int MODE>
-void launch_kernel(Ctx& ctx, const EvalArgs& A, unsigned blocks, unsigned threads, size_t lds) {
-    if (A.parts > 1)
-        hipLaunchKernelGGL((k_eval<EST, MODE | kSplit>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
-    else
-        hipLaunchKernelGGL((k_eval<EST, MODE>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
-    UPBP_HIP(hipGetLastError());
-    if constexpr (in_two(MODE)) {
-        if (A.count <= 1) return;  // one ray has one origin
-        if (A.parts > 1)
-            hipLaunchKernelGGL((k_eval<EST, MODE | kSplit | kSparse>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
-        else
-            hipLaunchKernelGGL((k_eval<EST, MODE | kSparse>), dim3(blocks), dim3(threads), lds, ctx.stream, A);
-        UPBP_HIP(hipGetLastError());
-    }
+// 2^shift items per block of a split, 64 or more (ItemPart::items): 32 to 64 blocks per part where there
+// are enough. Fewer balance worse (8: 22.0 against 20.0 ms on 200k rays without a common origin, 7.9
+// against 7.0 ms on traced beams), more make every part walk more of the tree.
+static uint32_t part_shift(int64_t items) {
+    uint32_t shift = 0;
+    while (((int64_t)32 << (shift + 1)) <= items) ++shift;
+    return shift;
 }
 
 template <int EST, int MODE>
-void launch_reduced(Ctx& ctx, const EvalArgs& A, unsigned blocks, unsigned threads, size_t lds = 0) {
-    if constexpr (EST == kEstBeams) {
-        if (A.red.max != 0) return launch_kernel<EST, MODE | kReduced>(ctx, A, blocks, threads, lds);
+void launch_waves(Ctx& ctx, const EvalArgs& A, int64_t waves, int tuned) {
+    // the tuned number of waves per block, 4 with tasks, or up to 4 parts of one tile
+    const bool adjoint = (MODE & 7) == (int)Mode::Adjoint;
+    const int wpb = A.tasks || (adjoint && A.log_parts == 0) ? 4
+                    : A.log_parts > 0                        ? std::min(1 << A.log_parts, 4)
+                                                             : std::min(std::max(tuned, 1), 4);
+    const dim3 blocks((unsigned)((waves + wpb - 1) / wpb)), threads((unsigned)(wpb * kWave));
+    // LDS gradient slabs for the media actually present: fewer bytes, more resident waves
+    const size_t lds = adjoint ? (size_t)wpb * A.lds_media_n * 6 * kWave * sizeof(float) : 0;
+    if (A.tasks || A.log_parts > 0)
+        hipLaunchKernelGGL((k_eval<EST, MODE | kSplit>), blocks, threads, lds, ctx.stream, A);
+    else
+        hipLaunchKernelGGL((k_eval<EST, MODE>), blocks, threads, lds, ctx.stream, A);
+    UPBP_HIP(hipGetLastError());
+}
+
+// An evaluation's launches, with its split set up. A plan gives the tiles with a common origin their parts;
+// the others are split uniformly.
+template <int EST, int MODE>
+void launch_kernel(Ctx& ctx, EvalArgs A, const Split& s, const TilePlan& p, int tuned) {
+    const int64_t tiles = (A.count + kWave - 1) / kWave;
+    if (s.planned) {
+        EvalArgs B = A;
+        B.tasks = p.tasks;
+        B.plan = p.words;
+        const PlanArgs P = {tiles, (uint32_t)s.waves, s.log_most, s.log_parts, in_two(MODE), p.cost, p.info, p.tasks, p.words};
+        const int steps = (int)std::min<int64_t>(std::max<int64_t>(tiles / 128, 16), kCostSteps);
+        hipLaunchKernelGGL(k_tile_cost<EST>, dim3(grid_for(tiles, 4)), dim3(256), 0, ctx.stream, B, steps, p.cost);
+        hipLaunchKernelGGL(k_plan_parts, dim3(grid_for(tiles)), dim3(256), 0, ctx.stream, P);
+        hipLaunchKernelGGL(k_plan_tasks, dim3(grid_for(tiles)), dim3(256), 0, ctx.stream, P);
+        UPBP_HIP(hipGetLastError());
+        launch_waves<EST, MODE>(ctx, B, tiles + s.waves, tuned);
+        A.row0 = (uint32_t)s.waves;
+    } else {
+        launch_waves<EST, MODE>(ctx, A, tiles << s.log_parts, tuned);
     }
-    launch_kernel<EST, MODE>(ctx, A, blocks, threads, lds);
+    if constexpr (in_two(MODE))
+        if (A.count > 1)  // one ray has one origin
+            launch_waves<EST, MODE | kSparse>(ctx, A, tiles << s.log_parts, tuned);
+}
+
+template <int EST, int MODE>
+void launch_reduced(Ctx& ctx, const EvalArgs& A, const Split& s, const TilePlan& p, int tuned) {
+    if constexpr (EST == kEstBeams) {
+        if (A.red.max != 0) return launch_kernel<EST, MODE | kReduced>(ctx, A, s, p, tuned);
+    }
+    launch_kernel<EST, MODE>(ctx, A, s, p, tuned);
 }
 
 template <int EST>
-void launch_mode(Ctx& ctx, Mode mode, const EvalArgs& A, unsigned blocks, unsigned threads) {
+void launch_mode(Ctx& ctx, Mode mode, EvalArgs& A, const QueryView& q, int64_t items, int tuned) {
+    const Split& s = q.split[EST];
+    const TilePlan& p = q.plan[EST];
+    A.log_parts = s.log_parts;
+    A.shift = part_shift(items);
+    A.rows = p.rows;
     switch (mode) {
-        case Mode::Forward: return launch_reduced<EST, (int)Mode::Forward>(ctx, A, blocks, threads);
-        case Mode::Signature: return launch_reduced<EST, (int)Mode::Signature>(ctx, A, blocks, threads);
-        case Mode::Adjoint:
-            // LDS gradient slabs for the media actually present: fewer bytes, more resident waves
-            return launch_reduced<EST, (int)Mode::Adjoint>(
-                ctx, A, blocks, threads, (size_t)(threads / kWave) * A.lds_media_n * 6 * kWave * sizeof(float));
-        case Mode::Upbp: return launch_reduced<EST, (int)Mode::Upbp>(ctx, A, blocks, threads);
+        case Mode::Forward: return launch_reduced<EST, (int)Mode::Forward>(ctx, A, s, p, tuned);
+        case Mode::Signature: return launch_reduced<EST, (int)Mode::Signature>(ctx, A, s, p, tuned);
+        case Mode::Adjoint: return launch_reduced<EST, (int)Mode::Adjoint>(ctx, A, s, p, tuned);
+        case Mode::Upbp: return launch_reduced<EST, (int)Mode::Upbp>(ctx, A, s, p, tuned);
     }
 }
 
@@ -1987,47 +2294,42 @@ static void set_mis(EvalArgs& A, const MisDev* mis) {
     A.mis.p = mis->params;
 }
 
-uint32_t split_parts(int64_t count, int64_t items, int est, Mode mode) {
-    const int64_t tiles = (count + kWave - 1) / kWave;
-    uint32_t parts = 1;
-    if (items < kSplitFrom) return parts;
-    const int64_t waves = mode == Mode::Upbp || est == kEstPhotons ? kSplitWavesLight : kSplitWaves;
-    while (parts < kSplitMost && 2 * parts * tiles <= waves && 2 * parts * kSplitItems <= items) parts *= 2;
-    return parts;
-}
-
-uint32_t split_blocks(uint32_t parts) { return parts > 4 ? parts / 4 : 1; }
-
-// 2^shift items per block of a split, 64 or more (ItemPart::items): 32 to 64 blocks per part where there
-// are enough. Fewer balance worse (8: 22.0 against 20.0 ms on 200k rays without a common origin, 7.9
-// against 7.0 ms on traced beams), more make every part walk more of the tree.
-static uint32_t part_shift(int64_t items, uint32_t parts) {
-    uint32_t shift = 6;
-    while (parts > 1 && ((int64_t)parts * 32 << (shift + 1)) <= items) ++shift;
-    return shift;
+Split split_of(int64_t count, int64_t items, int est, Mode mode) {
+    Split s;
+    if (items < kSplitFrom) return s;
+    s.tiles = (count + kWave - 1) / kWave;
+    const bool light = mode == Mode::Upbp || est == kEstPhotons;
+    s.waves = light ? kSplitWavesLight : kSplitWaves;
+    const auto fits = [&](uint32_t lg) { return (kSplitItems << lg) <= items; };
+    while ((2u << s.log_parts) <= kSplitMost && (s.tiles << (s.log_parts + 1)) <= s.waves && fits(s.log_parts + 1))
+        ++s.log_parts;
+    s.planned = !light && s.tiles >= kPlanTiles && s.tiles <= s.waves;
+    if (s.planned) {
+        if (s.tiles <= kPlanFewTiles) s.waves = kPlanWaves;
+        while ((2u << s.log_most) <= kPlanMost && fits(s.log_most + 1)) ++s.log_most;
+    }
+    if (mode != Mode::Adjoint)
+        s.rows = (s.planned ? s.waves : 0) + (s.log_parts > 0 ? s.tiles << s.log_parts : 0);
+    return s;
 }
 
 template <class T, int N>
-static void sum_parts(Ctx& ctx, const QueryView& q, T* ph, T* bm) {
-    const uint32_t a = split_blocks(q.parts[kEstPhotons]), b = split_blocks(q.parts[kEstBeams]);
-    if (a == 1) ph = nullptr;
-    if (b == 1) bm = nullptr;
-    if (!ph && !bm) return;
-    hipLaunchKernelGGL((k_sum_parts<T, N>), dim3(grid_for(N * q.count)), dim3(256), 0, ctx.stream, q.count, q.perm, a,
-                       reinterpret_cast<const T*>(q.partial[kEstPhotons]), ph, b,
-                       reinterpret_cast<const T*>(q.partial[kEstBeams]), bm);
+static void sum_rows(Ctx& ctx, const QueryView& q, T* ph, T* bm) {
+    SumRows<T> a[2];
+    for (int e = 0; e < 2; ++e) {
+        const Split& s = q.split[e];
+        a[e] = {s.planned ? q.plan[e].info : nullptr, s.log_parts, reinterpret_cast<const T*>(q.plan[e].rows),
+                s.rows ? (e == kEstPhotons ? ph : bm) : nullptr};
+    }
+    if (!a[0].out && !a[1].out) return;
+    hipLaunchKernelGGL((k_sum_rows<T, N>), dim3((unsigned)((q.count + kWave - 1) / kWave), 2), dim3(256), 0, ctx.stream,
+                       q.count, q.perm, a[0], a[1]);
     UPBP_HIP(hipGetLastError());
 }
 
-void launch_sum_parts(Ctx& ctx, const QueryView& q, float* ph, float* bm) { sum_parts<float, 3>(ctx, q, ph, bm); }
-void launch_sum_parts_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* bm) {
-    sum_parts<uint32_t, 2>(ctx, q, ph, bm);
-}
-
-// Waves per block: the tuned number, or for split tiles (whose blocks hold parts of one tile) up to 4.
-static int block_waves(Mode mode, uint32_t parts, int tuned) {
-    if (parts > 1) return (int)std::min(parts, 4u);
-    return mode == Mode::Adjoint ? 4 : std::min(std::max(tuned, 1), 4);
+void launch_sum_rows(Ctx& ctx, const QueryView& q, float* ph, float* bm) { sum_rows<float, 3>(ctx, q, ph, bm); }
+void launch_sum_rows_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* bm) {
+    sum_rows<uint32_t, 2>(ctx, q, ph, bm);
 }
 
 void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& q, float* out, uint32_t* sig,
@@ -2042,12 +2344,8 @@ void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& 
     A.inc = ph.inc;
     A.orig = ph.orig;
     A.red = ph.sel;
-    A.parts = q.parts[kEstPhotons];
-    A.part_shift = part_shift(ph.n, A.parts);
     A.out = out;
     A.sig = sig;
-    A.partial = q.partial[kEstPhotons];
-    A.partial_sig = reinterpret_cast<uint32_t*>(q.partial[kEstPhotons]);
     if (adj) {
         A.grad_out = adj->grad_out;
         A.grad_media = adj->grad_media;
@@ -2055,9 +2353,7 @@ void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& 
     }
     const int want = ctx.tuning.photon_waves_per_block > 0 ? ctx.tuning.photon_waves_per_block
                                                            : ctx.tuning.waves_per_block;
-    const int wpb = block_waves(mode, A.parts, want);
-    const int64_t waves = (q.count + kWave - 1) / kWave * A.parts;
-    launch_mode<kEstPhotons>(ctx, mode, A, (unsigned)((waves + wpb - 1) / wpb), (unsigned)(wpb * kWave));
+    launch_mode<kEstPhotons>(ctx, mode, A, q, ph.n, want);
 }
 
 void launch_beams(Ctx& ctx, Mode mode, const BeamArgs& bm, const QueryView& q, float* out, uint32_t* sig,
@@ -2072,20 +2368,14 @@ void launch_beams(Ctx& ctx, Mode mode, const BeamArgs& bm, const QueryView& q, f
     A.orig = bm.piece_beam;
     A.end_bits = bm.end_bits;
     A.red = bm.red;
-    A.parts = q.parts[kEstBeams];
-    A.part_shift = part_shift(bm.pieces_n, A.parts);
     A.out = out;
     A.sig = sig;
-    A.partial = q.partial[kEstBeams];
-    A.partial_sig = reinterpret_cast<uint32_t*>(q.partial[kEstBeams]);
     if (adj) {
         A.grad_out = adj->grad_out;
         A.grad_media = adj->grad_media;
         A.grad_items = adj->grad_items;
     }
-    const int wpb = block_waves(mode, A.parts, ctx.tuning.waves_per_block);
-    const int64_t waves = (q.count + kWave - 1) / kWave * A.parts;
-    launch_mode<kEstBeams>(ctx, mode, A, (unsigned)((waves + wpb - 1) / wpb), (unsigned)(wpb * kWave));
+    launch_mode<kEstBeams>(ctx, mode, A, q, bm.pieces_n, ctx.tuning.waves_per_block);
 }
 
 void launch_rebase_nodes(Ctx& ctx, NodeDev* nodes, int64_t n, uint32_t node_off, uint32_t item_off) {
@@ -2110,8 +2400,6 @@ void prepare_batched(Ctx& ctx, int waves_per_block) {
 void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, uint32_t* counters,
                     const MergedDev& merged, int which, int grid_blocks, int waves_per_block) {
     EvalArgs A = {};
-    A.parts = 1;
-    A.part_shift = 6;
     A.media = ctx.media.as<MediumDev>();
     A.n_media = ctx.n_media;
     A.stats = ctx.stats.as<unsigned long long>();

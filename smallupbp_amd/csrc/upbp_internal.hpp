@@ -109,6 +109,14 @@ enum StatSlot : int {
 constexpr int kStatRows = 64;
 constexpr int kStatWords = kStatRows * kStatSlots;
 
+// What the kernels of a tile plan count (traverse.hip), cleared with the counters.
+struct PlanWords {
+    unsigned long long total[64][2];  // cost and number of the tiles with an estimate, spread over rows
+    uint32_t n_tasks, n_rows;
+    uint32_t hist[64], cursor[64];
+};
+constexpr int kStatAll = kStatWords + 2 * (int)(sizeof(PlanWords) / 8);  // with both estimators' plan words
+
 inline void sum_stats(const uint64_t* rows, uint64_t* st) {
     for (int k = 0; k < kStatSlots; ++k) st[k] = 0;
     for (int r = 0; r < kStatRows; ++r)
@@ -146,7 +154,7 @@ struct Ctx {
     // bumped by every upbp_set_media: a batched plan whose captured graph froze an older table
     // re-validates its instances and captures again
     uint64_t media_gen = 0;
-    DevBuf stats;       // kStatWords x uint64
+    DevBuf stats;       // kStatAll x uint64
     DevBuf sort_tmp;    // hipcub temporary storage
     TmpPool tmp;        // build temporaries
     DevBuf qkeys, qkeys2, qperm, qperm2;
@@ -155,7 +163,7 @@ struct Ctx {
     DevBuf photon_recs;  // 64-byte MIS record per light vertex of the current UPBP call
     DevBuf vm_rec;       // merge records (4 float4 per grid slot) of the current PP3D / SURF call
     DevBuf lt_slots[8];  // light tracing: per-path vertex, position and beam slots, counts, offsets, lights
-    DevBuf partial[2];  // sums of a split evaluation's parts, per estimator
+    DevBuf plan[2];  // a split evaluation's plan and rows, per estimator
     DevBuf staging[8];  // host-input staging copies
     hipEvent_t ev[6] = {};
     // second stream: the photon and beam kernels of one eval call run concurrently
@@ -212,17 +220,49 @@ struct Beams {
     int32_t grid_resolution = 0;
 };
 
+// How the items of a batch's tiles are split over waves (split_of): uniformly over 2^log_parts, or by a
+// plan that gives a tile up to 2^log_most parts.
+struct Split {
+    int64_t tiles = 0, waves = 0;
+    uint32_t log_parts = 0, log_most = 0;
+    bool planned = false;
+    int64_t rows = 0;  // sums of parts kept for k_sum_rows, 64 x 3 floats each
+};
+
+// Device memory of a split: the rows, and of a plan the tiles' costs, their part counts and first rows,
+// and the tasks.
+struct TilePlan {
+    uint32_t* cost = nullptr;
+    uint2 *info = nullptr, *tasks = nullptr;
+    PlanWords* words = nullptr;
+    float* rows = nullptr;
+    static size_t bytes(const Split& s) {
+        return (size_t)s.rows * 768 + (s.planned ? (size_t)s.tiles * 20 + (size_t)s.waves * 8 : 0);
+    }
+    // lays the plan of s out in bytes(s) of memory at p (256-byte aligned)
+    static TilePlan at(const Split& s, char* p) {
+        TilePlan t;
+        t.rows = reinterpret_cast<float*>(p);
+        if (s.planned) {
+            t.tasks = reinterpret_cast<uint2*>(p + (size_t)s.rows * 768);
+            t.info = t.tasks + (s.tiles + s.waves);
+            t.cost = reinterpret_cast<uint32_t*>(t.info + s.tiles);
+        }
+        return t;
+    }
+};
+
 // Device memory one evaluation works in besides its inputs and outputs: the kernels' counters,
 // the Morton keys and permutations of the query sort and the sort's temporary storage. The
 // context's own growable buffers by default; the allocation-free entry point passes a fixed
 // region instead.
 struct Workspace {
-    unsigned long long* stats = nullptr;  // kStatWords counters
+    unsigned long long* stats = nullptr;  // kStatAll words: kStatWords counters, two PlanWords
     uint32_t *keys = nullptr, *keys2 = nullptr, *perm = nullptr, *perm2 = nullptr;  // [max_sorted] each
     int64_t max_sorted = 0;
     void* sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
-    float* partial[2] = {nullptr, nullptr};  // per estimator, the sums of a split evaluation's parts
+    TilePlan plan[2];  // per estimator
 };
 
 // Device-resident view of a query batch.
@@ -235,10 +275,9 @@ struct QueryView {
     uint32_t beam_type = UPBP_LONG_BEAM;
     uint32_t lite = 0;
     const uint32_t* perm = nullptr;  // lane slot -> query index, or null (identity)
-    // per estimator, a tile's items split over this many waves (split_parts); with several blocks per
-    // tile each block's sums go to partial ([split_blocks][count][3] floats) for k_sum_parts
-    uint32_t parts[2] = {1, 1};
-    float* partial[2] = {nullptr, nullptr};
+    // per estimator
+    Split split[2];
+    TilePlan plan[2];
 };
 
 // A tile of 64 queries is one wave, and the GPU holds 8192 of them: a batch of fewer tiles leaves it
@@ -260,6 +299,20 @@ struct QueryView {
 constexpr int64_t kSplitWaves = 16384, kSplitWavesLight = 4096;
 constexpr int64_t kSplitItems = 256, kSplitFrom = 16384;
 constexpr uint32_t kSplitMost = 64;
+
+// From kPlanTiles tiles on, up to where nothing is split, a beam launch plans: a tile gets as many of
+// kPlanWaves waves, at most kPlanMost, as its share of the estimated cost, and the dearest parts start
+// first. Estimating takes 30 to 140 us, which fewer tiles do not earn back (256x256 rays x 100k photons
+// 220 -> 270 us with 1024 tiles; photons and the UPBP kernels gain nothing and don't plan). Above
+// kPlanFewTiles tiles kSplitWaves, so that average tiles stay whole. Measured uniform / planned with
+// 16384 / 24576 / 32768 waves:
+//   640x360 rays x 40k traced beams          7.99 / 3.92 / 3.83 / 3.88 ms
+//   512x512 rays, forward and adjoint        9.00 / 9.14 / 8.60 / 8.92 ms
+//   60k rays x 300k beams                    4.37 / 4.13 / 3.49 / 3.41 ms
+//   400x241 rays x 200k photons + 40k beams  1.10 / 1.06 / 0.96 / 1.00 ms
+//   1M rays x 2M beams                       45.8 / 38.8 / 41.6 / 41.7 ms
+constexpr uint32_t kPlanMost = 256;
+constexpr int64_t kPlanTiles = 512, kPlanFewTiles = 8192, kPlanWaves = 24576;
 
 // ---- lbvh.hip -------------------------------------------------------------
 // Builds an LBVH over n item boxes (lo/hi as float4 .xyz). On return
@@ -390,11 +443,10 @@ void launch_beam_records(Ctx& ctx, MisDev& mis, int64_t n_beams);
 void launch_photon_records(Ctx& ctx, MisDev& mis);
 // How many waves share a tile's items in an evaluation of count queries against items items (a power
 // of two), and how many blocks they form.
-uint32_t split_parts(int64_t count, int64_t items, int estimator, Mode mode);
-uint32_t split_blocks(uint32_t parts);
+Split split_of(int64_t count, int64_t items, int estimator, Mode mode);
 // Adds up a split evaluation's parts into the outputs (null: not evaluated), in query order.
-void launch_sum_parts(Ctx& ctx, const QueryView& q, float* ph, float* bm);
-void launch_sum_parts_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* bm);
+void launch_sum_rows(Ctx& ctx, const QueryView& q, float* ph, float* bm);
+void launch_sum_rows_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* bm);
 void launch_clear_u64(Ctx& ctx, uint64_t* p, int64_t n);
 void launch_clear_f32(Ctx& ctx, float* p, int64_t n);
 // gs += sign_s * (direct + d/d sigma_t), ga += sign_a * d/d sigma_t per medium and channel, summed
