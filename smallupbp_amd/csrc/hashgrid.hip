@@ -129,13 +129,17 @@ __global__ void k_grid_keys(const float* __restrict__ pos, const uint32_t* __res
     vals[i] = (uint32_t)i;
 }
 
-// Slots in bucket order and the end of each non-empty bucket (run boundaries).
+// Slots in bucket order, the slot of each vertex (kNoSlot outside the grid) and the end of each
+// non-empty bucket (run boundaries).
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 __global__ void k_grid_slots(const float* __restrict__ pos, const uint32_t* __restrict__ keys,
-                             const uint32_t* __restrict__ vals, int64_t n_sel, float4* __restrict__ slots,
-                             uint32_t* __restrict__ ends) {
+                             const uint32_t* __restrict__ vals, int64_t n, int64_t n_sel, float4* __restrict__ slots,
+                             uint32_t* __restrict__ slot_of, uint32_t* __restrict__ ends) {
     const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k >= n_sel) return;
+    if (k >= n) return;
     const uint32_t v = vals[k];
+    slot_of[v] = k < n_sel ? (uint32_t)k : kNoSlot;
+    if (k >= n_sel) return;
     slots[k] = make_float4(pos[3 * (int64_t)v], pos[3 * (int64_t)v + 1], pos[3 * (int64_t)v + 2], __uint_as_float(v));
     const uint32_t key = keys[k];
     if (k + 1 == n_sel || keys[k + 1] != key) ends[key] = (uint32_t)(k + 1);
@@ -208,13 +212,18 @@ constexpr int kRecWords = 4;
 constexpr uint32_t kRecConnectable = 1u;  // mConnectable
 constexpr uint32_t kRecBadIndex = 2u;     // the slot's vertex index is past the light vertices
 
-__global__ void k_vm_records(VmArgs A, uint32_t type, float4* __restrict__ rec) {
-    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k >= A.n_sel) return;
+// A thread per light vertex writes the record of the vertex's slot: a vertex is 112 bytes of which
+// neighbouring threads read neighbouring ones, and a record one 64-byte line. A thread per slot, which
+// gathered three or four lines per vertex, took 361 us on the vertices of 1M paths; this takes 253.
+__global__ void k_vm_records(VmArgs A, uint32_t type, const uint32_t* __restrict__ slot_of, int64_t n_src,
+                             float4* __restrict__ rec) {
+    const int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (v >= n_src) return;
+    const uint32_t k = slot_of[v];
+    if (k == kNoSlot) return;
     const MisGlobals& G = A.mis;
-    const uint32_t v = __float_as_uint(A.slots[k].w);
-    float4* r = rec + kRecWords * k;
-    if ((int64_t)v >= G.lv_count) {
+    float4* r = rec + kRecWords * (int64_t)k;
+    if (v >= G.lv_count) {
         r[0] = make_float4(0.f, 0.f, 0.f, 0.f);
         r[1] = make_float4(0.f, 0.f, 0.f, 0.f);
         r[2] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -224,7 +233,7 @@ __global__ void k_vm_records(VmArgs A, uint32_t type, float4* __restrict__ rec) 
     const upbp_light_vertex* __restrict__ lv = G.lv + v;
     float k0 = 0.f, k1 = 0.f;
     if (!(A.flags & UPBP_VM_NO_MIS) &&
-        !light_split(G, (int64_t)v, lv->path_idx, (int)lv->path_length, G.p.techniques, k0, k1))
+        !light_split(G, v, lv->path_idx, (int)lv->path_length, G.p.techniques, k0, k1))
         k1 = __builtin_nanf("");
     r[0] = make_float4(lv->dir_fix[0], lv->dir_fix[1], lv->dir_fix[2], __uint_as_float(lv->path_length));
     r[1] = make_float4(lv->throughput[0], lv->throughput[1], lv->throughput[2], lv->continuation_prob);
@@ -706,8 +715,10 @@ void hash_grid_build(Ctx& ctx, const float* pos, const uint32_t* flags, int64_t 
     DevBuf runs;
     runs.ensure((size_t)cells * 4);
     launch_fill_u32(ctx, runs.as<uint32_t>(), 0u, cells);
-    hipLaunchKernelGGL(k_grid_slots, dim3(blocks_for(out.n)), dim3(kBlock), 0, ctx.stream, pos, keys2.as<uint32_t>(),
-                       vals2.as<uint32_t>(), out.n, out.slots.as<float4>(), runs.as<uint32_t>());
+    out.slot_of.ensure((size_t)n * 4);
+    hipLaunchKernelGGL(k_grid_slots, dim3(blocks_for(n)), dim3(kBlock), 0, ctx.stream, pos, keys2.as<uint32_t>(),
+                       vals2.as<uint32_t>(), n, out.n, out.slots.as<float4>(), out.slot_of.as<uint32_t>(),
+                       runs.as<uint32_t>());
     UPBP_HIP(hipGetLastError());
     inclusive_max_u32(ctx, runs.as<uint32_t>(), out.ends.as<uint32_t>(), cells);
     UPBP_HIP(hipStreamSynchronize(ctx.stream));
@@ -750,8 +761,8 @@ void vm_eval(Ctx& ctx, const HashGrid& grid, const Query* q, int64_t count, cons
     A.rec = nullptr;
     if (out && grid.n > 0) {
         ctx.vm_rec.ensure((size_t)grid.n * kRecWords * sizeof(float4));
-        hipLaunchKernelGGL(k_vm_records, dim3(blocks_for(grid.n)), dim3(kBlock), 0, ctx.stream, A, grid.type,
-                           ctx.vm_rec.as<float4>());
+        hipLaunchKernelGGL(k_vm_records, dim3(blocks_for(grid.n_src)), dim3(kBlock), 0, ctx.stream, A, grid.type,
+                           grid.slot_of.as<uint32_t>(), grid.n_src, ctx.vm_rec.as<float4>());
         UPBP_HIP(hipGetLastError());
         A.rec = ctx.vm_rec.as<float4>();
     }

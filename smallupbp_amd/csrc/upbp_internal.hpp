@@ -463,6 +463,7 @@ struct HashGrid {
     float radius = 0.f, r2 = 0.f, inv_cell = 0.f;
     float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
     DevBuf slots;  // float4 [n]: position, light-vertex index (bits); bucket order
+    DevBuf slot_of;  // uint32 [n_src]: the slot of each light vertex, all ones outside the grid
     DevBuf ends;   // uint32 [cells]: one past each bucket's last slot
 };
 // flags[i * stride] holds the UPBP_LV_* word of light vertex i (device pointers).
