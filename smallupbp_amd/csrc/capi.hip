@@ -29,7 +29,9 @@ struct upbp_batch_plan {
     int64_t total_tiles = 0;
     std::vector<InstanceDev> host;
     DevBuf table;
-    DevBuf counters;  // [2] queue counters (photons, beams)
+    DevBuf counters;  // queue counters (photons, beams) and, from byte 64 on, both estimators' PlanWords
+    BatchSplit split;
+    DevBuf split_mem[2];
     // copies of every instance's structures, merged (see MergedDev)
     DevBuf m_ph_nodes, m_ph_pos_r2, m_ph_power, m_ph_inc, m_bm_nodes, m_bm_pieces, m_bm_flux;
     MergedDev merged = {};
@@ -1251,6 +1253,8 @@ static void merge_structures(Ctx& ctx, upbp_batch_plan* plan, const upbp_instanc
             UPBP_HIP(hipMemcpyAsync(plan->m_ph_inc.as<float4>() + pi, b->inc.p, b->n * 16, dd, ctx.stream));
             launch_rebase_nodes(ctx, dst, b->bvh.n_nodes, (uint32_t)pn, (uint32_t)pi);
             d.ph_root = (uint32_t)pn;
+            d.ph_log_most = batched_log_most(b->n);
+            d.ph_group = (uint32_t)std::max<int64_t>(64, b->n / 128);
             pn += std::max<int64_t>(b->bvh.n_nodes, b->n);
             pi += b->n;
         }
@@ -1262,6 +1266,8 @@ static void merge_structures(Ctx& ctx, upbp_batch_plan* plan, const upbp_instanc
             UPBP_HIP(hipMemcpyAsync(plan->m_bm_flux.as<float4>() + bi, m->piece_flux.p, m->pieces * 16, dd, ctx.stream));
             launch_rebase_nodes(ctx, dst, m->bvh.n_nodes, (uint32_t)bn, (uint32_t)bi);
             d.bm_root = (uint32_t)bn;
+            d.bm_log_most = batched_log_most(m->pieces);
+            d.bm_group = (uint32_t)std::max<int64_t>(64, m->pieces / 128);
             bn += std::max<int64_t>(m->bvh.n_nodes, m->pieces);
             bi += m->pieces;
         }
@@ -1357,7 +1363,18 @@ upbp_status upbp_batch_plan_create(upbp_ctx* ctx, const upbp_instance* instances
         plan->table.ensure(count * sizeof(InstanceDev));
         UPBP_HIP(hipMemcpyAsync(plan->table.p, plan->host.data(), count * sizeof(InstanceDev), hipMemcpyHostToDevice,
                                 ctx->stream));
-        plan->counters.ensure(16);
+        plan->counters.ensure(64 + 2 * sizeof(PlanWords));
+        plan->split.planned = tiles >= kPlanBatchTiles && tiles <= kPlanBatchMost;
+        if (plan->split.planned)
+            for (int e = 0; e < 2; ++e) {
+                Split s;
+                s.tiles = tiles;
+                s.waves = s.rows = kPlanWaves;
+                s.planned = true;
+                plan->split_mem[e].ensure(TilePlan::bytes(s));
+                plan->split.plan[e] = TilePlan::at(s, plan->split_mem[e].as<char>());
+                plan->split.plan[e].words = reinterpret_cast<PlanWords*>(plan->counters.as<char>() + 64) + e;
+            }
         UPBP_HIP(hipStreamSynchronize(ctx->stream));
     });
     if (st != UPBP_OK) {
@@ -1384,13 +1401,16 @@ upbp_status upbp_batch_plan_destroy(upbp_batch_plan* plan) {
 // kernel frees as its queue drains.
 static void enqueue_batch(Ctx& ctx, upbp_batch_plan* plan, int blocks) {
     launch_clear_u64(ctx, ctx.stats.as<uint64_t>(), kStatWords);
-    launch_fill_u32(ctx, plan->counters.as<uint32_t>(), 0u, 2);
+    launch_fill_u32(ctx, plan->counters.as<uint32_t>(), 0u, (int64_t)(64 + 2 * sizeof(PlanWords)) / 4);
+    const InstanceDev* table = plan->table.as<InstanceDev>();
     hipStream_t main_stream = ctx.stream;
     UPBP_HIP(hipEventRecord(ctx.fork, main_stream));
     UPBP_HIP(hipStreamWaitEvent(ctx.side, ctx.fork, 0));
+    launch_batched_plan(ctx, table, plan->n, plan->total_tiles, plan->split, plan->merged, 1);
     ctx.stream = ctx.side;
     try {
-        launch_batched(ctx, plan->table.as<InstanceDev>(), plan->n, plan->total_tiles, plan->counters.as<uint32_t>(),
+        launch_batched_plan(ctx, table, plan->n, plan->total_tiles, plan->split, plan->merged, 0);
+        launch_batched(ctx, table, plan->n, plan->total_tiles, plan->counters.as<uint32_t>(), plan->split,
                        plan->merged, 0, blocks, ctx.tuning.waves_per_block);
         UPBP_HIP(hipEventRecord(ctx.join, ctx.side));
     } catch (...) {
@@ -1398,8 +1418,8 @@ static void enqueue_batch(Ctx& ctx, upbp_batch_plan* plan, int blocks) {
         throw;
     }
     ctx.stream = main_stream;
-    launch_batched(ctx, plan->table.as<InstanceDev>(), plan->n, plan->total_tiles, plan->counters.as<uint32_t>(),
-                   plan->merged, 1, blocks, ctx.tuning.waves_per_block);
+    launch_batched(ctx, table, plan->n, plan->total_tiles, plan->counters.as<uint32_t>(), plan->split, plan->merged, 1,
+                   blocks, ctx.tuning.waves_per_block);
     UPBP_HIP(hipStreamWaitEvent(main_stream, ctx.join, 0));
 }
 
@@ -1423,7 +1443,7 @@ upbp_status upbp_batch_run(upbp_ctx* ctx, upbp_batch_plan* plan, int use_graph, 
         // blocks_per_cu 0: each persistent kernel fills the GPU to its own occupancy limit
         const int per_cu = std::max(ctx->tuning.blocks_per_cu, 0);
         const int blocks = ctx->num_cus * per_cu;
-        if (per_cu == 0) prepare_batched(*ctx, ctx->tuning.waves_per_block);
+        if (per_cu == 0) prepare_batched(*ctx, ctx->tuning.waves_per_block, plan->split.planned);
         if (stats) UPBP_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
         if (use_graph) {
             UPBP_REQUIRE(ctx->stream != nullptr, UPBP_EINVAL, "graph capture needs a non-default stream");

@@ -1612,48 +1612,81 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
     flush_stats(E, ls);
 }
 
-// Persistent batched kernel: waves take (instance, tile) items from a device
-// counter until the queue drains; every wave exits when an item index passes
-// total_tiles. Structures come from the plan's merged arrays through the kernel
+// The instance of a batched plan that owns a tile (wave-uniform).
+__device__ __forceinline__ const InstanceDev& tile_instance(const InstanceDev* inst, int n_inst, int64_t tile) {
+    int lo_i = 0, hi_i = n_inst - 1;
+    while (lo_i < hi_i) {
+        const int mid = (lo_i + hi_i + 1) >> 1;
+        if (inst[mid].tile_begin <= tile) lo_i = mid; else hi_i = mid - 1;
+    }
+    return inst[lo_i];
+}
+
+// The arguments of an instance's tiles.
+template <int EST>
+__device__ __forceinline__ EvalArgs instance_args(const EvalArgs& A, const InstanceDev& I) {
+    EvalArgs B = A;
+    B.root = uni(EST == kEstPhotons ? I.ph_root : I.bm_root);
+    B.origin = uni_global(I.origin);
+    B.direction = uni_global(I.direction);
+    B.offsets = uni_global(I.offsets);
+    B.segments = uni_global(I.segments);
+    B.perm = I.perm ? uni_global(I.perm) : nullptr;
+    B.count = uni64(I.count);
+    B.short_query = (int32_t)uni((uint32_t)(I.beam_type == UPBP_SHORT_BEAM));
+    B.lite = (int32_t)uni(I.lite);
+    B.media_base = (int32_t)uni((uint32_t)I.media_base);
+    // an instance's media are the table entries from media_base on: run_tile bounds every
+    // instance-local medium id by this count (<= 0 rejects every segment)
+    B.n_media = A.n_media - B.media_base;
+    B.out = uni_global(EST == kEstPhotons ? I.out_photons : I.out_beams);
+    return B;
+}
+
+// Persistent batched kernel: waves take (instance, tile) items, or a plan's tasks, from a device
+// counter until the queue drains; every wave exits when an index passes
+// their number. Structures come from the plan's merged arrays through the kernel
 // argument A (wave-uniform scalar loads, as in k_eval); only the instance's root
 // node, query pointers and flags come from the instance table. Six waves per SIMD
-// (at most 80 VGPRs) measured faster than the unconstrained allocation.
-template <int EST>
-__global__ __launch_bounds__(256, 6) void k_eval_batched(EvalArgs A, const InstanceDev* __restrict__ inst,
+// (at most 80 VGPRs) measured faster than the unconstrained allocation, and no more: the beam kernel's
+// blocks take the registers that the photon kernel's leave and hold them to the end, and with blocks of
+// 72 registers before blocks of 80 a quarter of them never found room.
+template <int EST, bool PLAN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_eval_batched(EvalArgs A, const InstanceDev* __restrict__ inst,
                                                             int n_inst, int64_t total_tiles, uint32_t* queue) {
+    constexpr int kMode = (int)Mode::Forward | (PLAN ? kSplit : 0);
     const int lane = threadIdx.x & (kWave - 1);
     unsigned long long ls[kStatSlots] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int64_t n_items = PLAN ? (int64_t)as_global(A.plan)->n_tasks : total_tiles;
     while (true) {
         uint32_t item = 0;
         if (lane == 0) item = atomicAdd(queue, 1u);
         item = uni((uint32_t)__shfl(item, 0, kWave));
-        if ((int64_t)item >= total_tiles) break;
-        // binary search of the instance owning this tile (uniform)
-        int lo_i = 0, hi_i = n_inst - 1;
-        while (lo_i < hi_i) {
-            const int mid = (lo_i + hi_i + 1) >> 1;
-            if (inst[mid].tile_begin <= (int64_t)item) lo_i = mid; else hi_i = mid - 1;
+        if ((int64_t)item >= n_items) break;
+        const TileTask t = PLAN ? tile_task(as_global(A.tasks), 0, 0, A.shift, item) : TileTask{item, 0u, 0u, {0u, 0u, 6u}};
+        const InstanceDev& I = tile_instance(inst, n_inst, t.tile);
+        if (!PLAN) {
+            const bool has = EST == kEstPhotons ? I.has_photons : I.has_beams;
+            if (!uni((uint32_t)has)) continue;
         }
-        const InstanceDev& I = inst[lo_i];
-        const bool has = EST == kEstPhotons ? I.has_photons : I.has_beams;
-        if (!uni((uint32_t)has)) continue;
-        EvalArgs B = A;
-        B.root = uni(EST == kEstPhotons ? I.ph_root : I.bm_root);
-        B.origin = uni_global(I.origin);
-        B.direction = uni_global(I.direction);
-        B.offsets = uni_global(I.offsets);
-        B.segments = uni_global(I.segments);
-        B.perm = I.perm ? uni_global(I.perm) : nullptr;
-        B.count = uni64(I.count);
-        B.short_query = (int32_t)uni((uint32_t)(I.beam_type == UPBP_SHORT_BEAM));
-        B.lite = (int32_t)uni(I.lite);
-        B.media_base = (int32_t)uni((uint32_t)I.media_base);
-        // an instance's media are the table entries from media_base on: run_tile bounds every
-        // instance-local medium id by this count (<= 0 rejects every segment)
-        B.n_media = A.n_media - B.media_base;
-        B.out = uni_global(EST == kEstPhotons ? I.out_photons : I.out_beams);
+        const EvalArgs B = instance_args<EST>(A, I);
         const int64_t tile_begin = uni64(I.tile_begin);
-        run_tile<EST, (int)Mode::Forward, false>(B, ((int64_t)item - tile_begin) * kWave, ItemPart{0u, 0u, 6u}, ls, nullptr);
+        run_tile<EST, kMode, false>(B, ((int64_t)t.tile - tile_begin) * kWave, t.part, ls, nullptr);
+        if (PLAN) {
+            const TileTask u = tile_task(as_global(A.tasks), 0, 0, A.shift, item);
+            const int64_t slot = ((int64_t)u.tile - tile_begin) * kWave + lane;
+            if (slot < B.count) {
+                float* out;
+                int64_t step = 1;
+                if (u.log_parts == 0) {
+                    out = as_global(B.out) + 3 * (B.perm ? (int64_t)as_global(B.perm)[slot] : slot);
+                } else {
+                    out = as_global(A.rows) + (size_t)u.row * 3 * kWave + lane;
+                    step = kWave;
+                }
+                for (int c = 0; c < 3; ++c) out[c * step] = g_part[threadIdx.x / kWave][c][lane];
+            }
+        }
     }
     flush_stats(A, ls);
 }
@@ -1699,6 +1732,26 @@ __global__ __launch_bounds__(256) void k_sum_rows(int64_t n, const uint32_t* __r
             ((part[0][w][lane] + part[1][w][lane]) + part[2][w][lane]) + part[3][w][lane];
 }
 
+// The same for a batched plan's tiles, whose outputs are their instances': a wave per tile, as most tiles
+// have nothing to add.
+__global__ __launch_bounds__(256) void k_sum_rows_batched(const InstanceDev* __restrict__ inst, int n_inst, int64_t tiles,
+                                                          bool beams, const uint2* __restrict__ infos,
+                                                          const float* __restrict__ rows) {
+    const uint32_t tile = uni(blockIdx.x * 4u + threadIdx.x / kWave);
+    if (tile >= tiles) return;
+    const uint2 info = infos[tile];
+    if (info.x == 0) return;
+    const InstanceDev& I = tile_instance(inst, n_inst, tile);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t slot = ((int64_t)tile - I.tile_begin) * kWave + lane;
+    if (slot >= I.count) return;
+    float v[3] = {};
+    for (uint32_t k = 0; k < (1u << info.x); ++k)
+        for (int c = 0; c < 3; ++c) v[c] += rows[((size_t)(info.y + k) * 3 + c) * kWave + lane];
+    float* out = (beams ? I.out_beams : I.out_photons) + 3 * (I.perm ? (int64_t)I.perm[slot] : slot);
+    for (int c = 0; c < 3; ++c) out[c] = v[c];
+}
+
 // ---- tile plans ----------------------------------------------------------------
 // What a tile costs is estimated before a split launch, so that expensive tiles are split into more parts
 // than cheap ones and start first. Parts of equal number left a launch waiting for a few waves: of
@@ -1708,19 +1761,27 @@ __global__ __launch_bounds__(256) void k_sum_rows(int64_t n, const uint32_t* __r
 // around the tile's rays within the segments that scatter, 64 nodes at a time (a lane tests a node, where
 // the gather tests one node with all rays), weighed as the gather's instruction counts are. Nothing but
 // the order and the number of the parts depends on it.
+constexpr uint32_t kNoTask = 64;
+struct PlanArgs {
+    int64_t tiles;
+    uint32_t waves, log_most, log_other;  // log_other: of tiles without an estimate
+    bool other_apart;                     // those are another launch's, with their rows after the plan's
+    uint32_t* cost;
+    uint2* info;  // {log2 of the parts, first row}; first the most parts, then the parts and the bucket
+    uint2* tasks;
+    PlanWords* words;
+};
+
 constexpr int kCostQueue = 1024;            // nodes that wait; what does not fit counts without being opened
 constexpr int kCostSteps = 64;              // as does what is left after so many steps, or a 128th of the tiles
 constexpr uint32_t kCostOther = 0xFFFFFFFFu;  // a wave without a common origin
+constexpr uint32_t kCostNone = 0;             // a tile with nothing to gather
 
 template <int EST>
-__global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, int steps, uint32_t* __restrict__ cost) {
-    __shared__ uint32_t queue[4][kCostQueue];
+__device__ __forceinline__ float tile_cost(const EvalArgs& A, int64_t slot, int steps, uint32_t group, uint32_t* nodes,
+                                           bool& one) {
     constexpr float kNode = 46.f, kLeaf = 73.f, kItem = EST == kEstPhotons ? 8.f : 20.f, kTile = 500.f;
     const int lane = threadIdx.x & (kWave - 1);
-    const uint32_t tile = uni(blockIdx.x * 4u + threadIdx.x / kWave);
-    const int64_t slot = (int64_t)tile * kWave + lane;
-    if ((int64_t)tile * kWave >= A.count) return;
-    uint32_t* const nodes = queue[threadIdx.x / kWave];
     float ox = 0.f, oy = 0.f, oz = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
     float t0 = __builtin_inff(), t1 = -__builtin_inff();
     if (slot < A.count) {
@@ -1733,7 +1794,7 @@ __global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, int steps, uint32
                 const upbp_volume_segment* sg = A.segments + k;
                 const int32_t m = sg->medium_id;
                 if (m < 0 || m >= A.n_media) break;
-                if (A.media[m].has_scattering) {
+                if (A.media[A.media_base + m].has_scattering) {
                     t0 = fminf(t0, sg->dist_min);
                     t1 = fmaxf(t1, sg->dist_max);
                 }
@@ -1741,7 +1802,7 @@ __global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, int steps, uint32
     }
     const uint64_t am = __ballot(t0 <= t1);
     float c = 0.f;
-    bool one = true;
+    one = true;
     if (am) {
         const int fl = __builtin_ctzll(am);
         const bool on = t0 <= t1;
@@ -1801,13 +1862,13 @@ __global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, int steps, uint32
                     if (!(near <= past)) continue;
                     const uint32_t items = kind[k] & kSpanMask;
                     float cost = kLeaf + (kLeaf / 64.f + kItem) * (float)items;
-                    if ((kind[k] & kInner) && items > A.frustum_leaf) {
+                    if ((kind[k] & kInner) && items > 64u) {
                         // of a larger subtree, the runs of 64 items that the cone crosses
                         const float part = __builtin_amdgcn_exp2f(
-                            __builtin_amdgcn_logf((float)A.frustum_leaf / (float)items) * (1.f / 3.f));
+                            __builtin_amdgcn_logf(64.f / (float)items) * (1.f / 3.f));
                         const float f = (e + part * rad) * __builtin_amdgcn_rcpf(e + rad);
                         cost *= f * f;
-                        go[k] = step < steps;
+                        go[k] = items > group && step < steps;
                     }
                     if (go[k])
                         skipped[k] = cost;
@@ -1830,30 +1891,59 @@ __global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, int steps, uint32
         }
     }
     for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);
-    if (lane == 0) {
-        const uint32_t v = (uint32_t)fminf(c + kTile, 4e9f);
-        cost[tile] = one ? v : kCostOther;
-        if (one) {
-            PlanWords* p = A.plan;
-            atomicAdd(&p->total[blockIdx.x % 64][0], (unsigned long long)v);
-            atomicAdd(&p->total[blockIdx.x % 64][1], 1ull);
-        }
+    return c + kTile;
+}
+
+// Writes a tile's cost and the most parts it may have (log2), and adds it to the total.
+__device__ __forceinline__ void put_cost(const PlanArgs& P, uint32_t tile, float c, bool one, uint32_t log_most) {
+    if ((threadIdx.x & (kWave - 1)) != 0) return;
+    const uint32_t v = (uint32_t)fminf(c, 4e9f);
+    P.cost[tile] = one ? v : kCostOther;
+    P.info[tile] = make_uint2(one ? log_most : P.log_other, 0u);
+    if (one) {
+        atomicAdd(&P.words->total[blockIdx.x % 64][0], (unsigned long long)v);
+        atomicAdd(&P.words->total[blockIdx.x % 64][1], 1ull);
     }
+}
+
+template <int EST>
+__global__ __launch_bounds__(256) void k_tile_cost(EvalArgs A, PlanArgs P, int steps) {
+    __shared__ uint32_t queue[4][kCostQueue];
+    const uint32_t tile = uni(blockIdx.x * 4u + threadIdx.x / kWave);
+    if (tile >= P.tiles) return;
+    bool one;
+    const float c = tile_cost<EST>(A, (int64_t)tile * kWave + (threadIdx.x & (kWave - 1)), steps,
+                                   A.frustum_leaf, queue[threadIdx.x / kWave], one);
+    put_cost(P, tile, c, one, P.log_most);
+}
+
+// The same over the tiles of a batched plan's instances, of which there are many: one estimate, from every
+// kBatchStride-th ray, for kBatchStride consecutive tiles of an instance.
+constexpr int kBatchStride = 16, kBatchSteps = 16;
+template <int EST>
+__global__ __launch_bounds__(256) void k_tile_cost_batched(EvalArgs A, PlanArgs P, const InstanceDev* __restrict__ inst, int n_inst) {
+    __shared__ uint32_t queue[4][kCostQueue];
+    const uint32_t tile = uni(blockIdx.x * 4u + threadIdx.x / kWave);
+    if (tile >= P.tiles) return;
+    const InstanceDev& I = tile_instance(inst, n_inst, tile);
+    if (!uni((uint32_t)(EST == kEstPhotons ? I.has_photons : I.has_beams))) {
+        if ((threadIdx.x & (kWave - 1)) == 0) P.cost[tile] = kCostNone;
+        return;
+    }
+    const int64_t local = (int64_t)tile - uni64(I.tile_begin);
+    if (local % kBatchStride != 0) return;
+    const EvalArgs B = instance_args<EST>(A, I);
+    bool one;
+    const float c = tile_cost<EST>(B, local * kWave + (threadIdx.x & (kWave - 1)) * kBatchStride, kBatchSteps,
+                                   uni(EST == kEstPhotons ? I.ph_group : I.bm_group), queue[threadIdx.x / kWave], one);
+    const int64_t tiles = (B.count + kWave - 1) / kWave;
+    for (int k = 0; k < kBatchStride && local + k < tiles; ++k)
+        put_cost(P, tile + k, c, one, uni(EST == kEstPhotons ? I.ph_log_most : I.bm_log_most));
 }
 
 // Parts per tile: the share of `waves` that its cost is of the whole, rounded down to a power of two, so
 // that all parts together are no more than `waves`. Then a counting sort of the parts by what one costs,
 // in quarter octaves, dearest first.
-constexpr uint32_t kNoTask = 64;
-struct PlanArgs {
-    int64_t tiles;
-    uint32_t waves, log_most, log_other;  // log_other: of tiles without an estimate
-    bool other_apart;                     // those are another launch's, with their rows after the plan's
-    const uint32_t* cost;
-    uint2* info;  // {log2 of the parts, first row}; k_plan_parts leaves the bucket in y
-    uint2* tasks;
-    PlanWords* words;
-};
 
 __global__ __launch_bounds__(256) void k_plan_parts(PlanArgs P) {
     __shared__ uint32_t hist[64];
@@ -1872,11 +1962,15 @@ __global__ __launch_bounds__(256) void k_plan_parts(PlanArgs P) {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i < P.tiles) {
         const uint32_t c = P.cost[i];
-        uint32_t lg = P.log_other, bucket = 0;
-        if (c != kCostOther) {
+        const uint32_t most = P.info[i].x;
+        uint32_t lg = most, bucket = 0;
+        if (c == kCostNone) {
+            lg = 0;
+            bucket = kNoTask;
+        } else if (c != kCostOther) {
             const float want = (float)c * share;
             lg = 0;
-            while (lg < P.log_most && want >= (float)(2u << lg)) ++lg;
+            while (lg < most && want >= (float)(2u << lg)) ++lg;
             const int q = (int)(__float_as_uint(want / (float)(1u << lg)) >> 21) - (int)(__float_as_uint(1.f) >> 21);
             bucket = (uint32_t)min(max(24 - q, 0), 63);
         }
@@ -2074,6 +2168,14 @@ void launch_waves(Ctx& ctx, const EvalArgs& A, int64_t waves, int tuned) {
     UPBP_HIP(hipGetLastError());
 }
 
+static int cost_steps(int64_t tiles) { return (int)std::min<int64_t>(std::max<int64_t>(tiles / 128, 16), kCostSteps); }
+
+static void launch_plan(Ctx& ctx, const PlanArgs& P) {
+    hipLaunchKernelGGL(k_plan_parts, dim3(grid_for(P.tiles)), dim3(256), 0, ctx.stream, P);
+    hipLaunchKernelGGL(k_plan_tasks, dim3(grid_for(P.tiles)), dim3(256), 0, ctx.stream, P);
+    UPBP_HIP(hipGetLastError());
+}
+
 // An evaluation's launches, with its split set up. A plan gives the tiles with a common origin their parts;
 // the others are split uniformly.
 template <int EST, int MODE>
@@ -2084,11 +2186,9 @@ void launch_kernel(Ctx& ctx, EvalArgs A, const Split& s, const TilePlan& p, int 
         B.tasks = p.tasks;
         B.plan = p.words;
         const PlanArgs P = {tiles, (uint32_t)s.waves, s.log_most, s.log_parts, in_two(MODE), p.cost, p.info, p.tasks, p.words};
-        const int steps = (int)std::min<int64_t>(std::max<int64_t>(tiles / 128, 16), kCostSteps);
-        hipLaunchKernelGGL(k_tile_cost<EST>, dim3(grid_for(tiles, 4)), dim3(256), 0, ctx.stream, B, steps, p.cost);
-        hipLaunchKernelGGL(k_plan_parts, dim3(grid_for(tiles)), dim3(256), 0, ctx.stream, P);
-        hipLaunchKernelGGL(k_plan_tasks, dim3(grid_for(tiles)), dim3(256), 0, ctx.stream, P);
-        UPBP_HIP(hipGetLastError());
+        const int steps = cost_steps(tiles);
+        hipLaunchKernelGGL(k_tile_cost<EST>, dim3(grid_for(tiles, 4)), dim3(256), 0, ctx.stream, B, P, steps);
+        launch_plan(ctx, P);
         launch_waves<EST, MODE>(ctx, B, tiles + s.waves, tuned);
         A.row0 = (uint32_t)s.waves;
     } else {
@@ -2420,21 +2520,29 @@ void launch_rebase_nodes(Ctx& ctx, NodeDev* nodes, int64_t n, uint32_t node_off,
     UPBP_HIP(hipGetLastError());
 }
 
-void prepare_batched(Ctx& ctx, int waves_per_block) {
+void prepare_batched(Ctx& ctx, int waves_per_block, bool planned) {
     const int wpb = std::min(std::max(waves_per_block, 1), 4);
-    if (ctx.batched_wpb == wpb) return;
-    int p = 0, b = 0;
-    UPBP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &p, reinterpret_cast<const void*>(&k_eval_batched<kEstPhotons>), wpb * kWave, 0));
-    UPBP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &b, reinterpret_cast<const void*>(&k_eval_batched<kEstBeams>), wpb * kWave, 0));
-    ctx.batched_per_cu[0] = std::max(p, 1);
-    ctx.batched_per_cu[1] = std::max(b, 1);
-    ctx.batched_wpb = wpb;
+    const int key = planned ? 4 + wpb : wpb;
+    if (ctx.batched_key == key) return;
+    const void* const kernels[2][2] = {{reinterpret_cast<const void*>(&k_eval_batched<kEstPhotons, false>),
+                                        reinterpret_cast<const void*>(&k_eval_batched<kEstBeams, false>)},
+                                       {reinterpret_cast<const void*>(&k_eval_batched<kEstPhotons, true>),
+                                        reinterpret_cast<const void*>(&k_eval_batched<kEstBeams, true>)}};
+    for (int e = 0; e < 2; ++e) {
+        int n = 0;
+        UPBP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernels[planned][e], wpb * kWave, 0));
+        ctx.batched_per_cu[e] = std::max(n, 1);
+    }
+    ctx.batched_key = key;
 }
 
-void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, uint32_t* counters,
-                    const MergedDev& merged, int which, int grid_blocks, int waves_per_block) {
+uint32_t batched_log_most(int64_t items) {
+    uint32_t lg = 0;
+    while (items >= kSplitFrom && (2u << lg) <= kPlanMost && (kSplitItems << (lg + 1)) <= items) ++lg;
+    return lg;
+}
+
+static EvalArgs batched_args(Ctx& ctx, const BatchSplit& split, const MergedDev& merged, int which) {
     EvalArgs A = {};
     A.media = ctx.media.as<MediumDev>();
     A.n_media = ctx.n_media;
@@ -2450,20 +2558,54 @@ void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total
         A.pieces = merged.bm_pieces;
         A.piece_flux = merged.bm_flux;
     }
-    const unsigned threads = (unsigned)(std::min(std::max(waves_per_block, 1), 4) * kWave);
-    uint32_t* queue = counters + which;
+    if (split.planned) {
+        const TilePlan& p = split.plan[which];
+        A.tasks = p.tasks;
+        A.plan = p.words;
+        A.rows = p.rows;
+        A.shift = part_shift(kSplitFrom);  // instances are small: 64 items per block from 8 parts on
+    }
+    return A;
+}
+
+template <int EST>
+static void plan_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t tiles, const BatchSplit& split,
+                         const MergedDev& merged) {
+    const TilePlan& p = split.plan[EST];
+    const PlanArgs P = {tiles, (uint32_t)kPlanWaves, 0, 0, false, p.cost, p.info, p.tasks, p.words};
+    hipLaunchKernelGGL(k_tile_cost_batched<EST>, dim3(grid_for(tiles, 4)), dim3(256), 0, ctx.stream,
+                       batched_args(ctx, split, merged, EST), P, inst, n_inst);
+    launch_plan(ctx, P);
+}
+
+void launch_batched_plan(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, const BatchSplit& split,
+                         const MergedDev& merged, int which) {
+    if (!split.planned) return;
+    if (which == kEstPhotons)
+        plan_batched<kEstPhotons>(ctx, inst, n_inst, total_tiles, split, merged);
+    else
+        plan_batched<kEstBeams>(ctx, inst, n_inst, total_tiles, split, merged);
+}
+
+void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, uint32_t* counters,
+                    const BatchSplit& split, const MergedDev& merged, int which, int grid_blocks, int waves_per_block) {
+    const EvalArgs A = batched_args(ctx, split, merged, which);
+    const int wpb = std::min(std::max(waves_per_block, 1), 4);
     if (grid_blocks <= 0) {
         // persistent grid: as many blocks as can be resident at once on every CU
-        UPBP_REQUIRE(ctx.batched_wpb == (int)(threads / kWave) && ctx.batched_per_cu[which] > 0, UPBP_EDEVICE,
+        UPBP_REQUIRE(ctx.batched_key == (split.planned ? 4 + wpb : wpb) && ctx.batched_per_cu[which] > 0, UPBP_EDEVICE,
                      "batched occupancy not prepared");
         grid_blocks = ctx.num_cus * ctx.batched_per_cu[which];
     }
-    if (which == kEstPhotons)
-        hipLaunchKernelGGL(k_eval_batched<kEstPhotons>, dim3(grid_blocks), dim3(threads), 0, ctx.stream, A, inst,
-                           n_inst, total_tiles, queue);
-    else
-        hipLaunchKernelGGL(k_eval_batched<kEstBeams>, dim3(grid_blocks), dim3(threads), 0, ctx.stream, A, inst, n_inst,
-                           total_tiles, queue);
+    const auto kernel = which == kEstPhotons
+                            ? (split.planned ? k_eval_batched<kEstPhotons, true> : k_eval_batched<kEstPhotons, false>)
+                            : (split.planned ? k_eval_batched<kEstBeams, true> : k_eval_batched<kEstBeams, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid_blocks), dim3((unsigned)(wpb * kWave)), 0, ctx.stream, A, inst, n_inst,
+                       total_tiles, counters + which);
+    UPBP_HIP(hipGetLastError());
+    if (!split.planned) return;
+    hipLaunchKernelGGL(k_sum_rows_batched, dim3(grid_for(total_tiles, 4)), dim3(256), 0, ctx.stream, inst, n_inst,
+                       total_tiles, which == kEstBeams, split.plan[which].info, split.plan[which].rows);
     UPBP_HIP(hipGetLastError());
 }
 

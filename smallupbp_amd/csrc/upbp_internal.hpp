@@ -170,8 +170,8 @@ struct Ctx {
     // (fork from `stream`, join back), so one kernel's tail overlaps the other's work
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
-    // resident blocks per CU of the two persistent batched kernels at batched_wpb waves per block
-    int batched_wpb = 0;
+    // resident blocks per CU of the two persistent batched kernels at batched_key waves per block
+    int batched_key = 0;
     int batched_per_cu[2] = {0, 0};
     int num_cus = 256;
     Tuning tuning;
@@ -313,6 +313,13 @@ constexpr uint32_t kSplitMost = 64;
 //   1M rays x 2M beams                       45.8 / 38.8 / 41.6 / 41.7 ms
 constexpr uint32_t kPlanMost = 256;
 constexpr int64_t kPlanTiles = 512, kPlanFewTiles = 8192, kPlanWaves = 24576;
+// Batched plans of this many tiles are planned too, both estimators, with kPlanWaves waves. Tiles of small
+// instances stay whole there; the order alone shortens the tail. Measured in queue order / planned:
+//   16 instances, 4.6M rays                  7.36 / 5.08 ms
+//   18 instances x 26k rays                  6.16 / 1.77 ms
+//   5 instances x 22k rays                   1.91 / 0.93 ms
+//   15 instances x 358k rays                 3.91 / 4.07 ms (16384 waves: 3.91)
+constexpr int64_t kPlanBatchTiles = 1024, kPlanBatchMost = 1 << 20;
 
 // ---- lbvh.hip -------------------------------------------------------------
 // Builds an LBVH over n item boxes (lo/hi as float4 .xyz). On return
@@ -499,6 +506,8 @@ struct InstanceDev {
     int32_t has_beams;
     uint32_t ph_root;  // root of this instance's photon tree in the plan's merged node array
     uint32_t bm_root;  // root of its beam tree in the merged beam node array
+    uint32_t ph_log_most, bm_log_most;  // log2 of the most parts its tiles may be split into
+    uint32_t ph_group, bm_group;        // subtrees of at most this many items are estimated as one
     int32_t pad;
 };
 
@@ -518,9 +527,18 @@ struct MergedDev {
 void launch_rebase_nodes(Ctx& ctx, NodeDev* nodes, int64_t n, uint32_t node_off, uint32_t item_off);
 
 // Queries (outside any graph capture) how many blocks of each persistent kernel fit on a CU.
-void prepare_batched(Ctx& ctx, int waves_per_block);
+void prepare_batched(Ctx& ctx, int waves_per_block, bool planned);
+// How a batched plan's tiles are split, with the memory of each estimator's tile plan. A tile of an
+// instance with fewer than kSplitFrom items stays whole (batched_log_most).
+struct BatchSplit {
+    bool planned = false;
+    TilePlan plan[2];
+};
+uint32_t batched_log_most(int64_t items);
+void launch_batched_plan(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, const BatchSplit& split,
+                         const MergedDev& merged, int which);
 void launch_batched(Ctx& ctx, const InstanceDev* inst, int n_inst, int64_t total_tiles, uint32_t* counters,
-                    const MergedDev& merged, int which, int grid_blocks, int waves_per_block);
+                    const BatchSplit& split, const MergedDev& merged, int which, int grid_blocks, int waves_per_block);
 void launch_fill_u32(Ctx& ctx, uint32_t* p, uint32_t v, int64_t n);
 
 // ---- lighttrace.hip: light sub-path tracing in media ---------------------------
