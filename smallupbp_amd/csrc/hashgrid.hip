@@ -457,7 +457,7 @@ constexpr int kHitRing = 128;  // a ballot adds at most 64 to fewer than 64 queu
 template <class Cam>
 struct VmLds {
     uint32_t slot[kWaves][kHitRing];
-    uint32_t owner[kWaves][kHitRing];
+    uint8_t owner[kWaves][kHitRing];
     float cam[kWaves][Cam::kWords][64];
     float acc[kWaves][3][64];
 };
@@ -484,16 +484,24 @@ __device__ __forceinline__ void vm_drain(const VmArgs& A, VmLds<Cam>& L, uint32_
 
 // HashGrid::Process (HashGrid.hxx:130-186), one lane per camera vertex: the eight buckets' ranges are
 // read at once, then each bucket is walked kStep slots at a time, so that its loads are in flight
-// together. 1M camera vertices: PP3D 1.28 -> 0.78 ms, SURF 12.05 -> 7.76 ms.
+// together. 1M camera vertices: PP3D 1.28 -> 0.78 ms, SURF 12.05 -> 7.76 ms. Bound by the lanes' gathers of
+// slots and records and by the weighing of the hits. The blocks, which are sorted by place, go to the 8 XCDs
+// in chunks of kXcdChunk, so that neighbours share an L2 (SURF 8.40 -> 8.13 ms for the call); the hits'
+// owners take a byte each, with which a fifth SURF block fits the LDS of a CU.
+constexpr uint32_t kXcdChunk = 8;
 template <class Query, bool SIG>
-__global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __restrict__ queries) {
+__global__ __launch_bounds__(kBlock, SIG ? 1 : 5) void k_vm_eval(VmArgs A, const Query* __restrict__ queries) {
     using Cam = typename CameraOf<Query>::type;
     static_assert(sizeof(Cam) == (Cam::kWords - kCamWords) * 4, "camera state words");
     constexpr int kStep = 4;
     __shared__ VmLds<Cam> L;  // unused with SIG
     const int w = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63u;
-    const int64_t slot = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const uint32_t first_block = blockIdx.x / (8u * kXcdChunk) * (8u * kXcdChunk);
+    uint32_t block = blockIdx.x;
+    if (first_block + 8u * kXcdChunk <= gridDim.x)
+        block = first_block + blockIdx.x % 8u * kXcdChunk + (blockIdx.x - first_block) / 8u;
+    const int64_t slot = block * (int64_t)blockDim.x + threadIdx.x;
     const bool valid = slot < A.count;
     uint32_t err = 0, processed = 0, sig_h = 0;
     uint64_t tested = 0;
@@ -589,7 +597,7 @@ __global__ __launch_bounds__(kBlock) void k_vm_eval(VmArgs A, const Query* __res
                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
                     const uint32_t at = (tail + rank) & (kHitRing - 1);
                     L.slot[w][at] = k + (uint32_t)i;
-                    L.owner[w][at] = lane;
+                    L.owner[w][at] = (uint8_t)lane;
                 }
                 tail += (uint32_t)__popcll(m);
                 if (tail - head >= 64u) {
