@@ -1148,7 +1148,7 @@ upbp_status upbp_adjoint(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* b
         // upstream gradients on the device
         const float* gph = do_ph ? stage_q(*ctx, 4, grad_out_photons, 3 * Q, memory) : nullptr;
         const float* gbm = do_bm ? stage_q(*ctx, 5, grad_out_beams, 3 * Q, memory) : nullptr;
-        DevBuf gmedia, items_ph, items_bm, gs_d, ga_d;
+        TmpBuf gmedia(ctx->tmp), items_ph(ctx->tmp), items_bm(ctx->tmp);
         gmedia.ensure((size_t)kGradRows * M * 6 * 4);
         launch_clear_f32(*ctx, gmedia.as<float>(), (int64_t)kGradRows * M * 6);
         float* dpp = grad_photon_power;
@@ -1166,7 +1166,7 @@ upbp_status upbp_adjoint(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* b
             }
         }
         // item gradients must have somewhere to go
-        DevBuf dummy_ph, dummy_bm;
+        TmpBuf dummy_ph(ctx->tmp), dummy_bm(ctx->tmp);
         if (do_ph && !dpp) {
             dummy_ph.ensure(bre->n_in * 12);
             dpp = dummy_ph.as<float>();

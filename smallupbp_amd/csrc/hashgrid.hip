@@ -669,7 +669,7 @@ void hash_grid_build(Ctx& ctx, const float* pos, const uint32_t* flags, int64_t 
     out.ends.ensure((size_t)cells * 4);
     launch_fill_u32(ctx, out.ends.as<uint32_t>(), 0u, cells);
     if (n == 0) return;
-    DevBuf part;
+    TmpBuf part(ctx.tmp);
     part.ensure(kBoundsBlocks * 8 * sizeof(float));
     hipLaunchKernelGGL(k_grid_bounds, dim3(kBoundsBlocks), dim3(kBlock), 0, ctx.stream, pos, flags, stride, n,
                        want_medium, part.as<float>());
@@ -709,7 +709,7 @@ void hash_grid_build(Ctx& ctx, const float* pos, const uint32_t* flags, int64_t 
     g.r2 = out.r2;
     g.inv_cell = out.inv_cell;
     g.cells = (uint32_t)cells;
-    DevBuf keys, keys2, vals, vals2;
+    TmpBuf keys(ctx.tmp), keys2(ctx.tmp), vals(ctx.tmp), vals2(ctx.tmp);
     keys.ensure(n * 4);
     keys2.ensure(n * 4);
     vals.ensure(n * 4);
@@ -720,7 +720,7 @@ void hash_grid_build(Ctx& ctx, const float* pos, const uint32_t* flags, int64_t 
     sort_pairs_u32(ctx, keys.as<uint32_t>(), keys2.as<uint32_t>(), vals.as<uint32_t>(), vals2.as<uint32_t>(), n,
                    bits_for((uint64_t)cells));
     out.slots.ensure((size_t)out.n * sizeof(float4));
-    DevBuf runs;
+    TmpBuf runs(ctx.tmp);
     runs.ensure((size_t)cells * 4);
     launch_fill_u32(ctx, runs.as<uint32_t>(), 0u, cells);
     out.slot_of.ensure((size_t)n * 4);

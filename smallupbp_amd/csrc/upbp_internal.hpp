@@ -284,7 +284,7 @@ struct QueryView {
 // partly idle, and one of a few times more waits for the waves that meet most of the items. So a
 // tile's items are split over as many waves as bring the launch to kSplitWaves, at most kSplitMost, each
 // for at least kSplitItems items. Structures of fewer than kSplitFrom items stay whole: little is left to
-// split there, and their sums stay the same bits as a batched plan's, which splits nothing. Every part
+// split there, and their sums stay the same bits as a batched plan's, which leaves them whole too. Every part
 // walks the top of the tree again, so photons, which are tested in less time than beams, and the UPBP
 // kernels, of which the GPU holds half as many waves, stop at kSplitWavesLight. Measured unsplit / at
 // 4096 / 8192 / 16384 / 32768 waves for every estimator:
@@ -339,15 +339,21 @@ void sort_pairs_u32_in(Ctx& ctx, void* tmp, size_t tmp_bytes, uint32_t* keys_in,
 
 // ---- knn.hip --------------------------------------------------------------
 // Point LBVH answering "squared distance to the k-th nearest point" queries.
+// Its memory is the context's build temporaries, for the object's lifetime.
 struct KnnIndex {
     int64_t n = 0;
     Lbvh bvh;
-    DevBuf points;  // float4 [n] in leaf order
+    TmpBuf points;  // float4 [n] in leaf order
+    explicit KnnIndex(Ctx& ctx);
+    ~KnnIndex();
     // points: device xyz [*][3]; keep: optional device index list of the points to use
     void build(Ctx& ctx, int64_t n_points, const float* pts, const uint32_t* keep);
     // out[i] (device) = k-th smallest squared distance from q[i] (device xyz) to the points;
     // with n <= k the largest of the n.
     void kth_d2(Ctx& ctx, int64_t nq, const float* q, int k, float* out);
+
+  private:
+    TmpBuf nodes_;  // lends bvh.nodes its memory
 };
 // KNN_RADIUS of EmbreeBre::build: out_radius[i] (device, [n_in]) = radius * 2 sqrt(d2_k)
 // for the kept photons (keep: kept -> input index, or null for all).
