@@ -2439,7 +2439,7 @@ Split split_of(int64_t count, int64_t items, int est, Mode mode) {
     const auto fits = [&](uint32_t lg) { return (kSplitItems << lg) <= items; };
     while ((2u << s.log_parts) <= kSplitMost && (s.tiles << (s.log_parts + 1)) <= s.waves && fits(s.log_parts + 1))
         ++s.log_parts;
-    s.planned = !light && s.tiles >= kPlanTiles && s.tiles <= s.waves;
+    s.planned = !light && s.tiles >= kPlanTiles && s.tiles <= kPlanMostTiles;
     if (s.planned) {
         if (s.tiles <= kPlanFewTiles) s.waves = kPlanWaves;
         while ((2u << s.log_most) <= kPlanMost && fits(s.log_most + 1)) ++s.log_most;

@@ -295,12 +295,13 @@ struct QueryView {
 //   60k rays x 300k beams                    13.0 /  6.9 /  4.7 /  4.4 /  3.8 ms
 //   200k rays without a common origin        17.2 / 16.9 / 16.8 / 14.5 / 14.6 ms
 //   300x168 rays, UPBP                        699 /  445 /  504 /  637 /  892 us
-// Above that many tiles nothing is split: 1920x1080 rays took 12.4 ms either way at 2 parts, 13.7 at 4.
+// Above that many tiles nothing is split without a plan: 1920x1080 rays took 12.4 ms either way at 2
+// parts, 13.7 at 4.
 constexpr int64_t kSplitWaves = 16384, kSplitWavesLight = 4096;
 constexpr int64_t kSplitItems = 256, kSplitFrom = 16384;
 constexpr uint32_t kSplitMost = 64;
 
-// From kPlanTiles tiles on, up to where nothing is split, a beam launch plans: a tile gets as many of
+// From kPlanTiles to kPlanMostTiles tiles (2^21 queries) a beam launch plans: a tile gets as many of
 // kPlanWaves waves, at most kPlanMost, as its share of the estimated cost, and the dearest parts start
 // first. Estimating takes 30 to 140 us, which fewer tiles do not earn back (256x256 rays x 100k photons
 // 220 -> 270 us with 1024 tiles; photons and the UPBP kernels gain nothing and don't plan). Above
@@ -311,8 +312,12 @@ constexpr uint32_t kSplitMost = 64;
 //   60k rays x 300k beams                    4.37 / 4.13 / 3.49 / 3.41 ms
 //   400x241 rays x 200k photons + 40k beams  1.10 / 1.06 / 0.96 / 1.00 ms
 //   1M rays x 2M beams                       45.8 / 38.8 / 41.6 / 41.7 ms
+//   1920x1080 rays x 125k traced beams       88.0 / 35.2 ms
+//   1600x900 rays x 25k traced beams         20.8 / 6.07 ms
+//   1920x1080 rays x 1M photons, 200k beams  9.02 / 8.86 ms
+//   1500x1001 rays x 500k photons, 20k beams 2.02 / 2.09 ms
 constexpr uint32_t kPlanMost = 256;
-constexpr int64_t kPlanTiles = 512, kPlanFewTiles = 8192, kPlanWaves = 24576;
+constexpr int64_t kPlanTiles = 512, kPlanMostTiles = 32768, kPlanFewTiles = 8192, kPlanWaves = 24576;
 // Batched plans of this many tiles are planned too, both estimators, with kPlanWaves waves. Tiles of small
 // instances stay whole there; the order alone shortens the tail. Measured in queue order / planned:
 //   16 instances, 4.6M rays                  7.36 / 5.08 ms

@@ -1,4 +1,4 @@
-"""Beam evaluations of 512 to 16384 tiles split each tile by what it is estimated to cost (traverse.hip:
+"""Beam evaluations of 512 to 32768 tiles split each tile by what it is estimated to cost (traverse.hip:
 k_tile_cost, k_plan_parts, k_plan_tasks). Against the oracle where the plan can go wrong: the fewest
 tiles and a ragged last one, beams that all leave one point (a few tiles carry most of the cost and get
 the most parts), and batches in which some or all waves have no common origin. A second evaluation and
@@ -57,7 +57,7 @@ def test_planned_tiles_match_the_oracle(n_queries, n_items, clustered, other):
     bm.destroy()
 
 
-@pytest.mark.parametrize("n_queries", [32_768, 524_288, 1_048_576])
+@pytest.mark.parametrize("n_queries", [32_768, 524_288, 1_048_576, 2_097_152])
 def test_noalloc_plans_give_the_same_bits(n_queries):
     print_case("tile_plan_noalloc", q=n_queries)
     w = scene(n_queries, 16_384, False, 0.0)
