@@ -697,7 +697,8 @@ upbp_status upbp_batch_run(upbp_ctx* ctx, upbp_batch_plan* plan, int use_graph,
  * wave-per-block and waves-per-CU settings and keeps the fastest per
  * (structure size, query count) bucket. */
 typedef struct upbp_tuning {
-    int32_t waves_per_block;        /* 1..4: waves per workgroup of the traversal kernels */
+    int32_t waves_per_block;        /* 1..4: waves per workgroup of the traversal kernels (launches
+                                       that split their tiles choose their own) */
     int32_t blocks_per_cu;          /* persistent kernels: resident blocks per CU; 0 = occupancy-derived */
     int32_t photon_waves_per_block; /* 1..4: the photon kernel's own count; 0 = waves_per_block */
     int32_t frustum_leaf;           /* 1..64: a wave whose rays share their origin tests an inner

@@ -1541,7 +1541,7 @@ __device__ __forceinline__ int64_t xcd_block(int64_t bid, int64_t nblk) {
 // the last third of a launch; 16 neighbouring tiles at a time still share an L2. Beams and photons of
 // 1920x1080 rays: 10.9 ms with one range per XCD, 9.04 / 9.00 / 8.95 / 8.87 ms with chunks of 1 / 4 / 16 /
 // 64 blocks; a million rays on two million beams: 55.4, 46.0 / 45.5 / 47.1 / 49.0 ms.
-constexpr int64_t kXcdChunk = 4;
+constexpr int64_t kXcdChunk = 4;  // blocks of 4 waves; as many tiles of smaller blocks
 __device__ __forceinline__ int64_t xcd_round_block(int64_t bid, int64_t nblk, int64_t chunk) {
     const int64_t first = bid / (8 * chunk) * (8 * chunk);
     const int64_t left = nblk - first;
@@ -1558,7 +1558,7 @@ __global__ __launch_bounds__(256, ((MODE & 7) == (int)Mode::Upbp ? 4 : (MODE & 7
     const int waves_per_block = blockDim.x / kWave;
     // the parts of a split without a plan are spread over the blocks already
     const int64_t blk = (MODE & kSplit) && !A.tasks ? xcd_block(blockIdx.x, gridDim.x)
-                                                    : xcd_round_block(blockIdx.x, gridDim.x, kXcdChunk);
+                                                    : xcd_round_block(blockIdx.x, gridDim.x, kXcdChunk * 4 / waves_per_block);
     // wave-uniform (fewer than 2^32 waves: at most 2^26 tiles, and splits only of small batches)
     const uint32_t w = uni((uint32_t)(blk * waves_per_block + wave_in_block));
     if ((MODE & kSplit) && A.tasks && w >= as_global(A.plan)->n_tasks) return;
@@ -2157,11 +2157,15 @@ static uint32_t part_shift(int64_t items) {
     return shift;
 }
 
+// A block of one wave gives its place up as soon as that wave ends: with 1 / 2 / 4 waves of a plan per block
+// 1M rays on 2M beams take 36.7 / 38.0 / 38.7 ms, 1920x1080 rays 8.57 / 8.67 / 8.81 ms (adjoint blocks keep 4).
+constexpr int kTaskWaves = 1;
 template <int EST, int MODE>
 void launch_waves(Ctx& ctx, const EvalArgs& A, int64_t waves, int tuned) {
-    // the tuned number of waves per block, 4 with tasks, or up to 4 parts of one tile
+    // the tuned number of waves per block, one of a plan's tasks, or up to 4 parts of one tile
     const bool adjoint = (MODE & 7) == (int)Mode::Adjoint;
-    const int wpb = A.tasks || (adjoint && A.log_parts == 0) ? 4
+    const int wpb = A.tasks && !adjoint                    ? kTaskWaves
+                    : A.tasks || (adjoint && A.log_parts == 0) ? 4
                     : A.log_parts > 0                        ? std::min(1 << A.log_parts, 4)
                                                              : std::min(std::max(tuned, 1), 4);
     const dim3 blocks((unsigned)((waves + wpb - 1) / wpb)), threads((unsigned)(wpb * kWave));

@@ -312,9 +312,9 @@ constexpr uint32_t kSplitMost = 64;
 //   60k rays x 300k beams                    4.37 / 4.13 / 3.49 / 3.41 ms
 //   400x241 rays x 200k photons + 40k beams  1.10 / 1.06 / 0.96 / 1.00 ms
 //   1M rays x 2M beams                       45.8 / 38.8 / 41.6 / 41.7 ms
-//   1920x1080 rays x 125k traced beams       88.0 / 35.2 ms
+//   1920x1080 rays x 125k traced beams       88.0 / 23.0 ms
 //   1600x900 rays x 25k traced beams         20.8 / 6.07 ms
-//   1920x1080 rays x 1M photons, 200k beams  9.02 / 8.86 ms
+//   1920x1080 rays x 1M photons, 200k beams  9.02 / 8.57 ms (8.04 / 8.71 at waves_per_block 1)
 //   1500x1001 rays x 500k photons, 20k beams 2.02 / 2.09 ms
 constexpr uint32_t kPlanMost = 256;
 constexpr int64_t kPlanTiles = 512, kPlanMostTiles = 32768, kPlanFewTiles = 8192, kPlanWaves = 24576;
