@@ -1199,6 +1199,50 @@ __device__ __forceinline__ float* grad_row(const EvalArgs& A) {
     return as_global(A.grad_media) + (size_t)(blockIdx.x % kGradRows) * A.n_media * 6;
 }
 
+// A lane's query: whether its ray is evaluated (its offsets are in order and its numbers finite), else
+// with the error bits that say why not. Zeros for a lane past the last query.
+struct QueryIn {
+    float o[3], d[3];
+    int64_t s0;
+    int nseg;
+    uint32_t qi, err;  // fewer than 2^32 queries
+    bool alive;
+};
+__device__ __forceinline__ QueryIn read_query(const EvalArgs& A, int64_t slot) {
+    QueryIn q = {};
+    if (slot >= A.count) return q;
+    q.qi = A.perm ? A.perm[slot] : (uint32_t)slot;
+    const float* o = A.origin + 3 * (int64_t)q.qi;
+    const float* d = A.direction + 3 * (int64_t)q.qi;
+    for (int a = 0; a < 3; ++a) {
+        q.o[a] = o[a];
+        q.d[a] = d[a];
+    }
+    q.s0 = A.offsets[q.qi];
+    const int64_t s1 = A.offsets[(int64_t)q.qi + 1], sq = A.offsets[A.count];
+    q.nseg = (int)(s1 - q.s0);
+    q.alive = true;
+    if (!(q.s0 >= 0 && q.s0 <= s1 && s1 <= sq)) {
+        q.err |= kErrBadOffsets;
+        q.alive = false;
+    }
+    if (!finite3(q.o[0], q.o[1], q.o[2]) || !finite3(q.d[0], q.d[1], q.d[2])) {
+        q.err |= kErrNonFinite;
+        q.alive = false;
+    }
+    return q;
+}
+
+// Whether the wave's evaluated rays start at one point (true of none), with or without segments to gather.
+// This one answer says which of the two launches (in_two) a tile belongs to: the launches themselves and
+// the tile plan, which gives tasks and rows to the tiles of the first, both take it from here.
+__device__ __forceinline__ bool common_origin(const QueryIn& q) {
+    const uint64_t am = __ballot(q.alive);
+    const int fl = am ? __builtin_ctzll(am) : 0;
+    const float ox = __shfl(q.o[0], fl, kWave), oy = __shfl(q.o[1], fl, kWave), oz = __shfl(q.o[2], fl, kWave);
+    return __ballot(q.alive && !(q.o[0] == ox && q.o[1] == oy && q.o[2] == oz)) == 0;
+}
+
 __shared__ float g_part[4][3][kWave];  // the sums of a split launch's waves
 
 // Processes the 64 queries of one tile (wave) against its part of the items. `slot0` is the first
@@ -1209,41 +1253,15 @@ __device__ bool run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t slot = slot0 + lane;
     const bool valid = slot < A.count;
-    uint32_t qi = 0;  // fewer than 2^32 queries
-    if (valid) qi = A.perm ? A.perm[slot] : (uint32_t)slot;
-    uint32_t err = 0;
+    const QueryIn in = read_query(A, slot);
+    const uint32_t qi = in.qi;
+    uint32_t err = in.err;
     Ray r = {};
-    int nseg = 0;
-    bool alive = false;
-    if (valid) {
-        const float* o = A.origin + 3 * (int64_t)qi;
-        const float* d = A.direction + 3 * (int64_t)qi;
-        r.ox = o[0];
-        r.oy = o[1];
-        r.oz = o[2];
-        r.dx = d[0];
-        r.dy = d[1];
-        r.dz = d[2];
-        const int64_t s0 = A.offsets[qi], s1 = A.offsets[(int64_t)qi + 1];
-        const int64_t sq = A.offsets[A.count];
-        nseg = (int)(s1 - s0);
-        alive = true;
-        if (!(s0 >= 0 && s0 <= s1 && s1 <= sq)) {
-            err |= kErrBadOffsets;
-            alive = false;
-        }
-        if (!finite3(r.ox, r.oy, r.oz) || !finite3(r.dx, r.dy, r.dz)) {
-            err |= kErrNonFinite;
-            alive = false;
-        }
-    }
-    if (KARG && in_two(MODE)) {
-        const uint64_t am = __ballot(alive);
-        const int fl = am ? __builtin_ctzll(am) : 0;
-        const float ox = __shfl(r.ox, fl, kWave), oy = __shfl(r.oy, fl, kWave), oz = __shfl(r.oz, fl, kWave);
-        const bool one = __ballot(alive && !(r.ox == ox && r.oy == oy && r.oz == oz)) == 0;
-        if (one == ((MODE & kSparse) != 0)) return false;
-    }
+    r.ox = in.o[0], r.oy = in.o[1], r.oz = in.o[2];
+    r.dx = in.d[0], r.dy = in.d[1], r.dz = in.d[2];
+    int nseg = in.nseg;
+    bool alive = in.alive;
+    if (KARG && in_two(MODE) && common_origin(in) == ((MODE & kSparse) != 0)) return false;
     r.ix = guard_inv(r.dx);
     r.iy = guard_inv(r.dy);
     r.iz = guard_inv(r.dz);
@@ -1785,32 +1803,26 @@ __device__ __forceinline__ float tile_cost(const EvalArgs& A, int64_t slot, int 
                                            bool& one) {
     constexpr float kNode = 46.f, kLeaf = 73.f, kItem = EST == kEstPhotons ? 8.f : 20.f, kTile = 500.f;
     const int lane = threadIdx.x & (kWave - 1);
-    float ox = 0.f, oy = 0.f, oz = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
+    const QueryIn in = read_query(A, slot);
+    const float dx = in.d[0], dy = in.d[1], dz = in.d[2];
     float t0 = __builtin_inff(), t1 = -__builtin_inff();
-    if (slot < A.count) {
-        const int64_t q = A.perm ? (int64_t)A.perm[slot] : slot;
-        ox = A.origin[3 * q], oy = A.origin[3 * q + 1], oz = A.origin[3 * q + 2];
-        dx = A.direction[3 * q], dy = A.direction[3 * q + 1], dz = A.direction[3 * q + 2];
-        const int64_t s0 = A.offsets[q], s1 = A.offsets[q + 1];
-        if (s0 >= 0 && s0 <= s1 && s1 <= A.offsets[A.count] && finite3(ox, oy, oz) && finite3(dx, dy, dz))
-            for (int64_t k = s0; k < s1; ++k) {
-                const upbp_volume_segment* sg = A.segments + k;
-                const int32_t m = sg->medium_id;
-                if (m < 0 || m >= A.n_media) break;
-                if (A.media[A.media_base + m].has_scattering) {
-                    t0 = fminf(t0, sg->dist_min);
-                    t1 = fmaxf(t1, sg->dist_max);
-                }
+    if (in.alive)
+        for (int64_t k = in.s0; k < in.s0 + in.nseg; ++k) {
+            const upbp_volume_segment* sg = A.segments + k;
+            const int32_t m = sg->medium_id;
+            if (m < 0 || m >= A.n_media) break;
+            if (A.media[A.media_base + m].has_scattering) {
+                t0 = fminf(t0, sg->dist_min);
+                t1 = fmaxf(t1, sg->dist_max);
             }
-    }
+        }
     const uint64_t am = __ballot(t0 <= t1);
     float c = 0.f;
-    one = true;
+    one = common_origin(in);
     if (am) {
         const int fl = __builtin_ctzll(am);
         const bool on = t0 <= t1;
-        const float px = __shfl(ox, fl, kWave), py = __shfl(oy, fl, kWave), pz = __shfl(oz, fl, kWave);
-        one = __ballot(on && !(ox == px && oy == py && oz == pz)) == 0;
+        const float px = __shfl(in.o[0], fl, kWave), py = __shfl(in.o[1], fl, kWave), pz = __shfl(in.o[2], fl, kWave);
         const float len = __builtin_sqrtf((dx * dx + dy * dy) + dz * dz);
         const float il = on && len > 0.f ? 1.f / len : 0.f;
         const float ux = dx * il, uy = dy * il, uz = dz * il;
