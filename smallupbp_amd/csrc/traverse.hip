@@ -199,8 +199,8 @@ __device__ __forceinline__ int64_t uni64(int64_t x) { return (int64_t)uni_u64((u
 // Lane state of one segment being gathered.
 struct SegState {
     float tmin, tmax;
-    float e0, e1, e2;  // sigma_t log2(e) per channel: transmittances are exp2(-e t)
-    float ek;          // the smallest sigma_t's (what SHORT beams are normalised by)
+    float x0, x1, x2;  // per channel, what a length of the query adds to log2 of its factor (set_factors)
+    float ek;          // sigma_t log2(e) of the smallest sigma_t (what SHORT beams are normalised by)
     float ss0, ss1, ss2;
     float g;           // 0 for isotropic media, where phase_pdf gives the constant exactly
     int32_t kidx;      // the smallest sigma_t's channel (adjoint)
@@ -264,19 +264,38 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
 }
 
 // ---- leaf visitors ---------------------------------------------------------
-// One fused multiply-add and one exp2 per channel: the exponents with their products, differences and
-// selections, and the per-lane choice of phase function, were 50 of the 80 vector instructions of a beam
-// hit, which made 1920x1080 rays x 200k SHORT beams 11.8 ms; 10.9 ms with these and the record read
-// in one go (test_beam_beam).
-// exp2 of the channels' transmittance exponents along `dist` with the SHORT normalisations folded in:
-// exp2(-e_c dist + ek norm) = T_c(dist) / T_k(norm), norm the part of dist that is SHORT.
+// A hit's transmittance factors, exp2 of an exponent per channel c: a length adds -e_c to it, e_c =
+// sigma_t_c log2(e), or where it is SHORT, whose transmittance is divided by channel k's, e_k - e_c. That
+// is formed before it is multiplied by the length, so that the factor of channel k (of all channels of a
+// grey medium) is exactly 1 there, however thick the medium: e_k times the SHORT lengths, rounded, less
+// e_c times all lengths was off by 5e-6 of it at sigma_t 80 (and two instructions per beam hit less: 8.55
+// instead of 8.64 ms for 1920x1080 rays x 1M photons + 200k SHORT beams). Three multiplies for a photon
+// hit, three instructions per channel for a beam hit, and one exp2 each: the exponents with products,
+// differences and selections per lane, and the per-lane choice of phase function, were 50 of the 80
+// vector instructions of a beam hit and made that evaluation 11.8 ms; 10.9 ms without those and with the
+// record read in one go (test_beam_beam).
 struct Trans {
     float c0, c1, c2;
 };
-__device__ __forceinline__ Trans transmittance(const SegState& s, float dist, float norm) {
-    const float k = s.ek * norm;
-    return {__builtin_amdgcn_exp2f(__builtin_fmaf(-s.e0, dist, k)), __builtin_amdgcn_exp2f(__builtin_fmaf(-s.e1, dist, k)),
-            __builtin_amdgcn_exp2f(__builtin_fmaf(-s.e2, dist, k))};
+__device__ __forceinline__ void set_factors(SegState& s, float st0, float st1, float st2, int min_idx, bool short_q) {
+    const float stk = pick3(min_idx, st0, st1, st2);
+    s.ek = stk * kLog2e;
+    s.x0 = (short_q ? stk - st0 : -st0) * kLog2e;
+    s.x1 = (short_q ? stk - st1 : -st1) * kLog2e;
+    s.x2 = (short_q ? stk - st2 : -st2) * kLog2e;
+}
+// of a photon at dt along the query
+__device__ __forceinline__ Trans transmittance(const SegState& s, float dt) {
+    return {__builtin_amdgcn_exp2f(s.x0 * dt), __builtin_amdgcn_exp2f(s.x1 * dt), __builtin_amdgcn_exp2f(s.x2 * dt)};
+}
+// of dq along the query and t2 along a beam; kb: 1 for a SHORT beam less 1 for a SHORT query (short_diff)
+__device__ __forceinline__ float short_diff(bool short_b, bool short_q) {
+    return (short_b ? 1.f : 0.f) - (short_q ? 1.f : 0.f);
+}
+__device__ __forceinline__ Trans transmittance(const SegState& s, float dq, float t2, float kb) {
+    return {__builtin_amdgcn_exp2f(__builtin_fmaf(__builtin_fmaf(kb, s.ek, s.x0), t2, s.x0 * dq)),
+            __builtin_amdgcn_exp2f(__builtin_fmaf(__builtin_fmaf(kb, s.ek, s.x1), t2, s.x1 * dq)),
+            __builtin_amdgcn_exp2f(__builtin_fmaf(__builtin_fmaf(kb, s.ek, s.x2), t2, s.x2 * dq))};
 }
 
 // Sums the three channels' item gradients over the wave (DPP) and adds them once: lanes 0 to 2 add one
@@ -325,7 +344,7 @@ __device__ void photon_hit_mis(const EvalArgs& A, const Ray& r, SegState& s, con
     // roots are the single hardware instructions.
     const float dt = t - s.tmin;
     const float pdf = __builtin_amdgcn_exp2f(-s.ek * dt);
-    const Trans tr = transmittance(s, dt, short_q ? dt : 0.f);
+    const Trans tr = transmittance(s, dt);
     const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
     float ray_pdf = s.min_comp * pdf;
     float ray_rev = (ml.seg_flags & UPBP_ORIGIN_IN_MEDIUM) ? ray_pdf : pdf;
@@ -398,7 +417,7 @@ __device__ void beam_hit_mis(const EvalArgs& A, const Ray& r, SegState& s, const
     // beam transmittances together (with the SHORT normalisations folded into the exponent).
     const float dq = t1 - s.tmin;
     const float pq = __builtin_amdgcn_exp2f(-s.ek * dq), pb = __builtin_amdgcn_exp2f(-s.ek * t2);
-    const Trans tr = transmittance(s, dq + t2, (short_q ? dq : 0.f) + (short_b ? t2 : 0.f));
+    const Trans tr = transmittance(s, dq, t2, short_diff(short_b, short_q));
     const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
     float rsp_q = s.min_comp * pq;
     float rsr_q = (ml.seg_flags & UPBP_ORIGIN_IN_MEDIUM) ? rsp_q : pq;
@@ -492,9 +511,9 @@ __device__ __forceinline__ void owner_state(const Ray& r, const SegState& s, con
     ro.dy = from_lane(r.dy, owner);
     ro.dz = from_lane(r.dz, owner);
     so.tmin = from_lane(s.tmin, owner);
-    so.e0 = from_lane(s.e0, owner);
-    so.e1 = from_lane(s.e1, owner);
-    so.e2 = from_lane(s.e2, owner);
+    so.x0 = from_lane(s.x0, owner);
+    so.x1 = from_lane(s.x1, owner);
+    so.x2 = from_lane(s.x2, owner);
     so.ek = from_lane(s.ek, owner);
     so.ss0 = from_lane(s.ss0, owner);
     so.ss1 = from_lane(s.ss1, owner);
@@ -635,7 +654,7 @@ __device__ __forceinline__ void photon_leaf(const EvalArgs& A, const Ray& r, Seg
             float gp0 = 0.f, gp1 = 0.f, gp2 = 0.f;
             if (hit) {
                 const float dt = t - s.tmin;
-                const Trans tr = transmittance(s, dt, short_q ? dt : 0.f);
+                const Trans tr = transmittance(s, dt);
                 const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
                 float ph = kInvPi * 0.25f;
                 if (lo.aniso) {
@@ -915,10 +934,8 @@ __device__ __forceinline__ void beam_leaf(const EvalArgs& A, const Ray& r, SegSt
             if (hit && red_n != 0) {
                 const bool short_b = (word & kShortBeamBit) != 0;
                 const float dq = t1 - s.tmin;
-                // T(t1 - tmin) [/ T_k] * T(t2) [/ T_k(t2)], one exponential per channel; the two
-                // normalised lengths are selected by scalar factors
-                const float kq = short_q ? 1.f : 0.f, kb = short_b ? 1.f : 0.f;
-                const Trans tr = transmittance(s, dq + t2, __builtin_fmaf(kq, dq, kb * t2));
+                // T(t1 - tmin) [/ T_k] * T(t2) [/ T_k(t2)], one exponential per channel
+                const Trans tr = transmittance(s, dq, t2, short_diff(short_b, short_q));
                 const float a0 = tr.c0, a1 = tr.c1, a2 = tr.c2;
                 // phase: Evaluate(ray.direction, beam direction), cos = -dot(d2, d1)
                 const float ph = lo.aniso ? phase_pdf(s.g, false, -dot3(pc.p1.x, pc.p1.y, pc.p1.z, r.dx, r.dy, r.dz))
@@ -995,9 +1012,9 @@ __device__ __forceinline__ void drain_pairs(const EvalArgs& A, const Ray& r, con
     const float dx = from_lane(r.dx, owner), dy = from_lane(r.dy, owner), dz = from_lane(r.dz, owner);
     const float tmin = from_lane(s.tmin, owner), tmax = from_lane(s.tmax, owner);
     SegState so;
-    so.e0 = from_lane(s.e0, owner);
-    so.e1 = from_lane(s.e1, owner);
-    so.e2 = from_lane(s.e2, owner);
+    so.x0 = from_lane(s.x0, owner);
+    so.x1 = from_lane(s.x1, owner);
+    so.x2 = from_lane(s.x2, owner);
     so.ek = from_lane(s.ek, owner);
     const float ss0 = from_lane(s.ss0, owner), ss1 = from_lane(s.ss1, owner), ss2 = from_lane(s.ss2, owner);
     const float g = from_lane(s.g, owner);
@@ -1010,7 +1027,7 @@ __device__ __forceinline__ void drain_pairs(const EvalArgs& A, const Ray& r, con
         if (hit && (MODE & 7) == (int)Mode::Forward) {
             const float4 pw = A.power[i];
             const float dt = t - tmin;
-            const Trans tr = transmittance(so, dt, short_q ? dt : 0.f);
+            const Trans tr = transmittance(so, dt);
             float ph = kInvPi * 0.25f;
             if (lo.aniso) {
                 const float4 in = A.inc[i];
@@ -1033,7 +1050,7 @@ __device__ __forceinline__ void drain_pairs(const EvalArgs& A, const Ray& r, con
         if (hit && (MODE & 7) == (int)Mode::Forward) {
             const float4 flux = A.piece_flux[i];
             const float dq = t1 - tmin;
-            const Trans tr = transmittance(so, dq + t2, (short_q ? dq : 0.f) + ((word & kShortBeamBit) ? t2 : 0.f));
+            const Trans tr = transmittance(so, dq, t2, short_diff((word & kShortBeamBit) != 0, short_q));
             const float ph = lo.aniso ? phase_pdf(g, false, -dot3(pc.p1.x, pc.p1.y, pc.p1.z, dx, dy, dz))
                                       : kInvPi * 0.25f;
             const float kern = radial_kernel(dist * dist, radius * radius);
@@ -1327,7 +1344,7 @@ __device__ bool run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
         SegState s;
         s.tmin = __builtin_inff();
         s.tmax = -__builtin_inff();
-        s.e0 = s.e1 = s.e2 = s.ek = 0.f;
+        s.x0 = s.x1 = s.x2 = s.ek = 0.f;
         s.ss0 = s.ss1 = s.ss2 = 0.f;
         s.g = 0.f;
         s.kidx = 0;
@@ -1367,10 +1384,7 @@ __device__ bool run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
                 if (scatter) {
                     s.tmin = tmin;
                     s.tmax = tmax;
-                    s.e0 = m->st[0] * kLog2e;
-                    s.e1 = m->st[1] * kLog2e;
-                    s.e2 = m->st[2] * kLog2e;
-                    s.ek = pick3(m->min_idx, s.e0, s.e1, s.e2);
+                    set_factors(s, m->st[0], m->st[1], m->st[2], m->min_idx, short_q);
                     s.ss0 = m->ss[0];
                     s.ss1 = m->ss[1];
                     s.ss2 = m->ss[2];
