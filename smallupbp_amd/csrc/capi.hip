@@ -321,6 +321,16 @@ struct RunOut {
     uint32_t* sig_bm = nullptr;
 };
 
+// Whether a caller records this stream into a graph. Such an evaluation splits nothing: a split's rows and
+// plan lie in buffers of the context that may have to be allocated, which a capture refuses, and that a
+// later, larger call replaces while the graph still holds their addresses. (An evaluation in the caller's
+// scratch region may split: that region stays.)
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    UPBP_HIP(hipStreamIsCapturing(stream, &st));
+    return st != hipStreamCaptureStatusNone;
+}
+
 // scratch_base: the fixed region that holds the call's workspace (null: the context's own buffers).
 void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch* q, Mode mode, RunOut o,
               upbp_memory out_mem, upbp_eval_stats* stats, const AdjointOut* adj_ph, const AdjointOut* adj_bm,
@@ -335,8 +345,9 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     if (timing) UPBP_HIP(hipEventRecord(ctx.ev[0], ctx.stream));
     float lo[3], hi[3];
     scene_bounds(bre, bm, lo, hi);
-    const Split split[2] = {want_ph ? split_of(Q, bre->n, 0, mode) : Split(),
-                            want_bm ? split_of(Q, bm->pieces, 1, mode) : Split()};
+    Split split[2] = {want_ph ? split_of(Q, bre->n, 0, mode) : Split(),
+                      want_bm ? split_of(Q, bm->pieces, 1, mode) : Split()};
+    if (!scratch_base && capturing(ctx.stream)) split[0] = split[1] = Split();
     const Workspace own = scratch_base ? scratch_workspace(scratch_base, Q, split) : context_workspace(ctx, q, split);
     const Workspace* ws = &own;
     QueryView v = make_view(ctx, q, lo, hi, !want_bm, *ws);
