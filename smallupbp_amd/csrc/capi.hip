@@ -347,7 +347,10 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
     scene_bounds(bre, bm, lo, hi);
     Split split[2] = {want_ph ? split_of(Q, bre->n, 0, mode) : Split(),
                       want_bm ? split_of(Q, bm->pieces, 1, mode) : Split()};
-    if (!scratch_base && capturing(ctx.stream)) split[0] = split[1] = Split();
+    const bool captured = !scratch_base && capturing(ctx.stream);
+    if (captured) split[0] = split[1] = Split();
+    const bool own_buffers = !scratch_base && !captured;
+    if (own_buffers && ctx.in_use) UPBP_HIP(hipStreamWaitEvent(ctx.stream, ctx.used, 0));
     const Workspace own = scratch_base ? scratch_workspace(scratch_base, Q, split) : context_workspace(ctx, q, split);
     const Workspace* ws = &own;
     QueryView v = make_view(ctx, q, lo, hi, !want_bm, *ws);
@@ -435,10 +438,17 @@ void run_eval(Ctx& ctx, const Bre* bre, const Beams* bm, const upbp_query_batch*
         if (o.sig_bm && want_bm) UPBP_HIP(hipMemcpyAsync(o.sig_bm, sbm, Q * 8, hipMemcpyDeviceToHost, ctx.stream));
     }
     const bool do_sync = ctx.sync || timing || force_sync || out_mem == UPBP_MEM_HOST || q->memory == UPBP_MEM_HOST;
-    if (!do_sync) return;
+    if (!do_sync) {
+        if (own_buffers) {
+            UPBP_HIP(hipEventRecord(ctx.used, ctx.stream));
+            ctx.in_use = true;
+        }
+        return;
+    }
     uint64_t rows[kStatWords], st[kStatSlots];
     UPBP_HIP(hipMemcpyAsync(rows, ws->stats, sizeof(rows), hipMemcpyDeviceToHost, ctx.stream));
     UPBP_HIP(hipStreamSynchronize(ctx.stream));
+    if (own_buffers) ctx.in_use = false;
     sum_stats(rows, st);
     float ms_other = 0.f, ms_ph = 0.f, ms_bm = 0.f;
     if (timing) {
@@ -478,6 +488,7 @@ upbp_status upbp_ctx_create(int device, upbp_ctx** out_ctx) {
         UPBP_HIP(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
         UPBP_HIP(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming));
         UPBP_HIP(hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming));
+        UPBP_HIP(hipEventCreateWithFlags(&ctx->used, hipEventDisableTiming));
         ctx->stats.ensure(kStatAll * 8);
         ctx->scratch = scratch_address(device, ctx->scratch_error);
         *out_ctx = ctx;
@@ -504,6 +515,7 @@ void ctx_release(Ctx* ctx) {
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     if (ctx->fork) (void)hipEventDestroy(ctx->fork);
     if (ctx->join) (void)hipEventDestroy(ctx->join);
+    if (ctx->used) (void)hipEventDestroy(ctx->used);
     if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete static_cast<upbp_ctx*>(ctx);

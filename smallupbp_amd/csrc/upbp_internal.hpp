@@ -170,6 +170,10 @@ struct Ctx {
     // (fork from `stream`, join back), so one kernel's tail overlaps the other's work
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
+    // An evaluation that returned before its work ended, and the end of that work: the next one, which may
+    // be on another stream (upbp_ctx_set_stream), waits for it, as both work in the buffers above.
+    bool in_use = false;
+    hipEvent_t used = nullptr;
     // resident blocks per CU of the two persistent batched kernels at batched_key waves per block
     int batched_key = 0;
     int batched_per_cu[2] = {0, 0};
