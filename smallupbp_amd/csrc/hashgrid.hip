@@ -468,18 +468,22 @@ template <class Cam>
 __device__ __forceinline__ void vm_drain(const VmArgs& A, VmLds<Cam>& L, uint32_t head, uint32_t n, uint32_t& err) {
     const int w = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63u;
-    if (lane >= n) return;
-    const uint32_t at = (head + lane) & (kHitRing - 1);
-    const uint32_t k = L.slot[w][at], o = L.owner[w][at];
-    Cam c;
-    float* words = reinterpret_cast<float*>(&c);
-    for (int i = 0; i < Cam::kWords - kCamWords; ++i) words[i] = L.cam[w][kCamWords + i][o];
-    const CamSplit cs = {L.cam[w][1][o], L.cam[w][2][o], L.cam[w][3][o]};
-    float v[3];
-    if (!vm_process(A, c, __float_as_uint(L.cam[w][0][o]), cs, k, v, err)) return;
-    atomicAdd(&L.acc[w][0][o], v[0]);
-    atomicAdd(&L.acc[w][1][o], v[1]);
-    atomicAdd(&L.acc[w][2][o], v[2]);
+    wave_lds_sync();
+    if (lane < n) {
+        const uint32_t at = (head + lane) & (kHitRing - 1);
+        const uint32_t k = L.slot[w][at], o = L.owner[w][at];
+        Cam c;
+        float* words = reinterpret_cast<float*>(&c);
+        for (int i = 0; i < Cam::kWords - kCamWords; ++i) words[i] = L.cam[w][kCamWords + i][o];
+        const CamSplit cs = {L.cam[w][1][o], L.cam[w][2][o], L.cam[w][3][o]};
+        float v[3];
+        if (vm_process(A, c, __float_as_uint(L.cam[w][0][o]), cs, k, v, err)) {
+            atomicAdd(&L.acc[w][0][o], v[0]);
+            atomicAdd(&L.acc[w][1][o], v[1]);
+            atomicAdd(&L.acc[w][2][o], v[2]);
+        }
+    }
+    wave_lds_sync();
 }
 
 // HashGrid::Process (HashGrid.hxx:130-186), one lane per camera vertex: the eight buckets' ranges are

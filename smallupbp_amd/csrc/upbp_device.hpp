@@ -164,6 +164,24 @@ __device__ __forceinline__ bool test_beam_beam(bool same_medium, float o1x, floa
     return ok;
 }
 
+// Between lanes of one wave that write LDS and lanes that read it (and the other way round). The LDS
+// carries out a wave's operations in order, so this adds no instruction: it keeps the compiler from
+// moving them, which without it sees each lane's own accesses only. The compiler counts it as a write to
+// all memory, though: where uniform reads have to stay scalar loads, the accesses themselves are
+// volatile instead (lds_read, lds_write), which are kept in order too.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+template <class T>
+__device__ __forceinline__ T lds_read(const T& x) {
+    return *(const volatile __attribute__((address_space(3))) T*)&x;
+}
+template <class T>
+__device__ __forceinline__ void lds_write(T& x, T v) {
+    *(volatile __attribute__((address_space(3))) T*)&x = v;
+}
+
 constexpr float kLog2e = 1.4426950408889634f;
 // exp(x) for x <= 0 through the hardware base-2 exponential.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
