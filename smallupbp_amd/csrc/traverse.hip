@@ -1126,7 +1126,7 @@ __device__ __forceinline__ uint64_t end_pieces(const EvalArgs& A, uint32_t start
 
 // ---- wave-cooperative traversal ------------------------------------------
 // The items [start, start + cnt) (cnt <= 64) of a leaf that the rays of `lanes` meet the box of, culled
-// against the wave's frustum first when it has one.
+// against the wave's frustum first when it has one. tested: the items that the whole wave tests.
 template <int EST, int MODE>
 __device__ __forceinline__ void visit_leaf(const EvalArgs& A, const Frustum& F, bool fr, ItemPart part,
                                            uint64_t lanes, const Ray& r, SegState& s, LaneOut<MODE>& lo,
@@ -1134,7 +1134,7 @@ __device__ __forceinline__ void visit_leaf(const EvalArgs& A, const Frustum& F, 
     const uint64_t all = (MODE & kSplit) ? part.items(start, cnt) : cnt >= 64u ? ~0ull : ((1ull << cnt) - 1ull);
     if ((MODE & kSparse) && __popcll(lanes) <= kSparseLanes) {
         const uint64_t ends = EST == kEstPhotons ? 0ull : end_pieces(A, start) & all;
-        tested += (uint32_t)__popcll(all);
+        tested += (uint32_t)__popcll(ends);
         if (EST == kEstBeams) beam_leaf<MODE>(A, r, s, lo, start, ends, short_q);
         queue_pairs<EST, MODE>(A, r, s, lo, lanes, start, all & ~ends, short_q);
     } else if (EST == kEstPhotons) {
@@ -1157,6 +1157,7 @@ __device__ __forceinline__ void traverse(const EvalArgs& A, ItemPart part, const
     int sp = 0;
     uint32_t node = A.root;
     uint32_t tested = 0;
+    const uint32_t queued = lo.qt;
     Frustum F;
     const bool fr = !(MODE & kSparse) && make_frustum(r, s, F);
     while (true) {
@@ -1209,6 +1210,7 @@ __device__ __forceinline__ void traverse(const EvalArgs& A, ItemPart part, const
         }
     }
     tests += (uint64_t)tested * (uint32_t)__popcll(__ballot(s.tmin <= s.tmax));
+    if (MODE & kSparse) tests += lo.qt - queued;  // pairs
 }
 
 __device__ __forceinline__ bool finite3(float x, float y, float z) {
