@@ -693,9 +693,9 @@ upbp_status upbp_batch_run(upbp_ctx* ctx, upbp_batch_plan* plan, int use_graph,
                            upbp_eval_stats* stats);
 
 /* ---------------------------------------------------------------------------
- * Launch tuning. The autotuner times the traversal kernels over a grid of
- * wave-per-block and waves-per-CU settings and keeps the fastest per
- * (structure size, query count) bucket. */
+ * Launch tuning. The autotuner times the traversal kernels with 1, 2 and 4
+ * waves per block and keeps the fastest; the tuning stays as it is where every
+ * launch of the batch splits its tiles (and chooses its own). */
 typedef struct upbp_tuning {
     int32_t waves_per_block;        /* 1..4: waves per workgroup of the traversal kernels (launches
                                        that split their tiles choose their own) */

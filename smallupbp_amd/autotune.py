@@ -4,7 +4,8 @@ Searches the parameters that the GPU path exposes and keeps the fastest per
 workload-size bucket:
   build-time: LBVH leaf size (items per leaf tile, 4..64) for photons and for
               beam pieces, and the beam piece length (in units of the beam radius);
-  launch-time: waves per workgroup (1, 2, 4) and the query order (Morton-sorted
+  launch-time: waves per workgroup (1, 2, 4; where the launch takes them, see
+              takes_waves) and the query order (Morton-sorted
               bundles or the caller's order); with both estimators, the photon kernel's
               waves per workgroup once more on the joint (concurrent) step.
 Times come from the library's HIP events around each traversal kernel (median of
@@ -32,6 +33,24 @@ BEAM_LEAF = (4, 8, 16, 32, 64)
 PIECE_FACTOR = (4.0, 8.0, 16.0, 32.0)
 WAVES = (1, 2, 4)
 ORDERS = (_abi.ORDER_SORTED, _abi.ORDER_AS_GIVEN)
+
+
+# Launches that split their tiles of 64 queries over waves, or plan them, choose their waves per
+# workgroup themselves (csrc/upbp_internal.hpp: kSplitFrom items or more, and at most half of
+# kSplitWavesLight tiles for photons, kPlanMostTiles for beams).
+SPLIT_FROM = 16384
+PHOTON_SPLIT_TILES = 4096 // 2
+BEAM_SPLIT_TILES = 32768
+
+
+def takes_waves(estimator: str, n_items: int, n_queries: int) -> bool:
+    """Whether an evaluation of n_queries on n_items photons or beam pieces has the tuned waves per workgroup."""
+    most = PHOTON_SPLIT_TILES if estimator == "photons" else BEAM_SPLIT_TILES
+    return n_items < SPLIT_FROM or (n_queries + 63) // 64 > most
+
+
+def waves_to_try(ctx, estimator: str, n_items: int, n_queries: int):
+    return WAVES if takes_waves(estimator, n_items, n_queries) else (ctx.get_tuning()[0],)
 
 
 def bucket(n_photons: int, n_beams: int, n_queries: int) -> str:
@@ -104,7 +123,7 @@ def tune(w: scenes.Workload, reps: int = 3, path: Optional[str] = DEFAULT_CACHE,
         for leaf in PHOTON_LEAF:
             bre = native.EmbreeBre(ctx)
             bre.build(w.photons, leaf_size=leaf)
-            for wpb, order in itertools.product(WAVES, ORDERS):
+            for wpb, order in itertools.product(waves_to_try(ctx, "photons", bre.num_photons, w.queries.count), ORDERS):
                 ctx.set_tuning(wpb)
                 native.eval_batch(ctx, bre, None, qviews[order])  # warm
                 ms = _median_kernel_ms(ctx, bre, None, qviews[order], reps, "photons")
@@ -118,7 +137,7 @@ def tune(w: scenes.Workload, reps: int = 3, path: Optional[str] = DEFAULT_CACHE,
         for leaf, pf in itertools.product(BEAM_LEAF, PIECE_FACTOR):
             bm = native.PhotonBeamsEvaluator(ctx)
             bm.build(w.beams, leaf_size=leaf, piece_factor=pf)
-            for wpb, order in itertools.product(WAVES, ORDERS):
+            for wpb, order in itertools.product(waves_to_try(ctx, "beams", bm.pieces, w.queries.count), ORDERS):
                 ctx.set_tuning(wpb)
                 native.eval_batch(ctx, None, bm, qviews[order])
                 ms = _median_kernel_ms(ctx, None, bm, qviews[order], reps, "beams")
@@ -139,7 +158,7 @@ def tune(w: scenes.Workload, reps: int = 3, path: Optional[str] = DEFAULT_CACHE,
         bm.build(w.beams, leaf_size=best["beams"]["leaf_size"], piece_factor=best["beams"]["piece_factor"])
         qv = qviews[best["beams"]["order"]]
         joint = []
-        for wpb in WAVES:
+        for wpb in WAVES if takes_waves("photons", bre.num_photons, w.queries.count) else (best["photons"]["waves_per_block"],):
             ctx.set_tuning(best["beams"]["waves_per_block"], 0, wpb)
             native.eval_batch(ctx, bre, bm, qv)  # warm
             ms = _median_step_ms(ctx, bre, bm, qv, reps)

@@ -1543,7 +1543,11 @@ upbp_status upbp_autotune(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* 
         Tuning saved = ctx->tuning;
         float best_t = INFINITY;
         Tuning best_cfg = saved;
-        const int cand[3] = {1, 2, 4};
+        // launches that split their tiles choose their waves per block themselves: where all do, there is
+        // nothing to choose, and the tuning stays for other launches
+        const bool whole = (bre && bre->n > 0 && split_of(Q, bre->n, 0, Mode::Forward).whole()) ||
+                           (beams && beams->pieces > 0 && split_of(Q, beams->pieces, 1, Mode::Forward).whole());
+        const std::vector<int> cand = whole ? std::vector<int>{1, 2, 4} : std::vector<int>{saved.waves_per_block};
         for (int wpb : cand) {
             ctx->tuning.waves_per_block = wpb;
             RunOut o;

@@ -231,6 +231,8 @@ struct Split {
     uint32_t log_parts = 0, log_most = 0;
     bool planned = false;
     int64_t rows = 0;  // sums of parts kept for k_sum_rows, 64 x 3 floats each
+    // whether the launch has the tuned number of waves per block (launch_waves chooses for the others)
+    bool whole() const { return log_parts == 0 && !planned; }
 };
 
 // Device memory of a split: the rows, and of a plan the tiles' costs, their part counts and first rows,
