@@ -1392,8 +1392,11 @@ upbp_status upbp_batch_plan_create(upbp_ctx* ctx, const upbp_instance* instances
             for (int e = 0; e < 2; ++e) {
                 Split s;
                 s.tiles = tiles;
-                s.waves = s.rows = kPlanWaves;
+                s.waves = kPlanWaves;
                 s.planned = true;
+                // rows only where some instance is large enough for its tiles to be split
+                for (const InstanceDev& d : plan->host)
+                    if ((e == 0 ? d.ph_log_most : d.bm_log_most) > 0) s.rows = kPlanWaves;
                 plan->split_mem[e].ensure(TilePlan::bytes(s));
                 plan->split.plan[e] = TilePlan::at(s, plan->split_mem[e].as<char>());
                 plan->split.plan[e].words = reinterpret_cast<PlanWords*>(plan->counters.as<char>() + 64) + e;
