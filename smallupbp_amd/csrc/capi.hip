@@ -1172,8 +1172,9 @@ upbp_status upbp_adjoint(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* b
         const float* gph = do_ph ? stage_q(*ctx, 4, grad_out_photons, 3 * Q, memory) : nullptr;
         const float* gbm = do_bm ? stage_q(*ctx, 5, grad_out_beams, 3 * Q, memory) : nullptr;
         TmpBuf gmedia(ctx->tmp), items_ph(ctx->tmp), items_bm(ctx->tmp);
-        gmedia.ensure((size_t)kGradRows * M * 6 * 4);
-        launch_clear_f32(*ctx, gmedia.as<float>(), (int64_t)kGradRows * M * 6);
+        const int64_t n_grad = (int64_t)grad_rows(M) * M * 6;
+        gmedia.ensure((size_t)n_grad * 4);
+        launch_clear_f32(*ctx, gmedia.as<float>(), n_grad);
         float* dpp = grad_photon_power;
         float* dbp = grad_beam_power;
         if (memory == UPBP_MEM_HOST) {
@@ -1210,7 +1211,7 @@ upbp_status upbp_adjoint(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* b
                                        grad_absorption);
             UPBP_HIP(hipStreamSynchronize(ctx->stream));
         } else {
-            std::vector<float> rows((size_t)kGradRows * M * 6), gm((size_t)M * 6, 0.f);
+            std::vector<float> rows((size_t)n_grad), gm((size_t)M * 6, 0.f);
             UPBP_HIP(hipMemcpy(rows.data(), gmedia.p, rows.size() * 4, hipMemcpyDeviceToHost));
             for (size_t i = 0; i < rows.size(); ++i) gm[i % gm.size()] += rows[i];
             const std::vector<float>& sg = ctx->media_sign_host;

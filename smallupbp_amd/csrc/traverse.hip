@@ -61,7 +61,7 @@ struct EvalArgs {
     unsigned long long* __restrict__ stats;
     // adjoint
     const float* __restrict__ grad_out;
-    float* __restrict__ grad_media;  // [kGradRows][M][6]: a wave adds to its block's row
+    float* __restrict__ grad_media;  // [grad_mask + 1][M][6]: a wave adds to its block's row
     float* __restrict__ grad_items;  // [items][3]
     // UPBP mode
     const upbp_query_mis* __restrict__ qmis;
@@ -79,6 +79,7 @@ struct EvalArgs {
     PlanWords* __restrict__ plan;
     uint32_t shift;  // ItemPart::shift of one part; half the items per block for twice the parts, at least 64
     uint32_t log_parts, row0;
+    uint32_t grad_mask;  // adjoint
     float* __restrict__ rows;
 };
 
@@ -1219,7 +1220,7 @@ __device__ __forceinline__ bool finite3(float x, float y, float z) {
 
 // The block's row of the medium gradients (media_base is 0 outside batched plans, which have no adjoint).
 __device__ __forceinline__ float* grad_row(const EvalArgs& A) {
-    return as_global(A.grad_media) + (size_t)(blockIdx.x % kGradRows) * A.n_media * 6;
+    return as_global(A.grad_media) + (size_t)(blockIdx.x & A.grad_mask) * A.n_media * 6;
 }
 
 // A lane's query: whether its ray is evaluated (its offsets are in order and its numbers finite), else
@@ -2075,12 +2076,12 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, int64_t n) {
     if (i < n) p[i] = v;
 }
 
-__global__ void k_combine_media(const float* gm, const float* sign, int n, float* gs, float* ga) {
+__global__ void k_combine_media(const float* gm, int rows, const float* sign, int n, float* gs, float* ga) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 3 * n) return;
     const int m = i / 3, c = i % 3;
     float direct = 0.f, dt = 0.f;
-    for (int r = 0; r < kGradRows; ++r) {
+    for (int r = 0; r < rows; ++r) {
         direct += gm[6 * ((size_t)r * n + m) + c];
         dt += gm[6 * ((size_t)r * n + m) + 3 + c];
     }
@@ -2526,6 +2527,7 @@ void launch_photons(Ctx& ctx, Mode mode, const PhotonArgs& ph, const QueryView& 
     if (adj) {
         A.grad_out = adj->grad_out;
         A.grad_media = adj->grad_media;
+        A.grad_mask = (uint32_t)grad_rows(ctx.n_media) - 1u;
         A.grad_items = adj->grad_items;
     }
     const int want = ctx.tuning.photon_waves_per_block > 0 ? ctx.tuning.photon_waves_per_block
@@ -2550,6 +2552,7 @@ void launch_beams(Ctx& ctx, Mode mode, const BeamArgs& bm, const QueryView& q, f
     if (adj) {
         A.grad_out = adj->grad_out;
         A.grad_media = adj->grad_media;
+        A.grad_mask = (uint32_t)grad_rows(ctx.n_media) - 1u;
         A.grad_items = adj->grad_items;
     }
     launch_mode<kEstBeams>(ctx, mode, A, q, bm.pieces_n, ctx.tuning.waves_per_block);
@@ -2680,8 +2683,8 @@ void launch_fill_u32(Ctx& ctx, uint32_t* p, uint32_t v, int64_t n) {
 }
 
 void launch_combine_media_grads(Ctx& ctx, const float* gm, const float* sign, int n_media, float* gs, float* ga) {
-    hipLaunchKernelGGL(k_combine_media, dim3(grid_for(3 * n_media)), dim3(256), 0, ctx.stream, gm, sign, n_media, gs,
-                       ga);
+    hipLaunchKernelGGL(k_combine_media, dim3(grid_for(3 * n_media)), dim3(256), 0, ctx.stream, gm, grad_rows(n_media), sign,
+                       n_media, gs, ga);
     UPBP_HIP(hipGetLastError());
 }
 

@@ -423,11 +423,18 @@ struct BeamArgs {
     RedDev red;
 };
 // Rows of medium gradients that the adjoint's waves spread their atomics over (each wave adds 6 values
-// per medium: on one row they queue for the same words).
+// per medium: on one row they queue for the same words), a power of two: up to kGradRows, and for a table
+// of more than 1024 media as few as keep them all within 1.5 MB (64 rows of a million would be 1.5 GB).
 constexpr int kGradRows = 64;
+constexpr int64_t kGradRowMedia = 65536;
+inline int grad_rows(int64_t n_media) {
+    int rows = kGradRows;
+    while (rows > 1 && rows * n_media > kGradRowMedia) rows /= 2;
+    return rows;
+}
 struct AdjointOut {
     const float* grad_out;  // [Q][3]
-    float* grad_media;      // [kGradRows][M][6]: dsigma_s direct (0..2), dsigma_t (3..5)
+    float* grad_media;      // [grad_rows(M)][M][6]: dsigma_s direct (0..2), dsigma_t (3..5)
     float* grad_items;      // photon [n_in][3] or beam [n][3]
 };
 
@@ -474,7 +481,7 @@ void launch_sum_rows_sig(Ctx& ctx, const QueryView& q, uint32_t* ph, uint32_t* b
 void launch_clear_u64(Ctx& ctx, uint64_t* p, int64_t n);
 void launch_clear_f32(Ctx& ctx, float* p, int64_t n);
 // gs += sign_s * (direct + d/d sigma_t), ga += sign_a * d/d sigma_t per medium and channel, summed
-// over the kGradRows rows of gm (sign: [M][6] of ctx.media_sign).
+// over the grad_rows rows of gm (sign: [M][6] of ctx.media_sign).
 void launch_combine_media_grads(Ctx& ctx, const float* gm, const float* sign, int n_media, float* gs, float* ga);
 
 // ---- hashgrid.hip: vertex-merging hashed grid (PP3D, SURF) --------------------
