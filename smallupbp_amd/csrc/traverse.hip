@@ -1257,14 +1257,31 @@ __device__ __forceinline__ QueryIn read_query(const EvalArgs& A, int64_t slot) {
     return q;
 }
 
-// Whether the wave's evaluated rays start at one point (true of none), with or without segments to gather.
-// This one answer says which of the two launches (in_two) a tile belongs to: the launches themselves and
-// the tile plan, which gives tasks and rows to the tiles of the first, both take it from here.
-__device__ __forceinline__ bool common_origin(const QueryIn& q) {
-    const uint64_t am = __ballot(q.alive);
-    const int fl = am ? __builtin_ctzll(am) : 0;
+// Whether the rays of the lanes with `on` start at one point (true of none).
+__device__ __forceinline__ bool share_origin(const QueryIn& q, bool on) {
+    const uint64_t m = __ballot(on);
+    const int fl = m ? __builtin_ctzll(m) : 0;
     const float ox = __shfl(q.o[0], fl, kWave), oy = __shfl(q.o[1], fl, kWave), oz = __shfl(q.o[2], fl, kWave);
-    return __ballot(q.alive && !(q.o[0] == ox && q.o[1] == oy && q.o[2] == oz)) == 0;
+    return __ballot(on && !(q.o[0] == ox && q.o[1] == oy && q.o[2] == oz)) == 0;
+}
+
+// Whether a ray has a segment of a scattering medium (the walk ends at a bad medium, as the gather does).
+__device__ __forceinline__ bool gathers(const EvalArgs& A, const QueryIn& q) {
+    if (!q.alive) return false;
+    for (int k = 0; k < q.nseg; ++k) {
+        const int32_t m = A.segments[q.s0 + k].medium_id;
+        if (m < 0 || m >= A.n_media) return false;
+        if (A.media[A.media_base + m].has_scattering) return true;
+    }
+    return false;
+}
+
+// Whether those of the wave's rays that gather anything start at one point: rays that miss the media or
+// have ended may start anywhere (a frame padded with them keeps its frusta). This one answer says which
+// of the two launches (in_two) a tile belongs to: the launches themselves and the tile plan, which gives
+// tasks and rows to the tiles of the first, all take it from here.
+__device__ __forceinline__ bool common_origin(const EvalArgs& A, const QueryIn& q) {
+    return share_origin(q, q.alive) || share_origin(q, gathers(A, q));  // no segment is read for most frames
 }
 
 __shared__ float g_part[4][3][kWave];  // the sums of a split launch's waves
@@ -1285,7 +1302,7 @@ __device__ bool run_tile(const EvalArgs& A, int64_t slot0, ItemPart part, unsign
     r.dx = in.d[0], r.dy = in.d[1], r.dz = in.d[2];
     int nseg = in.nseg;
     bool alive = in.alive;
-    if (KARG && in_two(MODE) && common_origin(in) == ((MODE & kSparse) != 0)) return false;
+    if (KARG && in_two(MODE) && common_origin(A, in) == ((MODE & kSparse) != 0)) return false;
     r.ix = guard_inv(r.dx);
     r.iy = guard_inv(r.dy);
     r.iz = guard_inv(r.dz);
@@ -1839,7 +1856,7 @@ __device__ __forceinline__ float tile_cost(const EvalArgs& A, int64_t slot, int 
         }
     const uint64_t am = __ballot(t0 <= t1);
     float c = 0.f;
-    one = common_origin(in);
+    one = common_origin(A, in);
     if (am) {
         const int fl = __builtin_ctzll(am);
         const bool on = t0 <= t1;

@@ -77,3 +77,25 @@ def test_tiles_of_every_class_are_written(n_queries, gathering, camera):
             torch.cuda.synchronize()
             assert torch.equal(out, got)
     bm.destroy()
+
+
+@pytest.mark.parametrize("n_queries,gathering", [(5_000, 78), (40_005, 600), (600_000, 900)])
+def test_rays_that_gather_nothing_do_not_matter_to_the_others(n_queries, gathering):
+    """Where a tile's other rays start, if they meet no medium, changes nothing: camera rays padded with them
+    keep the launch, the order and so the bits that they have when all start at the camera."""
+    print_case("tile_padding", q=n_queries, gathering=gathering)
+    w, gone = scene(n_queries, 16_384, gathering, True)
+    ctx = gpu_context(w.media)
+    bm = native.PhotonBeamsEvaluator(ctx)
+    bm.build(w.beams)
+    res = []
+    for elsewhere in (True, False):
+        if not elsewhere:
+            w.queries.origin[gone] = EYE
+        qv = native.QueryBatchView.to_device(w.queries, order=1)
+        out = torch.full((n_queries, 3), -1.0, device="cuda")
+        native.eval_batch(ctx, None, bm, qv, None, out)
+        res.append((out, native.hit_signatures(ctx, None, bm, qv)[1]))
+    assert np.array_equal(res[0][1], res[1][1])
+    assert torch.equal(res[0][0], res[1][0])
+    bm.destroy()
