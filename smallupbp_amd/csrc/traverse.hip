@@ -1025,7 +1025,11 @@ __device__ __forceinline__ void beam_leaf(const EvalArgs& A, const Ray& r, SegSt
 // tested 64 at a time, a lane taking any ray and any item. An item is accepted only by rays that meet
 // its box (the boxes are widened for that), but for the pairs that a beam's first and last piece own
 // beyond its ends: those pieces are tested by the whole wave as ever.
+// Photons gain even in the smallest structures; beams of fewer than kSparseFrom pieces don't make up for
+// the second launch (6000 parallel rays x 200 beams 90 us in one launch, 97 in two; 700 and 6000 scattered
+// rays the same either way).
 constexpr int kSparseLanes = 16;
+constexpr int64_t kSparseFrom = 1024;
 constexpr int kPq = 128;  // a leaf adds at most 64 pairs per lane to fewer than 64 queued
 __shared__ uint32_t g_pq[kHqWaves][2][kPq];
 
@@ -2270,9 +2274,9 @@ static void launch_plan(Ctx& ctx, const PlanArgs& P) {
 // An evaluation's launches, with its split set up. A plan gives the tiles with a common origin their parts;
 // the others are split uniformly.
 template <int EST, int MODE>
-void launch_kernel(Ctx& ctx, EvalArgs A, const Split& s, const TilePlan& p, int tuned) {
-    // one ray has one origin
-    const bool two = A.count > 1;
+void launch_kernel(Ctx& ctx, EvalArgs A, const Split& s, const TilePlan& p, int64_t items, int tuned) {
+    // one ray has one origin; few pieces take less time than a second launch
+    const bool two = A.count > 1 && (EST == kEstPhotons || items >= kSparseFrom);
     const int64_t tiles = (A.count + kWave - 1) / kWave;
     A.known = s.planned || !two;
     if (s.planned) {
@@ -2294,11 +2298,11 @@ void launch_kernel(Ctx& ctx, EvalArgs A, const Split& s, const TilePlan& p, int 
 }
 
 template <int EST, int MODE>
-void launch_reduced(Ctx& ctx, const EvalArgs& A, const Split& s, const TilePlan& p, int tuned) {
+void launch_reduced(Ctx& ctx, const EvalArgs& A, const Split& s, const TilePlan& p, int64_t items, int tuned) {
     if constexpr (EST == kEstBeams) {
-        if (A.red.max != 0) return launch_kernel<EST, MODE | kReduced>(ctx, A, s, p, tuned);
+        if (A.red.max != 0) return launch_kernel<EST, MODE | kReduced>(ctx, A, s, p, items, tuned);
     }
-    launch_kernel<EST, MODE>(ctx, A, s, p, tuned);
+    launch_kernel<EST, MODE>(ctx, A, s, p, items, tuned);
 }
 
 template <int EST>
@@ -2309,10 +2313,10 @@ void launch_mode(Ctx& ctx, Mode mode, EvalArgs& A, const QueryView& q, int64_t i
     A.shift = part_shift(items);
     A.rows = p.rows;
     switch (mode) {
-        case Mode::Forward: return launch_reduced<EST, (int)Mode::Forward>(ctx, A, s, p, tuned);
-        case Mode::Signature: return launch_reduced<EST, (int)Mode::Signature>(ctx, A, s, p, tuned);
-        case Mode::Adjoint: return launch_reduced<EST, (int)Mode::Adjoint>(ctx, A, s, p, tuned);
-        case Mode::Upbp: return launch_reduced<EST, (int)Mode::Upbp>(ctx, A, s, p, tuned);
+        case Mode::Forward: return launch_reduced<EST, (int)Mode::Forward>(ctx, A, s, p, items, tuned);
+        case Mode::Signature: return launch_reduced<EST, (int)Mode::Signature>(ctx, A, s, p, items, tuned);
+        case Mode::Adjoint: return launch_reduced<EST, (int)Mode::Adjoint>(ctx, A, s, p, items, tuned);
+        case Mode::Upbp: return launch_reduced<EST, (int)Mode::Upbp>(ctx, A, s, p, items, tuned);
     }
 }
 
