@@ -318,7 +318,11 @@ upbp_status upbp_bre_eval_brute_force(upbp_ctx* ctx, const upbp_bre* bre, const 
  * path, SmallUPBP/src/Renderers/VolLightTracer.hxx:378,384). Normalisation by
  * the light-path count stays with the caller, as in the reference.
  * Either structure may be NULL, then its output is not written.
- * Outputs are [count][3] floats in the query order of the batch. */
+ * Outputs are [count][3] floats in the query order of the batch.
+ * Recorded into a graph by the caller (sync = 0, device memory, order
+ * UPBP_ORDER_AS_GIVEN or at most 64 queries), the call allocates nothing and
+ * the graph stays valid; small batches then run without splitting their tiles
+ * over waves, which upbp_eval_noalloc does there too. */
 upbp_status upbp_eval(upbp_ctx* ctx, const upbp_bre* bre, const upbp_beams* beams,
                       const upbp_query_batch* queries, float* out_photons, float* out_beams,
                       upbp_memory out_memory, upbp_eval_stats* stats);
@@ -681,14 +685,15 @@ typedef struct upbp_batch_plan upbp_batch_plan;
  * structures may be destroyed after this call; rebuilding or re-powering them
  * (upbp_bre_set_power) does not reach an existing plan. Query arrays and
  * output buffers are referenced, not copied: they must outlive the plan and
- * may be refilled between runs. */
+ * may be refilled between runs. Plans of 1024 query tiles or more also hold
+ * memory to plan each run in. */
 upbp_status upbp_batch_plan_create(upbp_ctx* ctx, const upbp_instance* instances,
                                    int32_t count, upbp_batch_plan** out_plan);
 upbp_status upbp_batch_plan_destroy(upbp_batch_plan* plan);
-/* Run the plan: one fill kernel that resets the queue counters, then one
- * persistent photon kernel and one persistent beam kernel. With
- * use_graph = 1 the three launches are captured once into a hipGraph and
- * replayed on later calls. */
+/* Run the plan: kernels that reset the counters and, for 1024 query tiles or
+ * more, order the tiles by estimated cost, then one persistent photon kernel
+ * and one persistent beam kernel. With use_graph = 1 the launches are captured
+ * once into a hipGraph and replayed on later calls. */
 upbp_status upbp_batch_run(upbp_ctx* ctx, upbp_batch_plan* plan, int use_graph,
                            upbp_eval_stats* stats);
 

@@ -309,7 +309,8 @@ constexpr uint32_t kSplitMost = 64;
 
 // From kPlanTiles to kPlanMostTiles tiles (2^21 queries) a beam launch plans: a tile gets as many of
 // kPlanWaves waves, at most kPlanMost, as its share of the estimated cost, and the dearest parts start
-// first. Estimating takes 30 to 140 us, which fewer tiles do not earn back (256x256 rays x 100k photons
+// first. Estimating takes 50 to 610 us alone (6250 to 32400 tiles) and runs next to the photon kernel in
+// calls with both; fewer tiles do not earn it back (256x256 rays x 100k photons
 // 220 -> 270 us with 1024 tiles; photons and the UPBP kernels gain nothing and don't plan). Above
 // kPlanFewTiles tiles kSplitWaves, so that average tiles stay whole. Measured uniform / planned with
 // 16384 / 24576 / 32768 waves:
@@ -325,11 +326,14 @@ constexpr uint32_t kSplitMost = 64;
 constexpr uint32_t kPlanMost = 256;
 constexpr int64_t kPlanTiles = 512, kPlanMostTiles = 32768, kPlanFewTiles = 8192, kPlanWaves = 24576;
 // Batched plans of this many tiles are planned too, both estimators, with kPlanWaves waves. Tiles of small
-// instances stay whole there; the order alone shortens the tail. Measured in queue order / planned:
-//   16 instances, 4.6M rays                  7.36 / 5.08 ms
-//   18 instances x 26k rays                  6.16 / 1.77 ms
-//   5 instances x 22k rays                   1.91 / 0.93 ms
-//   15 instances x 358k rays                 3.91 / 4.07 ms (16384 waves: 3.91)
+// instances stay whole there; the order alone shortens the tail. Instances whose tiles cost alike gain
+// nothing and pay for the estimates (0.2 to 0.4 ms). Measured in queue order / planned:
+//   16 instances, 4.6M rays                  6.86 / 3.81 ms
+//   18 instances x 26k rays                  5.98 / 1.45 ms
+//   5 instances x 22k rays                   1.92 / 0.74 ms
+//   15 instances x 358k rays                 3.23 / 2.93 ms
+//   8 even instances x 100k camera rays      0.63 / 0.85 ms
+//   8 even instances x 100k scattered rays   2.84 / 3.23 ms
 constexpr int64_t kPlanBatchTiles = 1024, kPlanBatchMost = 1 << 20;
 
 // ---- lbvh.hip -------------------------------------------------------------
@@ -472,8 +476,8 @@ void launch_light_tails(Ctx& ctx, MisDev& mis);
 void launch_beam_records(Ctx& ctx, MisDev& mis, int64_t n_beams);
 // The same per light vertex for the PB2D hits into ctx.photon_recs (mis.photon_recs).
 void launch_photon_records(Ctx& ctx, MisDev& mis);
-// How many waves share a tile's items in an evaluation of count queries against items items (a power
-// of two), and how many blocks they form.
+// How an evaluation of count queries against items items is split: into how many parts a tile's items go, or
+// whether a plan decides that tile by tile, and how many rows of partial sums that takes.
 Split split_of(int64_t count, int64_t items, int estimator, Mode mode);
 // Adds up a split evaluation's parts into the outputs (null: not evaluated), in query order.
 void launch_sum_rows(Ctx& ctx, const QueryView& q, float* ph, float* bm);
